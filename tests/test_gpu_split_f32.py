@@ -1,0 +1,82 @@
+"""GPU: the f32 convolutions that run on the bf16 matrix cores (three bf16 pieces per value, six
+piece products, csrc/split.h) against 64-bit sums, at the edges of their tiles and on values that
+are not finite.
+
+Bound: the matrix core rounds its f32 accumulator once per 8 products; the full-size accumulator
+takes 16 of the K products per 4 such roundings, its partner's are 2^-8 smaller, the pieces drop
+2^-26 of a product, and bias, final sum and store add three roundings. Every rounding is at most
+2^-23 (it may truncate) of a partial sum, itself at most S = |b| + sum |x w|, so
+|err| <= (K / 4 * (1 + 2^-7) + 4) * 2^-23 * S."""
+
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+from zenjpegai_amd import nn, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng():
+    e = nn.Engine(0, "f32")
+    yield e
+    e.close()
+
+
+def _layer(eng, kind, cin, cout, groups, seed):
+    k, stride = {"3x3": (3, 1), "s2": (3, 2), "2x2": (2, 1)}[kind]
+    w = synth.normal(seed, f"split/w{kind}{cin}{cout}", (cout, cin // groups, k, k), 1.0)
+    b = synth.normal(seed, f"split/b{cout}", (cout,), 1.0)
+    pad, ext = ((0, 0), (0, 0, 1, 1)) if kind == "2x2" else ((1, 1), (0, 0, 0, 0))
+
+    def ref(x, w, b):
+        x = torch.from_numpy(x).double()[None]
+        x = F.pad(x, (0, 1, 0, 1) if kind == "2x2" else (1, 1, 1, 1))
+        return F.conv2d(x, torch.from_numpy(w).double(), torch.from_numpy(b).double(), stride, 0, 1, groups)[0].numpy()
+
+    return w, b, lambda w, b: nn.ConvLayer(nn.Conv2d(cin, cout, (k, k), stride, pad, groups, w, b), eng, extra_pad=ext), ref
+
+
+# (kind, cin, cout, groups, h, w): every tile shape, channel counts off 16 and 64, one-row and
+# one-column maps, sizes around the 16-column and 4- / 8- / 16-row tiles.
+CASES = [("3x3", 4, 4, 1, 1, 1), ("3x3", 20, 24, 1, 9, 17), ("3x3", 160, 160, 1, 13, 19), ("3x3", 48, 40, 1, 130, 66),
+         ("3x3", 64, 128, 1, 90, 97), ("3x3", 32, 128, 1, 177, 190), ("3x3", 16, 192, 1, 200, 210),
+         ("3x3", 16, 128, 1, 260, 250), ("3x3", 64, 64, 4, 33, 31), ("3x3", 64, 64, 4, 150, 161),
+         ("3x3", 128, 128, 4, 15, 16), ("3x3", 128, 128, 4, 150, 161), ("s2", 20, 16, 1, 1, 7), ("s2", 64, 64, 1, 35, 33),
+         ("s2", 24, 32, 1, 66, 64), ("s2", 64, 64, 1, 175, 177), ("s2", 16, 128, 1, 255, 257), ("s2", 16, 128, 1, 440, 431),
+         ("s2", 16, 192, 1, 440, 431), ("2x2", 160, 256, 1, 4, 6), ("2x2", 20, 12, 1, 17, 15), ("2x2", 64, 128, 1, 128, 127),
+         ("2x2", 16, 192, 1, 150, 161)]
+
+
+@pytest.mark.parametrize("kind,cin,cout,groups,h,w", CASES)
+def test_error_against_64_bits(eng, kind, cin, cout, groups, h, w):
+    wt, b, make, ref = _layer(eng, kind, cin, cout, groups, 31)
+    x = synth.normal(32, f"split/x{cin}{h}", (cin, h, w), 1.0)
+    y = make(wt, b).forward(eng, nn.BTensor.from_planar(eng, x)).to_planar()
+    want, size = ref(x, wt, b), ref(np.abs(x), np.abs(wt), np.abs(b))
+    assert y.shape == want.shape
+    kk = wt[0].size
+    bound = (kk / 4 * (1 + 2.0 ** -7) + 4) * 2.0 ** -23 * size
+    assert np.all(np.abs(y - want) <= bound), float(np.max(np.abs(y - want) / bound))
+
+
+@pytest.mark.parametrize("kind", ["3x3", "s2", "2x2"])
+def test_values_that_are_not_finite(eng, kind):
+    """Infinities and NaN in the input or the weights reach the outputs that f32 arithmetic sends
+    them to, and only those."""
+    wt, b, make, ref = _layer(eng, kind, 32, 16, 1, 33)
+    wt[3, 5] = 0.0  # 0 * inf is NaN
+    x = synth.normal(34, "split/nf", (32, 24, 40), 1.0)
+    for ch, r, c, v in ((0, 2, 3, np.inf), (5, 7, 20, -np.inf), (9, 12, 33, np.nan), (31, 23, 39, np.inf), (5, 18, 8, np.inf), (6, 18, 9, -np.inf)):
+        x[ch, r, c] = v
+    for w in (wt, np.where(np.arange(16)[:, None, None, None] == 7, np.float32(np.inf), wt)):
+        w = np.ascontiguousarray(w)
+        y = make(w, b).forward(eng, nn.BTensor.from_planar(eng, x)).to_planar()
+        want = ref(x, w, b)
+        np.testing.assert_array_equal(np.isnan(y), np.isnan(want))
+        inf = np.isinf(want)
+        np.testing.assert_array_equal(y[inf], want[inf])
+        fin = np.isfinite(want)
+        assert np.isfinite(y[fin]).all() and np.allclose(y[fin], want[fin], rtol=1e-4, atol=1e-3)

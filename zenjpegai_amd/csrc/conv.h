@@ -66,6 +66,10 @@ struct TileCfg {
 
 enum ConvKind : int { CK_1x1 = 0, CK_2x2 = 1, CK_3x3 = 2, CK_3x3_S2 = 3, CK_T3 = 4 };
 
+// f32 layers of these kinds run on the bf16 matrix cores from weights packed in split form
+// (conv_f32.hip, split.h); everything else goes through launch_conv.
+inline bool conv_is_split(int kind, int dtype) { return dtype == DT_F32 && (kind == CK_2x2 || kind == CK_3x3 || kind == CK_3x3_S2); }
+hipError_t launch_conv_split(int kind, TileCfg cfg, const ConvParams& p, hipStream_t s);
 hipError_t launch_conv(int kind, int dtype, TileCfg cfg, const ConvParams& p, hipStream_t s);
 
 // Stride-2 transposed conv with 3x3 kernels (9 taps over the four output phases), all four

@@ -1327,6 +1327,10 @@ static hipError_t go(const ConvParams& p0, hipStream_t s) {
 
 template <typename T, int WC, int WP, int CF, int PF>
 static hipError_t go_kind(int kind, const ConvParams& p, hipStream_t s) {
+    if constexpr (sizeof(T) == 4) {
+        if (kind != CK_1x1 && kind != CK_T3) return hipErrorInvalidValue;  // launch_conv_split's
+        return kind == CK_1x1 ? go<T, 1, 1, 1, false, WC, WP, CF, PF>(p, s) : go<T, 3, 3, 1, true, WC, WP, CF, PF>(p, s);
+    } else
     switch (kind) {
         case CK_1x1: return go<T, 1, 1, 1, false, WC, WP, CF, PF>(p, s);
         case CK_2x2: return go<T, 2, 2, 1, false, WC, WP, CF, PF>(p, s);
@@ -1348,10 +1352,10 @@ static hipError_t go_kind(int kind, const ConvParams& p, hipStream_t s) {
 template <typename T>
 static hipError_t go_cfg(int kind, TileCfg c, const ConvParams& p, hipStream_t s) {
     if (c.wc == 2 && c.wp == 4 && c.cf == 2 && c.pf == 4)
-        return kind == CK_3x3 ? go<T, 3, 3, 1, false, 2, 4, 2, 4>(p, s) : hipErrorInvalidValue;
+        return sizeof(T) == 2 && kind == CK_3x3 ? go<std::conditional_t<sizeof(T) == 2, T, __bf16>, 3, 3, 1, false, 2, 4, 2, 4>(p, s) : hipErrorInvalidValue;
     if (c.wc == 4 && c.wp == 2 && c.cf == 2 && c.pf == 4) {
         if constexpr (sizeof(T) == 4) return kind == CK_1x1 ? go<T, 1, 1, 1, false, 4, 2, 2, 4>(p, s) : hipErrorInvalidValue;
-        return kind == CK_3x3_S2 ? go<T, 3, 3, 2, false, 4, 2, 2, 4>(p, s) : hipErrorInvalidValue;
+        else return kind == CK_3x3_S2 ? go<T, 3, 3, 2, false, 4, 2, 2, 4>(p, s) : hipErrorInvalidValue;
     }
 #define ZJAI_GO(a, b, cc, d) \
     if (c.wc == a && c.wp == b && c.cf == cc && c.pf == d) return go_kind<T, a, b, cc, d>(kind, p, s);

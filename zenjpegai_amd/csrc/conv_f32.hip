@@ -1,0 +1,299 @@
+// f32 implicit-GEMM convolution on the bf16 matrix cores (see split.h for the arithmetic).
+//
+// GEMM roles and tiling as conv_igemm (conv.hip): one workgroup computes TY = WP * PF output rows
+// x 16 columns x NB = WC * CF blocks of 16 output channels, K = input channels (16 per chunk) x
+// taps. Per chunk the input halo is loaded into registers one chunk ahead, split into its bf16
+// pieces and stored to LDS once (each staged value feeds 9 taps x NB * 16 outputs, so the split's
+// ~9 vector instructions per value disappear beside the MFMAs they allow); the weights are packed
+// already split and stream through a two-slot LDS ring by direct loads, TS taps per slot.
+//
+// LDS layout of a halo: planes [4 channel quads][NPX pixels] of 16-byte (p1, p0) units, then of
+// 8-byte p2 units, NPX = 16 (mod 32): a fragment read's 16 consecutive pixels x 4 quads then fall
+// on distinct banks for any first pixel (ds_read_b128 takes 16 lanes of two quads per pass,
+// ds_read_b64 32 lanes). Weight blocks are stored in lane order.
+//
+// The sum of an output is, for every tile shape: bias, then per chunk and tap the three MFMAs of
+// mma_split -- so the choice of tile never changes a bit.
+
+#include "conv.h"
+#include "epilogue.h"
+#include "split.h"
+
+namespace zjai {
+
+__device__ u32x4 g_zero_split[1];  // 16 zero bytes: the source of padding units
+
+template <int KH, int KW, int S, int WC, int WP, int CF, int PF, int TS, int NHB, int RW>
+__global__ void __launch_bounds__(WC * WP * 64, 2)
+conv_igemm_split(const ConvParams p) {
+    constexpr int NT = WC * WP * 64;
+    constexpr int TY = WP * PF;
+    constexpr int HY = (TY - 1) * S + KH, HX = 15 * S + KW, HP = HY * HX;
+    constexpr int NTAP = KH * KW, NST = NTAP / TS;
+    static_assert(NTAP % TS == 0, "whole stages");
+    constexpr int NB = WC * CF;
+    constexpr int NPX = (HP + 15) / 32 * 32 + 16;
+    static_assert(NPX >= HP, "plane size");
+    constexpr int HALO_U = 6 * NPX;                  // 16-byte units of one halo buffer
+    constexpr int W_U = NB * TS * SPLIT_BLOCK_U;     // of one weight slot
+    constexpr int OUT_LD = NB * 16 + 4;              // f32 output tile [positions][channels + 4]
+    constexpr int OUT_U = (TY * 16 * OUT_LD + 3) / 4;
+    constexpr int RUN_U = NHB * HALO_U + RW * W_U;
+    constexpr int LDS_U = RUN_U > OUT_U ? RUN_U : OUT_U;
+    constexpr int HN = (HP * 4 + NT - 1) / NT, WN = (W_U + NT - 1) / NT;
+    __shared__ u32x4 s_lds[LDS_U];
+    u32x4* const s_w = s_lds + NHB * HALO_U;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wc = wave % WC, wp = wave / WC;
+    const int col = lane & 15, grp = lane >> 4;
+
+    // Workgroup -> tile: the XCD-aware order of conv_igemm.
+    const int nz = p.ntiles;
+    const int total = p.gx * p.gy * p.N * nz;
+    const int bid = (int)blockIdx.x, xj = bid & 7, xk = bid >> 3;
+    const int q8 = total >> 3, r8 = total & 7;
+    const int lid = xj < r8 ? xj * (q8 + 1) + xk : r8 * (q8 + 1) + (xj - r8) * q8 + xk;
+    int rest = lid / nz;
+    const int nt = lid - rest * nz;
+    const int tx = rest % p.gx;
+    rest /= p.gx;
+    const int ty = rest % p.gy, bi = rest / p.gy;
+    const int gb = nt * NB;
+    const int g = gb / p.nblk_g, nb0 = gb - g * p.nblk_g;
+    const int ox0 = tx * 16, oy0 = ty * TY;
+    if (nb0 * 16 >= p.cout_g) return;  // padding blocks only (uniform)
+
+    f32x4 big[CF][PF], small[CF][PF];
+#pragma unroll
+    for (int cf = 0; cf < CF; ++cf) {
+        const int ocl = (nb0 + wc * CF + cf) * 16 + grp * 4;
+        f32x4 b;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            b[i] = (p.bias && ocl + i < p.cout_g) ? p.bias[g * p.cout_g + ocl + i] : 0.0f;
+#pragma unroll
+        for (int pf = 0; pf < PF; ++pf) {
+            big[cf][pf] = b;
+            small[cf][pf] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+
+    const int iy0 = oy0 * S - p.pad_t, ix0 = ox0 * S - p.pad_l;
+    const float* xg = (const float*)p.x.p + (long long)bi * p.x.bstride;
+    const long long xbase = (long long)p.x.c_off + (long long)g * p.cin_g;
+
+    // LDS slot of halo pixel (hy, hx): stride-2 halos keep each row's even columns, then its odd
+    // ones, so that a fragment's every-other-column reads are consecutive slots.
+    constexpr int HXE = (HX + 1) / 2;
+    auto hslot = [](int hy, int hx) __attribute__((always_inline)) {
+        return S == 2 ? hy * HX + ((hx & 1) ? HXE + (hx >> 1) : (hx >> 1)) : hy * HX + hx;
+    };
+    // This thread's halo units (channel quad q of a pixel): where the next chunk's is read from and
+    // how far that moves per chunk (padding reads 16 zero bytes and stays there), and its LDS slot.
+    const float* hp[HN];
+    int hstep[HN], hdst[HN];
+#pragma unroll
+    for (int i = 0; i < HN; ++i) {
+        const int u = tid + i * NT, pix = u >> 2, q = u & 3;
+        const int hy = pix / HX, hx = pix - hy * HX;
+        const int iy = iy0 + hy, ix = ix0 + hx;
+        const bool in = u < HP * 4 && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W;
+        hp[i] = in ? xg + (long long)iy * p.x.row + (long long)ix * p.x.cs + xbase + q * 4 : (const float*)g_zero_split;
+        hstep[i] = in ? 16 : 0;
+        hdst[i] = q * NPX + hslot(hy, hx);
+    }
+    const int qv = (tid & 3) * 4;
+    u32x4 rh[HN];
+    auto load_halo = [&](int chunk) __attribute__((always_inline)) {
+        if (chunk * 16 + 16 <= p.cin_g) {
+#pragma unroll
+            for (int i = 0; i < HN; ++i) {
+                rh[i] = *(const u32x4*)hp[i];
+                hp[i] += hstep[i];
+            }
+        } else {  // the last chunk of a cin_g off 16
+#pragma unroll
+            for (int i = 0; i < HN; ++i)
+                rh[i] = *(chunk * 16 + qv < p.cin_g ? (const u32x4*)hp[i] : g_zero_split);
+        }
+    };
+    auto store_halo = [&](int chunk) __attribute__((always_inline)) {
+        u32x4* dst = s_lds + (NHB == 2 ? (chunk & 1) * HALO_U : 0);
+        u32x2* hi = (u32x2*)(dst + 4 * NPX);
+#pragma unroll
+        for (int i = 0; i < HN; ++i) {
+            u32x4 v = rh[i];
+            if (p.relu6_in) v = relu6_vec<float>(v);
+            const SplitFrag f = split_f32(__builtin_bit_cast(f32x4, v));
+            if (tid + i * NT < HP * 4) {
+                dst[hdst[i]] = f.lo;
+                hi[hdst[i]] = f.hi;
+            }
+        }
+    };
+    // Weight slot of stage (chunk, j): taps j * TS .. of blocks nb0 .. nb0 + NB - 1, loaded RW - 1
+    // stages ahead (the slot was last read that many stages ago). The lanes' offsets stay, the
+    // uniform base moves.
+    const char* const wg = (const char*)((const u32x4*)p.w + ((long long)g * p.nchunks * p.nblk_g + nb0) * (NTAP * SPLIT_BLOCK_U));
+    const long long wchunk = (long long)p.nblk_g * (NTAP * SPLIT_BLOCK_U * 16);
+    unsigned woff[WN];
+#pragma unroll
+    for (int i = 0; i < WN; ++i) {
+        const int u = tid + i * NT, nb = u / (TS * SPLIT_BLOCK_U);
+        woff[i] = (unsigned)(nb * (NTAP * SPLIT_BLOCK_U) + (u - nb * (TS * SPLIT_BLOCK_U))) * 16;
+    }
+    auto issue_stage = [&](int st, int slot) __attribute__((always_inline)) {
+        const int c = NST == 1 ? st : st / NST;
+        const char* src = wg + c * wchunk + (st - c * NST) * (TS * SPLIT_BLOCK_U * 16);
+        u32x4* dst = s_w + slot * W_U;
+#pragma unroll
+        for (int i = 0; i < WN; ++i) {
+            const int ub = wave * 64 + i * NT;
+            if (ub >= W_U) break;
+            if (ub + lane < W_U) lds_dma16_at(src, woff[i], dst + ub);
+        }
+    };
+
+    constexpr int CW = W_U / NT;  // direct loads per stage that every wave issues at least
+    const int nchunks = p.nchunks, nst = nchunks * NST;
+    load_halo(0);
+    for (int k = 0; k < RW - 1 && k < nst; ++k) issue_stage(k, k);
+    int slot = 0, nslot = RW - 1;  // ring slots of stage st and of stage st + RW - 1
+#pragma unroll 1
+    for (int chunk = 0, st = 0; chunk < nchunks; ++chunk) {
+        const u32x4* s_halo = s_lds + (NHB == 2 ? (chunk & 1) * HALO_U : 0);
+        const u32x2* s_hhi = (const u32x2*)(s_halo + 4 * NPX);
+#pragma unroll 1
+        for (int j = 0; j < NST; ++j, ++st) {
+            if (j == 0) {
+                if (NHB == 1 && chunk > 0) __syncthreads();  // every wave is done with the last halo
+                store_halo(chunk);
+            }
+            // This wave's weight loads of the stage are in LDS; those of the next RW - 2 stages and
+            // the halo loads of the next chunk (issued after them) may still fly.
+            const bool more = RW == 3 && st + 1 < nst, halo = j >= 1 && j < RW && chunk + 1 < nchunks;
+            if (more && halo) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(CW + HN) : "memory");
+            else if (more) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(CW) : "memory");
+            else if (halo && RW == 2) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(HN) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+            __syncthreads();  // ... and every other wave's, and the split halo
+            if (st + RW - 1 < nst) issue_stage(st + RW - 1, nslot);
+            if (j == 0 && chunk + 1 < nchunks) load_halo(chunk + 1);
+            const u32x4* sw = s_w + slot * W_U;
+            slot = slot + 1 == RW ? 0 : slot + 1;
+            nslot = nslot + 1 == RW ? 0 : nslot + 1;
+#pragma unroll
+            for (int t = 0; t < TS; ++t) {
+                const int tap = j * TS + t, ky = tap / KW, kx = tap - ky * KW;
+                SplitFrag a[CF], b[PF];
+#pragma unroll
+                for (int cf = 0; cf < CF; ++cf) {
+                    const u32x4* w = sw + ((wc * CF + cf) * TS + t) * SPLIT_BLOCK_U;
+                    a[cf].lo = w[lane];
+                    a[cf].hi = ((const u32x2*)(w + 64))[lane];
+                }
+#pragma unroll
+                for (int pf = 0; pf < PF; ++pf) {
+                    const int s = grp * NPX + hslot((wp * PF + pf) * S + ky, col * S + kx);
+                    b[pf].lo = s_halo[s];
+                    b[pf].hi = s_hhi[s];
+                }
+#pragma unroll
+                for (int cf = 0; cf < CF; ++cf)
+#pragma unroll
+                    for (int pf = 0; pf < PF; ++pf) mma_split(big[cf][pf], small[cf][pf], a[cf], b[pf]);
+            }
+        }
+    }
+
+    // Transposed through LDS: every position's NB * 16 channels leave as one contiguous run.
+    __syncthreads();
+    float* so = reinterpret_cast<float*>(s_lds);
+#pragma unroll
+    for (int cf = 0; cf < CF; ++cf)
+#pragma unroll
+        for (int pf = 0; pf < PF; ++pf)
+            *reinterpret_cast<f32x4*>(so + ((wp * PF + pf) * 16 + col) * OUT_LD + (wc * CF + cf) * 16 + grp * 4) =
+                split_sum(big[cf][pf], small[cf][pf]);
+    __syncthreads();
+    const bool full = nb0 * 16 + NB * 16 <= p.cout_g;  // all of the tile's channels are real
+    if (full && epilogue_simple(p)) {
+        constexpr int QP8 = NB * 2;  // 8 channels per thread and step
+#pragma unroll 4
+        for (int u = tid; u < TY * 16 * QP8; u += NT) {
+            const int pos = u / QP8, c8 = u - pos * QP8;
+            const int oy = oy0 + (pos >> 4), ox = ox0 + (pos & 15);
+            const f32x4 v0 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8);
+            const f32x4 v1 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8 + 4);
+            if (oy < p.OH && ox < p.OW) epilogue_store8<float>(p, bi, oy, ox, g * p.cout_g + nb0 * 16 + c8 * 8, v0, v1);
+        }
+        return;
+    }
+    if (full && epilogue_ps2(p)) {
+        // Pixel shuffle by 2: conv channels 4 c + s of 4 consecutive output channels c, one
+        // sub-position s, as one vector store.
+        constexpr int QP = NB * 4;
+        for (int u = tid; u < TY * 16 * QP; u += NT) {
+            const int pos = u / QP, q = u - pos * QP, cq = q % NB, sub = q / NB;
+            const int oy = oy0 + (pos >> 4), ox = ox0 + (pos & 15);
+            if (oy >= p.OH || ox >= p.OW) continue;
+            const float* v = so + pos * OUT_LD + cq * 16 + sub;
+            epilogue_store_ps2<float>(p, bi, oy, ox, sub, (g * p.cout_g + nb0 * 16) / 4 + cq * 4,
+                                      f32x4{v[0], v[4], v[8], v[12]});
+        }
+        return;
+    }
+    constexpr int QP = NB * 4;
+    for (int u = tid; u < TY * 16 * QP; u += NT) {
+        const int pos = u / QP, cq = u - pos * QP;
+        const int oy = oy0 + (pos >> 4), ox = ox0 + (pos & 15);
+        const int ocl = nb0 * 16 + cq * 4;
+        if (oy >= p.OH || ox >= p.OW || ocl >= p.cout_g) continue;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + cq * 4);
+        epilogue_store<float>(p, bi, oy, ox, g * p.cout_g + ocl, min(4, p.cout_g - ocl), v);
+    }
+}
+
+namespace {
+
+template <int KH, int KW, int S, int WC, int WP, int CF, int PF, int TS, int NHB, int RW>
+hipError_t go_split(const ConvParams& p0, hipStream_t s) {
+    constexpr int TY = WP * PF;
+    ConvParams p = p0;
+    if (p.ntiles != p.groups * p.nblk_g / (WC * CF) || p.nblk_g % (WC * CF) || p.N < 1 || p.N > MAXB || p.w_bstride)
+        return hipErrorInvalidValue;
+    p.gx = (p.OW + 15) / 16;
+    p.gy = (p.OH + TY - 1) / TY;
+    const long long total = (long long)p.gx * p.gy * p.N * p.ntiles;
+    if (total <= 0 || total > (1ll << 30)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((conv_igemm_split<KH, KW, S, WC, WP, CF, PF, TS, NHB, RW>), dim3((unsigned)total),
+                       dim3(WC * WP * 64), 0, s, p);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// Instantiated shapes per kind: (wc, wp, cf, pf), taps per weight slot, halo buffers, slots.
+#define ZJAI_SPLIT(KIND, KH, KW, S, A, B, C, D, TS, NHB, RW) \
+    if (kind == KIND && c.wc == A && c.wp == B && c.cf == C && c.pf == D) return go_split<KH, KW, S, A, B, C, D, TS, NHB, RW>(p, s);
+
+hipError_t launch_conv_split(int kind, TileCfg c, const ConvParams& p, hipStream_t s) {
+    ZJAI_SPLIT(CK_3x3, 3, 3, 1, 2, 2, 4, 4, 1, 2, 3)
+    ZJAI_SPLIT(CK_3x3, 3, 3, 1, 1, 4, 4, 4, 1, 1, 3)
+    ZJAI_SPLIT(CK_3x3, 3, 3, 1, 1, 4, 4, 2, 3, 1, 2)
+    ZJAI_SPLIT(CK_3x3, 3, 3, 1, 1, 4, 2, 2, 3, 1, 2)
+    ZJAI_SPLIT(CK_3x3, 3, 3, 1, 1, 4, 1, 2, 9, 1, 2)
+    ZJAI_SPLIT(CK_3x3, 3, 3, 1, 1, 8, 1, 1, 9, 1, 2)
+    ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 2, 2, 4, 2, 1, 1, 3)
+    ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 4, 4, 2, 1, 1, 2)
+    ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 4, 4, 1, 3, 1, 2)
+    ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 4, 2, 1, 3, 1, 2)
+    ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 4, 1, 1, 9, 1, 2)
+    ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 4, 4, 2, 1, 1, 3)
+    ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 8, 2, 1, 4, 1, 2)
+    ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 8, 1, 1, 4, 1, 2)
+    return hipErrorInvalidValue;
+}
+
+}  // namespace zjai

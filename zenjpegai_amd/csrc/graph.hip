@@ -346,7 +346,7 @@ struct Fwd {
             {
                 char name[48];
                 static const char* ty[] = {"float", "_Float16", "__bf16"};
-                snprintf(name, sizeof name, "k_resau<%s, %d, %d>", ty[x->dtype], x->c, resau_rows(x->dtype, x->n, x->h, x->w));
+                snprintf(name, sizeof name, "k_resau<%s, %d, %d>", ty[x->dtype], x->c, resau_rows(x->n, x->h, x->w));
                 LaunchScope sc(ctx, name, 2.0 * npos * (C * 16 * 9 + C * C), 2.0 * dtype_size(x->dtype) * npos * C);
                 ZJAI_HIP(launch_resau(x->dtype, x->c, a, ctx.stream));
             }

@@ -69,6 +69,14 @@ __device__ __forceinline__ void lds_dma16(const void* src, void* wave_dst) {
                  : "memory", "m0");
 }
 
+// lds_dma16 from a uniform base and a 32-bit byte offset per lane.
+__device__ __forceinline__ void lds_dma16_at(const void* base, unsigned off, void* wave_dst) {
+    const unsigned m0 = __builtin_amdgcn_readfirstlane(
+        (unsigned)(size_t)(__attribute__((address_space(3))) void*)wave_dst);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(m0)
+                 : "memory", "m0");
+}
+
 // clamp(v, 0, 6) on a 16-byte vector of the storage type (ResAU's relu6 on load).
 template <typename T> __device__ __forceinline__ u32x4 relu6_vec(u32x4 v);
 template <> __device__ __forceinline__ u32x4 relu6_vec<float>(u32x4 v) {

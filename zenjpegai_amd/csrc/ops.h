@@ -81,7 +81,7 @@ struct ResauArgs {
     int nblk2;
 };
 bool resau_fused_supported(int C, int groups);
-int resau_rows(int dtype, int N, int h, int w);
+int resau_rows(int N, int h, int w);
 hipError_t launch_resau(int dtype, int C, const ResauArgs& p, hipStream_t s);
 // The attention branch's qkv = depthwise3x3(conv1x1(LN(x))) (dim -> 3 dim) in one kernel
 // (every storage type, dim 64 or 128); weights as FfnArgs. y must not alias x.

@@ -20,8 +20,8 @@
 // (the same few KB for every workgroup, L2-resident), so LDS holds only the halo and t and
 // several workgroups share a CU. Results equal the two unfused launches bit for bit.
 
-#include "mfma.h"
 #include "ops.h"
+#include "split.h"
 
 namespace zjai {
 
@@ -44,7 +44,7 @@ __device__ __forceinline__ void mma_rows(f32x4 (&acc)[N], u32x4 a, const u32x4 (
 }
 
 template <typename T, int C, int TR>
-__global__ void __launch_bounds__(256) k_resau(const ResauArgs p) {
+__global__ void __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) k_resau(const ResauArgs p) {
     constexpr int VEC = 16 / (int)sizeof(T);  // channels per 16-byte unit
     constexpr int CK = 4 * VEC;               // channels per K chunk (64 bytes)
     constexpr int G = C / 16;                 // groups of 16 channels
@@ -57,8 +57,15 @@ __global__ void __launch_bounds__(256) k_resau(const ResauArgs p) {
     constexpr int HU = HP * UPP, HIT = (HU + 255) / 256;
     static_assert(G == 2 || G == 4, "32 or 64 channels in groups of 16");
     static_assert(TR % WPG == 0 && NPW >= 1, "rows per wave");
-    __shared__ u32x4 s_h[HU];
-    __shared__ u32x4 s_t[TR * 16 * UPP];
+    // f32: the halo in split form (split.h) as planes [channel quad][NPX] of (p1, p0) units, then
+    // of p2 units; t takes its place once the 3x3 is done.
+    constexpr bool F32 = sizeof(T) == 4;
+    constexpr int NPX = (HP + 15) / 32 * 32 + 16;
+    constexpr int TU = TR * 16 * UPP;
+    __shared__ u32x4 s_h[F32 ? UPP * NPX * 3 / 2 : HU];
+    __shared__ u32x4 s_tb[F32 ? 1 : TU];
+    u32x4* const s_t = F32 ? s_h : s_tb;
+    u32x2* const s_hhi = (u32x2*)(s_h + (F32 ? UPP * NPX : 0));
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 15, grp = lane >> 4;
@@ -71,13 +78,22 @@ __global__ void __launch_bounds__(256) k_resau(const ResauArgs p) {
 
     // A fragments: grouped 3x3 packing [group][tap][16 out][CK], 1x1 packing [chunk][nblk][16][CK]
     // (16-byte units; lane (col, grp) holds row col, K group grp).
-    const u32x4* w1 = (const u32x4*)p.w1 + (long long)gi * 9 * 64;
+    const u32x4* w1 = (const u32x4*)p.w1 + (long long)gi * 9 * (F32 ? SPLIT_BLOCK_U : 64);
     const u32x4* w2 = (const u32x4*)p.w2;
-    u32x4 a1[9], a2[NC2];
+    u32x4 a1[F32 ? 1 : 9], a2[NC2];
+    SplitFrag an;  // f32: one tap at a time, the next one's loaded ahead
+    auto load_tap = [&](int t) __attribute__((always_inline)) {
+        const u32x4* w = w1 + t * SPLIT_BLOCK_U;
+        an = SplitFrag{w[lane], ((const u32x2*)(w + 64))[lane]};
+    };
+    if constexpr (F32) {
+        load_tap(0);
+    } else {
 #pragma unroll
-    for (int t = 0; t < 9; ++t) a1[t] = w1[(t * 16 + col) * 4 + grp];
+        for (int t = 0; t < 9; ++t) a1[t] = w1[(t * 16 + col) * 4 + grp];
+    }
 #pragma unroll
-    for (int c = 0; c < NC2; ++c) a2[c] = w2[((c * p.nblk2 + gi) * 16 + col) * 4 + grp];
+    for (int c = 0; c < (F32 ? 0 : NC2); ++c) a2[c] = w2[((c * p.nblk2 + gi) * 16 + col) * 4 + grp];
 
     // 1. relu6(x) halo. Every load reads a clamped (in-picture) pixel and off-picture ones take
     // zeros afterwards, so all of a thread's loads are in flight together.
@@ -97,7 +113,14 @@ __global__ void __launch_bounds__(256) k_resau(const ResauArgs p) {
         const int hy = pix / HX, hx = pix - hy * HX;
         const int iy = y0 - 1 + hy, ix = x0 - 1 + hx;
         const bool in = iy >= 0 && iy < p.h && ix >= 0 && ix < p.w;
-        s_h[pix * UPP + (q ^ (pix & (UPP - 1)))] = in ? relu6_vec<T>(hv[i]) : u32x4{0u, 0u, 0u, 0u};
+        const u32x4 v = in ? relu6_vec<T>(hv[i]) : u32x4{0u, 0u, 0u, 0u};
+        if constexpr (F32) {
+            const SplitFrag f = split_f32(__builtin_bit_cast(f32x4, v));
+            s_h[q * NPX + pix] = f.lo;
+            s_hhi[q * NPX + pix] = f.hi;
+        } else {
+            s_h[pix * UPP + (q ^ (pix & (UPP - 1)))] = v;
+        }
     }
     __syncthreads();
 
@@ -106,17 +129,36 @@ __global__ void __launch_bounds__(256) k_resau(const ResauArgs p) {
 #pragma unroll
     for (int r = 0; r < NPW; ++r) acc[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const int qb = gi * UG + (grp & (UG - 1));  // this lane's unit of the group
+    if constexpr (F32) {
+        f32x4 small[NPW];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) {
-        const int ky = t / 3, kx = t - 3 * (t / 3);
-        u32x4 bv[NPW];
+        for (int r = 0; r < NPW; ++r) small[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int t = 0; t < 9; ++t) {
+            const SplitFrag a = an;
+            load_tap(min(t + 1, 8));
+            const int i0 = qb * NPX + (r0 + t / 3) * HX + col + t % 3;
+            SplitFrag bv[NPW];
 #pragma unroll
-        for (int r = 0; r < NPW; ++r) {
-            const int pix = (r0 + r + ky) * HX + col + kx;
-            bv[r] = s_h[pix * UPP + (qb ^ (pix & (UPP - 1)))];
-            if (grp >= UG) bv[r] = u32x4{0u, 0u, 0u, 0u};  // 16-bit: K lanes 16..31 are padding
+            for (int r = 0; r < NPW; ++r) bv[r] = SplitFrag{s_h[i0 + r * HX], s_hhi[i0 + r * HX]};
+            mma_split_rows<NPW>(acc, small, a, bv);
         }
-        mma_rows<T, NPW>(acc, a1[t], bv);
+#pragma unroll
+        for (int r = 0; r < NPW; ++r) acc[r] = split_sum(acc[r], small[r]);
+        __syncthreads();  // the halo is no longer read: t takes its place
+    } else {
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const int ky = t / 3, kx = t - 3 * (t / 3);
+            u32x4 bv[NPW];
+#pragma unroll
+            for (int r = 0; r < NPW; ++r) {
+                const int pix = (r0 + r + ky) * HX + col + kx;
+                bv[r] = s_h[pix * UPP + (qb ^ (pix & (UPP - 1)))];
+                if (grp >= UG) bv[r] = u32x4{0u, 0u, 0u, 0u};  // 16-bit: K lanes 16..31 are padding
+            }
+            mma_rows<T, NPW>(acc, a1[t], bv);
+        }
     }
     // t (channel gi * 16 + 4 grp + k at position (r0 + r) * 16 + col) rounded to the storage type.
 #pragma unroll
@@ -136,7 +178,7 @@ __global__ void __launch_bounds__(256) k_resau(const ResauArgs p) {
     f32x4 acc2[NPW];
 #pragma unroll
     for (int r = 0; r < NPW; ++r) acc2[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
+#pragma unroll(F32 ? 1 : NC2)
     for (int c = 0; c < NC2; ++c) {
         u32x4 bv[NPW];
 #pragma unroll
@@ -144,7 +186,7 @@ __global__ void __launch_bounds__(256) k_resau(const ResauArgs p) {
             const int pos = (r0 + r) * 16 + col;
             bv[r] = s_t[pos * UPP + ((c * 4 + grp) ^ (pos & (UPP - 1)))];
         }
-        mma_rows<T, NPW>(acc2, a2[c], bv);
+        mma_rows<T, NPW>(acc2, F32 ? w2[((c * p.nblk2 + gi) * 16 + col) * 4 + grp] : a2[F32 ? 0 : c], bv);
     }
     T* yb = (T*)p.y.p + (long long)b * p.y.bstride + p.y.c_off;
     const int ch = gi * 16 + 4 * grp;
@@ -177,13 +219,8 @@ hipError_t go_resau(ResauArgs p, hipStream_t s) {
 
 template <typename T>
 hipError_t go_resau_t(int C, int tr, const ResauArgs& p, hipStream_t s) {
-    if constexpr (sizeof(T) == 4) {
-        if (C == 32) return go_resau<T, 32, 8>(p, s);
-        if (C == 64) return go_resau<T, 64, 8>(p, s);
-    } else {
-        if (C == 32) return tr == 8 ? go_resau<T, 32, 8>(p, s) : go_resau<T, 32, 4>(p, s);
-        if (C == 64) return tr == 8 ? go_resau<T, 64, 8>(p, s) : go_resau<T, 64, 4>(p, s);
-    }
+    if (C == 32) return tr == 8 ? go_resau<T, 32, 8>(p, s) : go_resau<T, 32, 4>(p, s);
+    if (C == 64) return tr == 8 ? go_resau<T, 64, 8>(p, s) : go_resau<T, 64, 4>(p, s);
     return hipErrorInvalidValue;
 }
 
@@ -191,12 +228,10 @@ hipError_t go_resau_t(int C, int tr, const ResauArgs& p, hipStream_t s) {
 
 bool resau_fused_supported(int C, int groups) { return (C == 32 || C == 64) && groups * 16 == C; }
 
-int resau_rows(int dtype, int N, int h, int w) {
-    // 8-row tiles unless that leaves fewer than 256 workgroups (one per CU). f32 keeps 8 rows:
-    // with the fewer accumulators of 4-row tiles the compiler renamed MFMA accumulator chains
-    // closer than the ISA guard allows.
+int resau_rows(int N, int h, int w) {
+    // 8-row tiles unless that leaves fewer than 256 workgroups (one per CU).
     const long long t8 = (long long)((w + 15) / 16) * ((h + 7) / 8) * N;
-    return (t8 >= 256 || dtype == DT_F32) ? 8 : 4;
+    return t8 >= 256 ? 8 : 4;
 }
 
 hipError_t launch_resau(int dtype, int C, const ResauArgs& p, hipStream_t s) {
@@ -204,9 +239,9 @@ hipError_t launch_resau(int dtype, int C, const ResauArgs& p, hipStream_t s) {
     if (p.N < 1 || p.N > MAXB || p.h < 1 || p.w < 1 || p.x.cs % vec || p.x.c_off % vec || p.x.row % vec ||
         p.x.bstride % vec || p.y.cs % vec || p.y.c_off % vec || (uintptr_t)p.x.p % 16 || (uintptr_t)p.y.p % 16)
         return hipErrorInvalidValue;
-    const int tr = resau_rows(dtype, p.N, p.h, p.w);
+    const int tr = resau_rows(p.N, p.h, p.w);
     switch (dtype) {
-        case DT_F32: return go_resau_t<float>(C, 8, p, s);
+        case DT_F32: return go_resau_t<float>(C, tr, p, s);
         case DT_F16: return go_resau_t<_Float16>(C, tr, p, s);
         case DT_BF16: return go_resau_t<__bf16>(C, tr, p, s);
     }

@@ -213,6 +213,9 @@ static uint16_t f32_to_bf16_bits(float v) {
     return (uint16_t)(r >> 16);
 }
 
+// Largest f32 that rounds to a finite bf16 (SPLIT_MAX of split.h).
+static constexpr float SPLIT_MAX_HOST = 3.39531337e38f;
+
 // The f32 value of a storage-dtype weight (f16 / bf16 upcasts are exact).
 static float storage_value(float v, int dtype) {
     if (dtype == DT_F32) return v;
@@ -262,6 +265,58 @@ static void* upload_as(Context& ctx, const std::vector<float>& host, int dtype, 
     return dev;
 }
 
+// A packed f32 weight ([..][16 outputs][16 channels] blocks) as three bf16 pieces per value in
+// the fragment order of split.h: per block the 64 lanes' (p1 x4, p0 x4), then their p2 x4, lane =
+// 16 * (channel / 4) + output. A value that is not finite as bf16 is kept whole in p2.
+static void* upload_split(const std::vector<float>& host, size_t* bytes_out, size_t* total) {
+    // Round to nearest even; v is finite as bf16 or NaN / infinite (whose low bits do not round up).
+    auto rne = [](float v) {
+        uint32_t b;
+        std::memcpy(&b, &v, 4);
+        const bool nan = (b & 0x7fffffff) > 0x7f800000;
+        const uint32_t r = (b + 0x7fff + ((b >> 16) & 1)) & 0xffff0000u;
+        return nan ? (b | 0x400000u) & 0xffff0000u : r;
+    };
+    auto f = [](uint32_t b) {
+        float v;
+        std::memcpy(&v, &b, 4);
+        return v;
+    };
+    const size_t nblk = host.size() / 256;
+    std::unique_ptr<uint16_t[]> h(new uint16_t[nblk * 768]);
+    for (size_t b = 0; b < nblk; ++b) {
+        uint16_t* lo = h.get() + b * 768;
+        uint16_t* hi = lo + 512;
+        for (int r = 0; r < 16; ++r) {
+            const float* src = host.data() + b * 256 + r * 16;
+            uint16_t p0[16], p1[16], p2[16];
+            for (int c = 0; c < 16; ++c) {  // one row of 16 channels, branch-free
+                const float v = src[c];
+                const bool fin = std::fabs(v) <= SPLIT_MAX_HOST;
+                const uint32_t b0 = rne(fin ? v : 0.0f);
+                const float r1 = v - f(b0);
+                const uint32_t b1 = rne(fin ? r1 : 0.0f);
+                p0[c] = (uint16_t)(b0 >> 16);
+                p1[c] = (uint16_t)(b1 >> 16);
+                p2[c] = (uint16_t)(rne(r1 - f(b1)) >> 16);
+            }
+            for (int q = 0; q < 4; ++q) {
+                const int lane = q * 16 + r;
+                std::memcpy(lo + lane * 8, p1 + 4 * q, 8);
+                std::memcpy(lo + lane * 8 + 4, p0 + 4 * q, 8);
+                std::memcpy(hi + lane * 4, p2 + 4 * q, 8);
+            }
+        }
+    }
+    const size_t bytes = nblk * 1536;
+    void* dev = nullptr;
+    ZJAI_HIP(hipMalloc(&dev, bytes));
+    ZJAI_HIP(hipMemcpy(dev, h.get(), bytes, hipMemcpyHostToDevice));
+    *bytes_out = bytes;
+    *total += *bytes_out;
+    return dev;
+}
+
 static float* upload_f32(const float* p, size_t n, size_t* total) {
     float* dev = nullptr;
     *total += n * 4;
@@ -296,6 +351,16 @@ void Layer::out_size(int h, int w, int* oh, int* ow) const {
 // each other's LDS and barrier waits: +2-3 % on the config-5 picture in every precision); fp32
 // 1x1 layers with >= 256 outputs the 8-wave 128-channel x 8-row tile (+2 % in fp32).
 TileCfg conv_tile_cfg(int cout_g, int kind, int dtype) {
+    if (conv_is_split(kind, dtype)) {  // the large-map shapes of conv_f32.hip
+        const bool wide = cout_g % 128 == 0;
+        if (kind == CK_3x3)
+            return cout_g <= 16 ? TileCfg{1, 4, 1, 2} : cout_g <= 32 ? TileCfg{1, 4, 2, 2}
+                   : wide ? TileCfg{2, 2, 4, 4} : TileCfg{1, 4, 4, 4};
+        if (kind == CK_3x3_S2)
+            return cout_g <= 16 ? TileCfg{1, 4, 1, 1} : cout_g <= 32 ? TileCfg{1, 4, 2, 1}
+                   : wide ? TileCfg{2, 2, 4, 2} : TileCfg{1, 4, 4, 2};
+        return cout_g <= 16 ? TileCfg{1, 8, 1, 1} : cout_g <= 32 ? TileCfg{1, 8, 2, 1} : TileCfg{1, 4, 4, 2};
+    }
     if (cout_g <= 16) return TileCfg{1, 4, 1, 2};
     if (cout_g <= 32) return TileCfg{1, 4, 2, 2};
     if (kind == CK_3x3) return TileCfg{2, 4, 2, 4};
@@ -347,16 +412,14 @@ LayerP make_conv(Context& ctx, int cin, int cout, int kh, int kw, int stride, in
     std::vector<float> pk((size_t)groups * L->nchunks * L->nblk_g * T * 16 * CK, 0.0f);
     for (int g = 0; g < groups; ++g)
         for (int ocl = 0; ocl < cout_g; ++ocl)
-            for (int icl = 0; icl < cin_g; ++icl)
-                for (int ky = 0; ky < kh; ++ky)
-                    for (int kx = 0; kx < kw; ++kx) {
-                        const int ch = icl / CK, kk = icl % CK, nb = ocl / 16, r = ocl % 16;
-                        const int t = ky * kw + kx;
-                        const size_t dst = ((((size_t)g * L->nchunks + ch) * L->nblk_g + nb) * T + t) * 16 * CK +
-                                           (size_t)r * CK + kk;
-                        pk[dst] = weight[(((size_t)(g * cout_g + ocl) * cin_g + icl) * kh + ky) * kw + kx];
-                    }
-    L->wpk = upload_as(ctx, pk, dtype, &L->wpk_bytes, &L->dev_bytes);
+            for (int icl = 0; icl < cin_g; ++icl) {
+                const int ch = icl / CK, kk = icl % CK, nb = ocl / 16, r = ocl % 16;
+                float* dst = pk.data() + (((size_t)g * L->nchunks + ch) * L->nblk_g + nb) * T * 16 * CK + (size_t)r * CK + kk;
+                const float* src = weight + ((size_t)(g * cout_g + ocl) * cin_g + icl) * T;
+                for (int t = 0; t < T; ++t) dst[(size_t)t * 16 * CK] = src[t];
+            }
+    L->wpk = conv_is_split(L->kind, dtype) ? upload_split(pk, &L->wpk_bytes, &L->dev_bytes)
+                                           : upload_as(ctx, pk, dtype, &L->wpk_bytes, &L->dev_bytes);
     if (dtype != DT_F32 && L->kind == CK_3x3 && groups == 1 && (cin == 64 || cin == 128) && cout % 64 == 0 && no_extra &&
         pad_h == 1 && pad_w == 1) {
         // conv3x3_m32's packing: [cin / 16][cout / mt][tap][channel half][mt][8].
@@ -512,6 +575,36 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
 
 // ------------------------------------------------------------------------------ conv launch
 // The kernel's name as profilers print it: conv_igemm<T, KH, KW, S, TR, WC, WP, CF, PF>.
+// Launch-time tile shape of an f32 layer on the bf16 matrix cores (conv_f32.hip; every shape gives
+// the same bits). Wide tiles read fewer LDS bytes per MFMA and split each halo value once for more
+// outputs; on a small map they leave CUs idle while each workgroup walks the whole K loop, so the
+// tile narrows with the number of 64-channel x 16-row (3x3) or x 8-row (stride 2, 2x2) workgroups.
+// The lines are where the per-layer sweep crosses (us, one launch):
+//   3x3 128 -> 128: 256^2 (512 workgroups) 128 ch x 8 rows 106, 64 x 8 114, 32 x 8 116, 16 x 8 143;
+//     176^2 (242) 75 / 60 / 62 / 75; 125^2 (128) 69 / 42 / 39 / 42; 88^2 (72) 66 / 38 / 34 / 29;
+//     52 x 76 (40) 16 x 8 by four waves 22.7, by eight waves of one row each 22.4; 160 -> 160 at
+//     40^2 (27) 22.3 / 18.6.
+//   stride 2, 128 -> 128: 432^2 (756) 128 ch x 4 rows 132, 64 x 4 134, 32 x 4 167; 256^2 (256)
+//     62 / 48 / 64; 172^2 (132) 58 / 43 / 43; 51 x 75 (24) 54 / 32 / 26, 16 x 4 19.
+//   2x2 160 -> 256: 135 x 240 (1020) 64 ch x 8 rows 74, 32 x 8 (eight waves) 91, 16 x 8 114; 64^2
+//     (128) 29 / 18 / 21; 144 -> 128 at 64^2 (64) 26 / 16 / 14.
+//   32-channel groups and outputs: 256^2 (512 of 32 x 8) 32 ch x 8 rows 16.1, 16 x 8 by eight waves
+//     18.0; five groups at 34 x 60 (100) 11.2 / 8.2.
+static TileCfg split_tile_cfg(const Layer& L, int N, int OH, int OW) {
+    const int nb = L.cfg.wc * L.cfg.cf;
+    const long long cols = (OW + 15) / 16, rows8 = (OH + 7) / 8, tiles = L.groups * (long long)(L.nblk_g / nb) * N;
+    if (L.kind == CK_3x3) {
+        if (nb <= 2) return cols * rows8 * tiles < (nb == 2 ? 256 : 512) ? TileCfg{1, 8, 1, 1} : L.cfg;
+        const long long w = cols * ((OH + 15) / 16) * (tiles * nb / 4);
+        return w < 56 ? TileCfg{1, 8, 1, 1} : w < 96 ? TileCfg{1, 4, 1, 2} : w < 200 ? TileCfg{1, 4, 2, 2}
+               : w < 384 ? TileCfg{1, 4, 4, 2} : L.cfg;
+    }
+    if (nb <= 2) return L.cfg;
+    const long long w = cols * rows8 * (tiles * nb / 4);
+    if (L.kind == CK_3x3_S2) return w < 48 ? TileCfg{1, 4, 1, 1} : w < 160 ? TileCfg{1, 4, 2, 1} : w < 512 ? TileCfg{1, 4, 4, 1} : L.cfg;
+    return w < 96 ? TileCfg{1, 8, 1, 1} : w < 384 ? TileCfg{1, 8, 2, 1} : L.cfg;
+}
+
 // Launch-time tile shape of a dense layer. The layer's own shape (64 channels x 16 or 8 rows)
 // suits large maps; on small ones its grid leaves most of the 256 CUs idle while each workgroup
 // walks the whole K loop, so narrower tiles (32 or 16 channels x 8 rows; the weights are packed
@@ -522,18 +615,18 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
 // (512 tiles) the 16-row tile stays fastest.
 static TileCfg launch_tile_cfg(const Layer& L, int N, int OH, int OW) {
     const TileCfg c = L.cfg;
+    if (conv_is_split(L.kind, L.dtype)) return split_tile_cfg(L, N, OH, OW);
     if (L.groups != 1) return c;
     const long long nt4 = L.nblk_g / 4;
     if (L.kind == CK_3x3 && c.wc == 2 && c.wp == 4 && c.cf == 2 && c.pf == 4) {
         const long long w0 = (long long)((OW + 15) / 16) * ((OH + 15) / 16) * N * nt4;
-        if (L.dtype == DT_F32) return w0 < 256 ? TileCfg{1, 4, 1, 2} : c;
         return w0 < 64 ? TileCfg{1, 4, 1, 2} : w0 < 256 ? TileCfg{1, 4, 2, 2} : c;
     }
     if (L.kind == CK_3x3_S2 && c.wc == 2 && c.wp == 2 && c.cf == 2 && c.pf == 4) {
         const long long w0 = (long long)((OW + 15) / 16) * ((OH + 7) / 8) * N * nt4;
         if (w0 < 128) return TileCfg{1, 4, 1, 2};
-        // 16-bit: 128-channel tiles (8 waves) share each staged halo between twice the outputs.
-        if (L.dtype != DT_F32 && L.nblk_g % 8 == 0 && w0 >= 512) return TileCfg{4, 2, 2, 4};
+        // 128-channel tiles (8 waves) share each staged halo between twice the outputs.
+        if (L.nblk_g % 8 == 0 && w0 >= 512) return TileCfg{4, 2, 2, 4};
         return c;
     }
     if (L.kind == CK_2x2 && c.wc == 2 && c.wp == 2 && c.cf == 2 && c.pf == 4) {
@@ -565,6 +658,10 @@ std::string conv_kernel_name(int kind, int dtype, TileCfg c) {
                                 "3, 3, 1, true"};
     static const char* ty[] = {"float", "_Float16", "__bf16"};
     char buf[128];
+    if (conv_is_split(kind, dtype)) {
+        snprintf(buf, sizeof buf, "conv_igemm_split<%s, %d, %d, %d, %d>", geo[kind], c.wc, c.wp, c.cf, c.pf);
+        return buf;
+    }
     const bool dma = dtype == DT_F32 && c.cf == 2 && c.pf == 4 &&
                      ((c.wc == 2 && (c.wp == 2 || c.wp == 4)) || (c.wc == 4 && c.wp == 2));
     if (dma)  // the fp32 dense shapes run conv_dma_f32 (conv.hip)
@@ -745,7 +842,8 @@ static TensorP conv_forward_impl(Context& ctx, const Layer& L, const TensorP& x,
     const TileCfg cfg = launch_tile_cfg(L, N, OH, OW);
     p.ntiles = L.groups * L.nblk_g / (cfg.wc * cfg.cf);
     LaunchScope sc(ctx, conv_kernel_name(L.kind, L.dtype, cfg), 2.0 * macs, bytes);
-    ZJAI_HIP(launch_conv(L.kind, L.dtype, cfg, p, ctx.stream));
+    if (conv_is_split(L.kind, L.dtype)) ZJAI_HIP(launch_conv_split(L.kind, cfg, p, ctx.stream));
+    else ZJAI_HIP(launch_conv(L.kind, L.dtype, cfg, p, ctx.stream));
     return y;
 }
 

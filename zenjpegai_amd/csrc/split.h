@@ -1,0 +1,103 @@
+// f32 products on the bf16 matrix cores (gfx950).
+//
+// An f32 value is the exact sum of three bf16 pieces, v = p0 + p1 + p2 (8 significant bits each,
+// rounded to nearest, so |p1| <= 2^-9 |v| and |p2| <= 2^-18 |v|). Of the nine piece products of
+// a * b the six largest carry everything down to 2^-26 of the product -- below half an ulp of the
+// f32 product -- so a sum of products takes six bf16 multiply-adds per f32 one, at sixteen times
+// the rate: v_mfma_f32_16x16x32_bf16 measured 1.95 PFLOP/s on registers, i.e. 325 TFLOP/s of f32
+// products, against 136-150 TFLOP/s for v_mfma_f32_16x16x4_f32, and unlike the f32 form it runs
+// beside vector work.
+//
+// A lane holds four channels of an operand as six registers [p1 x4 | p0 x4 | p2 x4]: its first
+// four (`lo`) are the pieces (p1, p0), its last four (`hi`) the pieces (p0, p2), each the eight K
+// slots of one 16x16x32 MFMA. With A = (a1, a0, a2) and B = (b1, b0, b2) the six products are
+//   lo . lo = a1 b1 + a0 b0,   lo . hi = a1 b0 + a0 b2,   hi . lo = a0 b1 + a2 b0,
+// so one MFMA triple covers 16 channels of K and the packing stays 16 channels per chunk.
+//
+// The first goes to one accumulator, the two small ones to another, added once at the end: the
+// matrix core rounds its accumulator once per 8 products, so the full-size sum is rounded K / 4
+// times where the f32 MFMA rounds it K times (K = 1152, against 64-bit sums: 3e-7 relative
+// instead of 4-6e-7).
+//
+// A value that is not finite (or above bf16's largest, 3.395e38) keeps its whole in p2, which
+// only ever meets b0: infinities and NaN then reach the result as in f32 arithmetic. Values below
+// 2^-110 lose low bits (the pieces become subnormal).
+#pragma once
+
+#include "mfma.h"
+
+namespace zjai {
+
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// Largest f32 that rounds to a finite bf16.
+constexpr float SPLIT_MAX = 3.39531337e38f;
+
+struct SplitFrag {
+    u32x4 lo;  // p1 of channels 0..3, p0 of channels 0..3
+    u32x2 hi;  // p2 of channels 0..3
+};
+
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+    bf16x2 r;
+    r[0] = (__bf16)a;
+    r[1] = (__bf16)b;
+    return __builtin_bit_cast(unsigned, r);
+}
+
+__device__ __forceinline__ SplitFrag split_f32(f32x4 v) {
+    SplitFrag f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const float x = v[2 * h], y = v[2 * h + 1];
+        const bool fx = __builtin_fabsf(x) <= SPLIT_MAX, fy = __builtin_fabsf(y) <= SPLIT_MAX;
+        const unsigned p0 = pack_bf16(fx ? x : 0.0f, fy ? y : 0.0f);
+        const float rx = x - __builtin_bit_cast(float, p0 << 16);
+        const float ry = y - __builtin_bit_cast(float, p0 & 0xffff0000u);
+        const unsigned p1 = pack_bf16(fx ? rx : 0.0f, fy ? ry : 0.0f);
+        f.lo[h] = p1;
+        f.lo[2 + h] = p0;
+        f.hi[h] = pack_bf16(rx - __builtin_bit_cast(float, p1 << 16), ry - __builtin_bit_cast(float, p1 & 0xffff0000u));
+    }
+    return f;
+}
+
+// big += lo . lo, small += the other two MFMAs (16 channels of K).
+__device__ __forceinline__ f32x4 mfma_bf16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ u32x4 split_hi(const SplitFrag& f) { return u32x4{f.lo[2], f.lo[3], f.hi[0], f.hi[1]}; }
+__device__ __forceinline__ void mma_split(f32x4& big, f32x4& small, const SplitFrag& a, const SplitFrag& b) {
+    big = mfma_bf16(a.lo, b.lo, big);
+    small = mfma_bf16(a.lo, split_hi(b), small);
+    small = mfma_bf16(split_hi(a), b.lo, small);
+}
+
+// mma_split for N accumulator pairs sharing A, one MFMA of the triple at a time over all of them.
+template <int N>
+__device__ __forceinline__ void mma_split_rows(f32x4 (&big)[N], f32x4 (&small)[N], const SplitFrag& a, const SplitFrag (&b)[N]) {
+    const u32x4 ahi = split_hi(a);
+#pragma unroll
+    for (int r = 0; r < N; ++r) small[r] = mfma_bf16(a.lo, split_hi(b[r]), small[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) big[r] = mfma_bf16(a.lo, b[r].lo, big[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) small[r] = mfma_bf16(ahi, b[r].lo, small[r]);
+}
+
+// The sum of a finished pair of accumulators. An infinite full-size sum stays infinite: its small
+// products may have overflowed to either sign.
+__device__ __forceinline__ f32x4 split_sum(f32x4 big, f32x4 small) {
+    f32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = __builtin_isinf(big[i]) ? big[i] : big[i] + small[i];
+    return r;
+}
+
+// A packed 16 x 16 weight block (16 outputs x 16 input channels) in split form: 96 16-byte
+// units, the `lo` of the 64 lanes of an A fragment (lane = 16 * (channel / 4) + output), then
+// their `hi`s.
+constexpr int SPLIT_BLOCK_U = 96;
+
+}  // namespace zjai
