@@ -4,9 +4,10 @@ are not finite.
 
 Bound: the matrix core rounds its f32 accumulator once per 8 products; the full-size accumulator
 takes 16 of the K products per 4 such roundings, its partner's are 2^-8 smaller, the pieces drop
-2^-26 of a product, and bias, final sum and store add three roundings. Every rounding is at most
-2^-23 (it may truncate) of a partial sum, itself at most S = |b| + sum |x w|, so
-|err| <= (K / 4 * (1 + 2^-7) + 4) * 2^-23 * S."""
+2^-26 of a product, and bias, final sum and store add three roundings; a 1x1 layer adds the two
+accumulators every 32 products. Every rounding is at most 2^-23 (it may truncate) of a partial sum,
+itself at most S = |b| + sum |x w|, so |err| <= (K / 4 * (1 + 2^-7) + 4 + [1x1] (K / 32 + 1)) *
+2^-23 * S."""
 
 import numpy as np
 import pytest
@@ -26,14 +27,14 @@ def eng():
 
 
 def _layer(eng, kind, cin, cout, groups, seed):
-    k, stride = {"3x3": (3, 1), "s2": (3, 2), "2x2": (2, 1)}[kind]
+    k, stride = {"1x1": (1, 1), "3x3": (3, 1), "s2": (3, 2), "2x2": (2, 1)}[kind]
     w = synth.normal(seed, f"split/w{kind}{cin}{cout}", (cout, cin // groups, k, k), 1.0)
     b = synth.normal(seed, f"split/b{cout}", (cout,), 1.0)
-    pad, ext = ((0, 0), (0, 0, 1, 1)) if kind == "2x2" else ((1, 1), (0, 0, 0, 0))
+    pad, ext = {"1x1": ((0, 0), (0, 0, 0, 0)), "2x2": ((0, 0), (0, 0, 1, 1))}.get(kind, ((1, 1), (0, 0, 0, 0)))
 
     def ref(x, w, b):
         x = torch.from_numpy(x).double()[None]
-        x = F.pad(x, (0, 1, 0, 1) if kind == "2x2" else (1, 1, 1, 1))
+        x = F.pad(x, {"1x1": (0, 0, 0, 0), "2x2": (0, 1, 0, 1)}.get(kind, (1, 1, 1, 1)))
         return F.conv2d(x, torch.from_numpy(w).double(), torch.from_numpy(b).double(), stride, 0, 1, groups)[0].numpy()
 
     return w, b, lambda w, b: nn.ConvLayer(nn.Conv2d(cin, cout, (k, k), stride, pad, groups, w, b), eng, extra_pad=ext), ref
@@ -47,7 +48,9 @@ CASES = [("3x3", 4, 4, 1, 1, 1), ("3x3", 20, 24, 1, 9, 17), ("3x3", 160, 160, 1,
          ("3x3", 128, 128, 4, 15, 16), ("3x3", 128, 128, 4, 150, 161), ("s2", 20, 16, 1, 1, 7), ("s2", 64, 64, 1, 35, 33),
          ("s2", 24, 32, 1, 66, 64), ("s2", 64, 64, 1, 175, 177), ("s2", 16, 128, 1, 255, 257), ("s2", 16, 128, 1, 440, 431),
          ("s2", 16, 192, 1, 440, 431), ("2x2", 160, 256, 1, 4, 6), ("2x2", 20, 12, 1, 17, 15), ("2x2", 64, 128, 1, 128, 127),
-         ("2x2", 16, 192, 1, 150, 161)]
+         ("2x2", 16, 192, 1, 150, 161), ("1x1", 4, 4, 1, 1, 1), ("1x1", 20, 24, 1, 9, 7), ("1x1", 48, 16, 1, 33, 64),
+         ("1x1", 160, 160, 1, 8, 15), ("1x1", 128, 64, 1, 128, 127), ("1x1", 96, 128, 1, 150, 130),
+         ("1x1", 32, 256, 1, 171, 190)]
 
 
 @pytest.mark.parametrize("kind,cin,cout,groups,h,w", CASES)
@@ -58,11 +61,11 @@ def test_error_against_64_bits(eng, kind, cin, cout, groups, h, w):
     want, size = ref(x, wt, b), ref(np.abs(x), np.abs(wt), np.abs(b))
     assert y.shape == want.shape
     kk = wt[0].size
-    bound = (kk / 4 * (1 + 2.0 ** -7) + 4) * 2.0 ** -23 * size
+    bound = (kk / 4 * (1 + 2.0 ** -7) + 4 + (kk / 32 + 1 if kind == "1x1" else 0)) * 2.0 ** -23 * size
     assert np.all(np.abs(y - want) <= bound), float(np.max(np.abs(y - want) / bound))
 
 
-@pytest.mark.parametrize("kind", ["3x3", "s2", "2x2"])
+@pytest.mark.parametrize("kind", ["1x1", "3x3", "s2", "2x2"])
 def test_values_that_are_not_finite(eng, kind):
     """Infinities and NaN in the input or the weights reach the outputs that f32 arithmetic sends
     them to, and only those."""

@@ -82,7 +82,11 @@ TensorP planar_upload(Context& c, const float* data, int ch, int h, int w, int d
 // process ends. In host code `scratch` is a host-side stand-in, not device memory: the array's
 // address on a device comes from hipGetSymbolAddress (scratch_setup, called by zjai_ctx_create
 // with that device current) and only that address is passed to kernels.
-static __device__ __align__(256) unsigned char scratch[ZJAI_NOALLOC_SCRATCH_BYTES];
+// The bytes past ZJAI_NOALLOC_SCRATCH_BYTES hold the third bf16 piece of an f32 call's folded
+// weight (half its f32 size; dim <= 639 by the Gram kernel's LDS stage), so that maps up to the
+// documented size fit as they do in f32 form.
+constexpr size_t SCRATCH_PIECE_BYTES = 1u << 20;
+static __device__ __align__(256) unsigned char scratch[ZJAI_NOALLOC_SCRATCH_BYTES + SCRATCH_PIECE_BYTES];
 
 namespace {
 
@@ -492,12 +496,13 @@ extern "C" int32_t zjai_channel_attention_noalloc(zjai_ctx* ctx, const void* qkv
         const int es = dtype_size(precision), CK = 64 / es;
         const TileCfg cfg = conv_tile_cfg(dim, CK_1x1, precision);
         const int nblk = round_up(ceil_div(dim, 16), cfg.wc * cfg.cf), nchunks = ceil_div(dim, CK);
-        const size_t w_bytes = (size_t)nchunks * nblk * 16 * CK * es;
+        const size_t w_plain = (size_t)nchunks * nblk * 16 * CK * es;
+        const size_t w_bytes = conv_is_split(CK_1x1, precision) ? w_plain / 2 * 3 : w_plain;
         // Scratch layout: Gram partials [nchunk][heads][c*c + 2c] f32 | attn [dim][c] f32 | weight.
         const int nchunk = attention_gram_chunks(h, w);
         const size_t part_bytes = (size_t)nchunk * heads * (c * c + 2 * c) * 4;
         const size_t attn_off = round_up256(part_bytes), w_off = round_up256(attn_off + (size_t)dim * c * 4);
-        if (w_off + w_bytes > ZJAI_NOALLOC_SCRATCH_BYTES)
+        if (w_off + w_plain > ZJAI_NOALLOC_SCRATCH_BYTES || w_bytes - w_plain > SCRATCH_PIECE_BYTES)
             throw Error(ZJAI_E_LIMIT, "attention: the map needs more than the allocation-free scratch");
         unsigned char* base = scratch_of(ctx->c.device);
         if (!base) throw Error(ZJAI_E_DEVICE, "allocation-free scratch not set up for this device");
@@ -547,8 +552,15 @@ extern "C" int32_t zjai_channel_attention_noalloc(zjai_ctx* ctx, const void* qkv
         p.ps = 1;
         p.out_mode = OUT_NHWC;
         p.sv = p.sh = 1;
-        LaunchScope sc(C, conv_kernel_name(CK_1x1, precision, cfg), 2.0 * n * dim * dim, es * 2.0 * n * dim + (double)w_bytes);
-        ZJAI_HIP(launch_conv(CK_1x1, precision, cfg, p, C.stream));
+        const double flops = 2.0 * n * dim * dim, bytes = es * 2.0 * n * dim + (double)w_bytes;
+        if (conv_is_split(CK_1x1, precision)) {  // views of a dim % 8 == 0 map on 16-byte buffers: always aligned
+            const TileCfg c1 = ring_split_cfg(nblk, (long long)h * w, 1);
+            LaunchScope sc(C, ring_split_name(c1), flops, bytes);
+            ZJAI_HIP(launch_conv1x1_ring_split(c1, p, C.stream));
+        } else {
+            LaunchScope sc(C, conv_kernel_name(CK_1x1, precision, cfg), flops, bytes);
+            ZJAI_HIP(launch_conv(CK_1x1, precision, cfg, p, C.stream));
+        }
     });
 }
 

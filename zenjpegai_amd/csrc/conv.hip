@@ -1327,10 +1327,9 @@ static hipError_t go(const ConvParams& p0, hipStream_t s) {
 
 template <typename T, int WC, int WP, int CF, int PF>
 static hipError_t go_kind(int kind, const ConvParams& p, hipStream_t s) {
-    if constexpr (sizeof(T) == 4) {
-        if (kind != CK_1x1 && kind != CK_T3) return hipErrorInvalidValue;  // launch_conv_split's
-        return kind == CK_1x1 ? go<T, 1, 1, 1, false, WC, WP, CF, PF>(p, s) : go<T, 3, 3, 1, true, WC, WP, CF, PF>(p, s);
-    } else
+    if constexpr (sizeof(T) == 4)  // every other kind is launch_conv_split's
+        return kind == CK_T3 ? go<T, 3, 3, 1, true, WC, WP, CF, PF>(p, s) : hipErrorInvalidValue;
+    else
     switch (kind) {
         case CK_1x1: return go<T, 1, 1, 1, false, WC, WP, CF, PF>(p, s);
         case CK_2x2: return go<T, 2, 2, 1, false, WC, WP, CF, PF>(p, s);
@@ -1344,7 +1343,7 @@ static hipError_t go_kind(int kind, const ConvParams& p, hipStream_t s) {
 // Instantiated tile shapes: (wc, wp, cf, pf).
 //   {2,2,2,4}: 64 channels x 8 rows, 4 waves  (dense layers)
 //   {2,4,2,4}: 64 channels x 16 rows, 8 waves (dense stride-1 3x3 layers only)
-//   {4,2,2,4}: 128 channels x 8 rows, 8 waves (fp32 1x1 layers with >= 256 outputs only)
+//   {4,2,2,4}: 128 channels x 8 rows, 8 waves (16-bit stride-2 3x3 layers only)
 //   {1,4,2,2}: 32 channels x 8 rows  (32-channel groups / outputs)
 //   {1,4,1,2}: 16 channels x 8 rows  (16-channel groups / narrow outputs)
 #define ZJAI_CFGS(X) X(2, 2, 2, 4) X(1, 4, 2, 2) X(1, 4, 1, 2)
@@ -1353,10 +1352,8 @@ template <typename T>
 static hipError_t go_cfg(int kind, TileCfg c, const ConvParams& p, hipStream_t s) {
     if (c.wc == 2 && c.wp == 4 && c.cf == 2 && c.pf == 4)
         return sizeof(T) == 2 && kind == CK_3x3 ? go<std::conditional_t<sizeof(T) == 2, T, __bf16>, 3, 3, 1, false, 2, 4, 2, 4>(p, s) : hipErrorInvalidValue;
-    if (c.wc == 4 && c.wp == 2 && c.cf == 2 && c.pf == 4) {
-        if constexpr (sizeof(T) == 4) return kind == CK_1x1 ? go<T, 1, 1, 1, false, 4, 2, 2, 4>(p, s) : hipErrorInvalidValue;
-        else return kind == CK_3x3_S2 ? go<T, 3, 3, 2, false, 4, 2, 2, 4>(p, s) : hipErrorInvalidValue;
-    }
+    if (c.wc == 4 && c.wp == 2 && c.cf == 2 && c.pf == 4)
+        return sizeof(T) == 2 && kind == CK_3x3_S2 ? go<std::conditional_t<sizeof(T) == 2, T, __bf16>, 3, 3, 2, false, 4, 2, 2, 4>(p, s) : hipErrorInvalidValue;
 #define ZJAI_GO(a, b, cc, d) \
     if (c.wc == a && c.wp == b && c.cf == cc && c.pf == d) return go_kind<T, a, b, cc, d>(kind, p, s);
     ZJAI_CFGS(ZJAI_GO)

@@ -1,10 +1,10 @@
 // 1x1 convolutions (stride 1, no padding, one group) as a GEMM: output channels x positions,
-// K = input channels, in every storage type.
+// K = input channels, in the 16-bit storage types (f32: conv_f32.hip).
 //
 // A workgroup of WC x WP waves computes NB * 16 output channels (NB = WC * CF 16-channel
 // blocks) for MP = WP * PF * 16 consecutive positions of one batch item (positions are the
 // row-major pixel index of the output map, so narrow maps waste no lanes). The K loop streams
-// 64 bytes of input channels per position per chunk (16 f32 or 32 f16 / bf16 channels) with
+// 64 bytes of input channels per position per chunk (32 channels) with
 // direct global -> LDS loads (global_load_lds_dwordx4: lane i's 16 bytes land at the wave's LDS
 // base + 16 i) through a ring of NS chunk slots, one barrier per chunk, NS - 2 chunks in flight
 // behind the one being consumed. A position's 64 bytes are read by 4 consecutive lanes as one
@@ -14,15 +14,13 @@
 // run per chunk.
 //
 // Numerics are those of the implicit-GEMM kernels for a 1x1 layer, so the two agree bit for
-// bit: the bias first, then chunk by chunk in ascending order; f32 as four
-// v_mfma_f32_16x16x4_f32 per chunk (k = 0..3, the K group of lane group g holding channels
-// 4g + k), f16 / bf16 as one v_mfma_f32_16x16x32 per chunk (lane group g holding channels
-// 8g..8g+7). The epilogue is the shared one (epilogue.h) through an LDS transpose.
+// bit: the bias first, then chunk by chunk in ascending order, one v_mfma_f32_16x16x32 per chunk
+// (lane group g holding channels 8g..8g+7). The epilogue is the shared one (epilogue.h) through an
+// LDS transpose.
 //
-// On the config-5 layer shapes (202 500 positions) this runs within 10-20 % of the vendor BLAS
-// on the same plain GEMM (f32 128 -> 1024: 663 vs 608 us; bf16 128 -> 384: 74 vs 83 us) with
-// the residual epilogue fused; persistent workgroups with a ring across tiles and a variant
-// that loads the fragments straight into registers (no LDS, no barriers) were both slower.
+// Against the vendor BLAS on the same plain GEMM (202 500 positions, bf16 128 -> 384): 74 vs
+// 83 us with the residual epilogue fused; persistent workgroups with a ring across tiles and a
+// variant that loads the fragments straight into registers (no LDS, no barriers) were both slower.
 
 #include "conv.h"
 #include "epilogue.h"
@@ -156,23 +154,10 @@ conv1x1_ring(const ConvParams p) {
             const int pos = bpos[pf];
             bv[pf] = sb[pos * 4 + (grp ^ ((pos & 4) >> 1))];
         }
-        if constexpr (sizeof(T) == 4) {
-            // k outermost: the four dependent MFMAs of an accumulator are CF x PF apart.
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
+        for (int cf = 0; cf < CF; ++cf)
 #pragma unroll
-                for (int cf = 0; cf < CF; ++cf)
-#pragma unroll
-                    for (int pf = 0; pf < PF; ++pf)
-                        acc[cf][pf] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f32x4, av[cf])[k],
-                                                                           __builtin_bit_cast(f32x4, bv[pf])[k],
-                                                                           acc[cf][pf], 0, 0, 0);
-        } else {
-#pragma unroll
-            for (int cf = 0; cf < CF; ++cf)
-#pragma unroll
-                for (int pf = 0; pf < PF; ++pf) Mma16<T>::run(acc[cf][pf], av[cf], bv[pf]);
-        }
+            for (int pf = 0; pf < PF; ++pf) Mma16<T>::run(acc[cf][pf], av[cf], bv[pf]);
     }
 
     // Epilogue: transpose through LDS so that consecutive threads store consecutive channels of
@@ -249,8 +234,8 @@ static hipError_t go_1x1(const ConvParams& p0, hipStream_t s) {
 static bool aligned4(const View& v) { return !(v.cs % 4) && !(v.c_off % 4) && !(v.row % 4) && !(v.bstride % 4); }
 
 bool conv1x1_ring_ok(const ConvParams& p, int dtype) {
-    const int vec = dtype == DT_F32 ? 4 : 8;
-    return p.groups == 1 && p.N >= 1 && p.N <= MAXB && !p.relu6_in && p.H == p.OH && p.W == p.OW &&
+    constexpr int vec = 8;
+    return dtype != DT_F32 && p.groups == 1 && p.N >= 1 && p.N <= MAXB && !p.relu6_in && p.H == p.OH && p.W == p.OW &&
            p.pad_t == 0 && p.pad_l == 0 && p.cin_g % (4 * vec) == 0 && p.nchunks * 4 * vec == p.cin_g &&
            p.cout_g % 64 == 0 && p.nblk_g % 4 == 0 && p.x.cs % vec == 0 && p.x.c_off % vec == 0 &&
            p.x.row % vec == 0 && p.x.bstride % vec == 0 && aligned4(p.y) && (!p.r1.p || aligned4(p.r1)) &&
@@ -261,25 +246,17 @@ int conv1x1_ring_nb(const ConvParams& p) { return (p.cout_g % 128 == 0 && p.nblk
 
 template <typename T>
 static hipError_t go_1x1_t(const ConvParams& p, hipStream_t s) {
-    // Co-resident workgroups cover each other's prologue and epilogue. f32: a ring of 3 chunks and
-    // two epilogue passes (48 KB of LDS, <= 168 registers: 3 workgroups per CU); 16-bit, whose
-    // layers are HBM-bound: a ring of 2 and four passes (32 KB, <= 128 registers: 4 per CU).
-    // Against a ring of 4 and one pass (2 per CU) on 202 500 positions: f32 128 -> 1024 664 ->
-    // 617 us, 128 -> 384 268 -> 239 us; bf16 128 -> 1024 223 -> 172 us, 512 -> 128 85 -> 74 us,
-    // 128 -> 384 76 -> 55 us (4 per CU: f32 no better, bf16 a further 7-10 %).
-    if constexpr (sizeof(T) == 4) {
-        if (conv1x1_ring_nb(p) == 8) return go_1x1<T, 2, 2, 4, 4, 3, 2, 3>(p, s);  // 128 ch x 128 positions
-        return go_1x1<T, 1, 4, 4, 2, 3, 2, 3>(p, s);                                 // 64 ch x 128 positions
-    } else {
-        if (conv1x1_ring_nb(p) == 8) return go_1x1<T, 2, 2, 4, 4, 2, 4, 4>(p, s);
-        return go_1x1<T, 1, 4, 4, 2, 2, 4, 4>(p, s);
-    }
+    // Co-resident workgroups cover each other's prologue and epilogue; the layers are HBM-bound: a
+    // ring of 2 and four passes (32 KB, <= 128 registers: 4 per CU). Against a ring of 4 and one
+    // pass (2 per CU) on 202 500 positions, bf16: 128 -> 1024 223 -> 172 us, 512 -> 128 85 -> 74 us,
+    // 128 -> 384 76 -> 55 us.
+    if (conv1x1_ring_nb(p) == 8) return go_1x1<T, 2, 2, 4, 4, 2, 4, 4>(p, s);
+    return go_1x1<T, 1, 4, 4, 2, 2, 4, 4>(p, s);
 }
 
 hipError_t launch_conv1x1_ring(int dtype, const ConvParams& p, hipStream_t s) {
     if (!conv1x1_ring_ok(p, dtype)) return hipErrorInvalidValue;
     switch (dtype) {
-        case DT_F32: return go_1x1_t<float>(p, s);
         case DT_F16: return go_1x1_t<_Float16>(p, s);
         case DT_BF16: return go_1x1_t<__bf16>(p, s);
     }

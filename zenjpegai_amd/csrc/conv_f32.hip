@@ -135,7 +135,7 @@ conv_igemm_split(const ConvParams p) {
     // Weight slot of stage (chunk, j): taps j * TS .. of blocks nb0 .. nb0 + NB - 1, loaded RW - 1
     // stages ahead (the slot was last read that many stages ago). The lanes' offsets stay, the
     // uniform base moves.
-    const char* const wg = (const char*)((const u32x4*)p.w + ((long long)g * p.nchunks * p.nblk_g + nb0) * (NTAP * SPLIT_BLOCK_U));
+    const char* const wg = (const char*)((const u32x4*)((const float*)p.w + bi * p.w_bstride) + ((long long)g * p.nchunks * p.nblk_g + nb0) * (NTAP * SPLIT_BLOCK_U));
     const long long wchunk = (long long)p.nblk_g * (NTAP * SPLIT_BLOCK_U * 16);
     unsigned woff[WN];
 #pragma unroll
@@ -204,6 +204,15 @@ conv_igemm_split(const ConvParams p) {
 #pragma unroll
                     for (int pf = 0; pf < PF; ++pf) mma_split(big[cf][pf], small[cf][pf], a[cf], b[pf]);
             }
+            if (NTAP == 1 && ((chunk & 1) || chunk + 1 == nchunks)) {  // mma_split32's order
+#pragma unroll
+                for (int cf = 0; cf < CF; ++cf)
+#pragma unroll
+                    for (int pf = 0; pf < PF; ++pf) {
+                        big[cf][pf] += small[cf][pf];
+                        small[cf][pf] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+            }
         }
     }
 
@@ -215,7 +224,7 @@ conv_igemm_split(const ConvParams p) {
 #pragma unroll
         for (int pf = 0; pf < PF; ++pf)
             *reinterpret_cast<f32x4*>(so + ((wp * PF + pf) * 16 + col) * OUT_LD + (wc * CF + cf) * 16 + grp * 4) =
-                split_sum(big[cf][pf], small[cf][pf]);
+                NTAP == 1 ? big[cf][pf] : split_sum(big[cf][pf], small[cf][pf]);
     __syncthreads();
     const bool full = nb0 * 16 + NB * 16 <= p.cout_g;  // all of the tile's channels are real
     if (full && epilogue_simple(p)) {
@@ -255,13 +264,208 @@ conv_igemm_split(const ConvParams p) {
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// 1x1 layers as a GEMM over row-major positions: WC * CF blocks of 16 channels x MP = WP * PF * 16
+// consecutive positions of one batch item per workgroup, K in stages of 32 channels. A stage's
+// positions are loaded into registers one stage ahead (8 lanes read a position's 128 bytes), split
+// and stored to planes [8 channel quads][positions], position p of quad q at p ^ q: the eight
+// quads a store pass holds of one position, and the 16 positions x 2 quads of a fragment read
+// pass, fall on distinct banks. The weights stream through a two-slot ring of direct loads. Sums
+// are mma_split32's, so a layer gives the same bits here and in conv_igemm_split.
+//
+// Bound by its traffic at the 128-channel shapes (128 -> 512 at 450^2: 2.9 TB/s before, on the f32
+// MFMA) once the products run on the bf16 matrix cores.
+// ---------------------------------------------------------------------------------------------
+template <int WC, int WP, int CF, int PF>
+__global__ void __launch_bounds__(WC * WP * 64, 2)
+conv1x1_ring_split(const ConvParams p) {
+    constexpr int NT = WC * WP * 64;
+    constexpr int NB = WC * CF, MP = WP * PF * 16;
+    constexpr int PXS = (MP + 15) / 32 * 32 + 16;
+    constexpr int X_U = 8 * PXS * 3 / 2, W_U = NB * SPLIT_BLOCK_U;  // W_U: one chunk's blocks
+    constexpr int OUT_LD = NB * 16 + 4, OUT_U = (MP * OUT_LD + 3) / 4;
+    constexpr int RUN_U = X_U + 4 * W_U;
+    constexpr int LDS_U = RUN_U > OUT_U ? RUN_U : OUT_U;
+    constexpr int XN = MP * 8 / NT, WN = (W_U + NT - 1) / NT;
+    static_assert(MP * 8 % NT == 0, "whole loads");
+    __shared__ u32x4 s_lds[LDS_U];
+    u32x2* const s_xhi = (u32x2*)(s_lds + 8 * PXS);
+    u32x4* const s_w = s_lds + X_U;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wc = wave % WC, wp = wave / WC;
+    const int col = lane & 15, grp = lane >> 4;
+
+    // XCD-aware order (conv_igemm's): the channel tiles of one position tile share an L2.
+    const int P = p.OH * p.OW;
+    const int ptiles = (P + MP - 1) / MP;
+    const int nct = p.ntiles;
+    const int total = p.N * ptiles * nct;
+    const int bid = (int)blockIdx.x, xj = bid & 7, xk = bid >> 3;
+    const int q8 = total >> 3, r8 = total & 7;
+    const int lid = xj < r8 ? xj * (q8 + 1) + xk : r8 * (q8 + 1) + (xj - r8) * q8 + xk;
+    int rest = lid / nct;
+    const int ct = lid - rest * nct;
+    const int pt = rest % ptiles, bi = rest / ptiles;
+    const int pos0 = pt * MP, nb0 = ct * NB;
+    if (nb0 * 16 >= p.cout_g) return;  // padding blocks only (uniform)
+
+    f32x4 acc[CF][PF];
+#pragma unroll
+    for (int cf = 0; cf < CF; ++cf) {
+        const int oc = (nb0 + wc * CF + cf) * 16 + grp * 4;
+        f32x4 b;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[i] = (p.bias && oc + i < p.cout_g) ? p.bias[oc + i] : 0.0f;
+#pragma unroll
+        for (int pf = 0; pf < PF; ++pf) acc[cf][pf] = b;
+    }
+
+    // This thread's position units (quad q of a stage's 32 channels): source, step per stage (0 for
+    // positions past the map, which read zeros) and LDS slot.
+    const float* xg = (const float*)p.x.p + (long long)bi * p.x.bstride + p.x.c_off;
+    const int q = tid & 7;
+    const float* xp[XN];
+    int xstep[XN], xdst[XN];
+#pragma unroll
+    for (int i = 0; i < XN; ++i) {
+        const int pos = (tid + i * NT) >> 3, pg = pos0 + pos;
+        const int oy = pg / p.OW, ox = pg - oy * p.OW;
+        xp[i] = pg < P ? xg + (long long)oy * p.x.row + (long long)ox * p.x.cs + q * 4 : (const float*)g_zero_split;
+        xstep[i] = pg < P ? 32 : 0;
+        xdst[i] = q * PXS + (pos ^ q);
+    }
+    u32x4 rx[XN];
+    auto load_x = [&](int st) __attribute__((always_inline)) {
+        if (st * 32 + 32 <= p.cin_g) {
+#pragma unroll
+            for (int i = 0; i < XN; ++i) {
+                rx[i] = *(const u32x4*)xp[i];
+                xp[i] += xstep[i];
+            }
+        } else {  // the last stage of a cin off 32
+#pragma unroll
+            for (int i = 0; i < XN; ++i)
+                rx[i] = *(st * 32 + q * 4 < p.cin_g ? (const u32x4*)xp[i] : g_zero_split);
+        }
+    };
+    const char* const wg = (const char*)((const u32x4*)((const float*)p.w + bi * p.w_bstride) + (long long)nb0 * SPLIT_BLOCK_U);
+    const long long wchunk = (long long)p.nblk_g * (SPLIT_BLOCK_U * 16);
+    const int nchunks = p.nchunks, nst = (nchunks + 1) / 2;
+    auto issue_w = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (2 * st + k >= nchunks) break;
+            u32x4* dst = s_w + ((st & 1) * 2 + k) * W_U;
+#pragma unroll
+            for (int i = 0; i < WN; ++i) {
+                const int ub = wave * 64 + i * NT;
+                if (ub >= W_U) break;
+                if (ub + lane < W_U) lds_dma16_at(wg + (2 * st + k) * wchunk, (ub + lane) * 16, dst + ub);
+            }
+        }
+    };
+
+    load_x(0);
+    issue_w(0);
+#pragma unroll 1
+    for (int st = 0; st < nst; ++st) {
+        if (st > 0) __syncthreads();  // every wave is done with the last stage's positions
+#pragma unroll
+        for (int i = 0; i < XN; ++i) {
+            const SplitFrag f = split_f32(__builtin_bit_cast(f32x4, rx[i]));
+            s_lds[xdst[i]] = f.lo;
+            s_xhi[xdst[i]] = f.hi;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // this wave's weights of the stage
+        __syncthreads();
+        if (st + 1 < nst) {
+            issue_w(st + 1);
+            load_x(st + 1);
+        }
+        const u32x4* sw = s_w + (st & 1) * 2 * W_U;
+        SplitFrag b[2][PF];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int pf = 0; pf < PF; ++pf) {
+                const int qq = 4 * k + grp, i = qq * PXS + (((wp * PF + pf) * 16 + col) ^ qq);
+                b[k][pf] = SplitFrag{s_lds[i], s_xhi[i]};
+            }
+        const bool two = 2 * st + 1 < nchunks;
+#pragma unroll
+        for (int cf = 0; cf < CF; ++cf) {
+            SplitFrag a[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const u32x4* w = sw + k * W_U + (wc * CF + cf) * SPLIT_BLOCK_U;
+                a[k] = SplitFrag{w[lane], ((const u32x2*)(w + 64))[lane]};
+            }
+            mma_split32<PF>(acc[cf], a[0], a[1], b[0], b[1], two);
+        }
+    }
+
+    // Transposed through LDS: every position's NB * 16 channels leave as one contiguous run.
+    __syncthreads();
+    float* so = reinterpret_cast<float*>(s_lds);
+#pragma unroll
+    for (int cf = 0; cf < CF; ++cf)
+#pragma unroll
+        for (int pf = 0; pf < PF; ++pf)
+            *reinterpret_cast<f32x4*>(so + ((wp * PF + pf) * 16 + col) * OUT_LD + (wc * CF + cf) * 16 + grp * 4) = acc[cf][pf];
+    __syncthreads();
+    const bool full = nb0 * 16 + NB * 16 <= p.cout_g;
+    if (full && epilogue_simple(p)) {
+        constexpr int QP8 = NB * 2;
+#pragma unroll 4
+        for (int u = tid; u < MP * QP8; u += NT) {
+            const int pos = u / QP8, c8 = u - pos * QP8, pg = pos0 + pos;
+            const f32x4 v0 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8);
+            const f32x4 v1 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8 + 4);
+            if (pg < P) {
+                const int oy = pg / p.OW, ox = pg - oy * p.OW;
+                epilogue_store8<float>(p, bi, oy, ox, nb0 * 16 + c8 * 8, v0, v1);
+            }
+        }
+    } else if (full && epilogue_ps2(p)) {
+        constexpr int QP = NB * 4;
+#pragma unroll 2
+        for (int u = tid; u < MP * QP; u += NT) {
+            const int pos = u / QP, r = u - pos * QP, sub = r / NB, cq = r - sub * NB, pg = pos0 + pos;
+            if (pg >= P) continue;
+            const int oy = pg / p.OW, ox = pg - oy * p.OW;
+            const float* v = so + pos * OUT_LD + cq * 16 + sub;
+            epilogue_store_ps2<float>(p, bi, oy, ox, sub, nb0 * 4 + cq * 4, f32x4{v[0], v[4], v[8], v[12]});
+        }
+    } else {
+        constexpr int QP = NB * 4;
+        for (int u = tid; u < MP * QP; u += NT) {
+            const int pos = u / QP, cq = u - pos * QP, pg = pos0 + pos, oc = nb0 * 16 + cq * 4;
+            if (pg >= P || oc >= p.cout_g) continue;
+            const int oy = pg / p.OW, ox = pg - oy * p.OW;
+            epilogue_store<float>(p, bi, oy, ox, oc, min(4, p.cout_g - oc), *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + cq * 4));
+        }
+    }
+}
+
 namespace {
+
+template <int WC, int WP, int CF, int PF>
+hipError_t go_1x1_split(const ConvParams& p0, hipStream_t s) {
+    constexpr int NB = WC * CF, MP = WP * PF * 16;
+    ConvParams p = p0;
+    p.ntiles = p.nblk_g / NB;
+    const long long total = ((long long)p.OH * p.OW + MP - 1) / MP * p.N * p.ntiles;
+    if (p.nblk_g % NB || total <= 0 || total > (1ll << 30)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((conv1x1_ring_split<WC, WP, CF, PF>), dim3((unsigned)total), dim3(WC * WP * 64), 0, s, p);
+    return hipGetLastError();
+}
 
 template <int KH, int KW, int S, int WC, int WP, int CF, int PF, int TS, int NHB, int RW>
 hipError_t go_split(const ConvParams& p0, hipStream_t s) {
     constexpr int TY = WP * PF;
     ConvParams p = p0;
-    if (p.ntiles != p.groups * p.nblk_g / (WC * CF) || p.nblk_g % (WC * CF) || p.N < 1 || p.N > MAXB || p.w_bstride)
+    if (p.ntiles != p.groups * p.nblk_g / (WC * CF) || p.nblk_g % (WC * CF) || p.N < 1 || p.N > MAXB)
         return hipErrorInvalidValue;
     p.gx = (p.OW + 15) / 16;
     p.gy = (p.OH + TY - 1) / TY;
@@ -279,6 +483,9 @@ hipError_t go_split(const ConvParams& p0, hipStream_t s) {
     if (kind == KIND && c.wc == A && c.wp == B && c.cf == C && c.pf == D) return go_split<KH, KW, S, A, B, C, D, TS, NHB, RW>(p, s);
 
 hipError_t launch_conv_split(int kind, TileCfg c, const ConvParams& p, hipStream_t s) {
+    ZJAI_SPLIT(CK_1x1, 1, 1, 1, 1, 4, 4, 2, 1, 1, 2)
+    ZJAI_SPLIT(CK_1x1, 1, 1, 1, 1, 4, 2, 2, 1, 1, 2)
+    ZJAI_SPLIT(CK_1x1, 1, 1, 1, 1, 4, 1, 2, 1, 1, 2)
     ZJAI_SPLIT(CK_3x3, 3, 3, 1, 2, 2, 4, 4, 1, 2, 3)
     ZJAI_SPLIT(CK_3x3, 3, 3, 1, 1, 4, 4, 4, 1, 1, 3)
     ZJAI_SPLIT(CK_3x3, 3, 3, 1, 1, 4, 4, 2, 3, 1, 2)
@@ -293,6 +500,24 @@ hipError_t launch_conv_split(int kind, TileCfg c, const ConvParams& p, hipStream
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 4, 4, 2, 1, 1, 3)
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 8, 2, 1, 4, 1, 2)
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 8, 1, 1, 4, 1, 2)
+    return hipErrorInvalidValue;
+}
+
+bool conv1x1_ring_split_ok(const ConvParams& p) {
+    auto al = [](const View& v) { return !(v.cs % 4) && !(v.c_off % 4) && !(v.row % 4) && !(v.bstride % 4); };
+    return p.groups == 1 && p.N >= 1 && p.N <= MAXB && !p.relu6_in && p.H == p.OH && p.W == p.OW && p.pad_t == 0 &&
+           p.pad_l == 0 && al(p.x) && (p.out_mode != OUT_NHWC || al(p.y)) && (!p.r1.p || al(p.r1)) && (!p.r2.p || al(p.r2));
+}
+
+hipError_t launch_conv1x1_ring_split(TileCfg c, const ConvParams& p, hipStream_t s) {
+    if (!conv1x1_ring_split_ok(p)) return hipErrorInvalidValue;
+#define ZJAI_1X1(A, B, C, D) \
+    if (c.wc == A && c.wp == B && c.cf == C && c.pf == D) return go_1x1_split<A, B, C, D>(p, s);
+    ZJAI_1X1(1, 4, 4, 2)
+    ZJAI_1X1(1, 4, 4, 1)
+    ZJAI_1X1(1, 4, 2, 1)
+    ZJAI_1X1(1, 4, 1, 1)
+#undef ZJAI_1X1
     return hipErrorInvalidValue;
 }
 

@@ -24,7 +24,7 @@
 // and every sum runs in the unfused kernels' order, so the two paths agree bit for bit.
 // The weights of slice s + 1 are fetched into registers while slice s computes.
 
-#include "mfma.h"
+#include "split.h"
 #include "ops.h"
 
 namespace zjai {
@@ -673,6 +673,13 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 __device__ u32x4 g_zero_ffn32[8];  // 128 zero bytes: the source of absent biases
 
+// The thread index as the compiler cannot know it: what a phase of the slice loop derives from it
+// is computed in that phase, instead of being kept in registers (or spilled) across the others.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // s_waitcnt vmcnt(N) (expcnt and lgkmcnt not waited for); gfx9 splits vmcnt over [3:0] and [15:14].
 template <int N>
 __device__ __forceinline__ void ffn_wait_vmcnt() {
@@ -681,15 +688,16 @@ __device__ __forceinline__ void ffn_wait_vmcnt() {
 }
 
 // LayerNorm of this wave's halo positions into B fragments: u[i][c] holds channels
-// 16 c + 4 grp .. + 3 of halo position (2 wave + i) * 16 + col. Statistics as k_layer_norm: one
+// 16 c + 4 grp .. + 3 of halo position (2 wave + i) * 16 + col, split (split.h). Statistics as k_layer_norm: one
 // thread per halo position sums its channels in order in f64 (positions outside the picture
 // read zeros; their values are never used, the 1x1's output is zeroed there). Ends after the
 // statistics barrier; the caller's direct loads issued before it are waited for by the loads here.
 template <int DIM>
 __device__ __forceinline__ void ln_frags_f32(const float* xb, const View& xv, int y0, int x0, int h, int w,
                                              const float* ln_w, const float* ln_b, float* s_stat, int tid,
-                                             int wave, int col, int grp, f32x4 (&u)[2][DIM / 16]) {
+                                             int wave, int col, int grp, SplitFrag (&us)[2][DIM / 16]) {
     constexpr int NCH = DIM / 16;
+    f32x4 u[2][NCH];
     if (tid < FNP) {
         const int iy = y0 - 1 + tid / FH, ix = x0 - 1 + tid % FH;
         double mean = 0.0, var = 0.0;
@@ -743,68 +751,73 @@ __device__ __forceinline__ void ln_frags_f32(const float* xb, const View& xv, in
                 e = e * lw[k];
                 u[i][c][k] = e + lb[k];
             }
+            us[i][c] = split_f32(u[i][c]);
         }
     }
 }
 
-// acc[cb][i] = bias + W (64 rows: four 16-row blocks in LDS as [chunk][block][16][4 units], unit q
-// of row r at q ^ gswz(r)) x u for this wave's two position blocks, the 1x1's f32 instruction
-// sequence.
+// acc[j][i] = bias + W x u of the slice's 16-row blocks cb0 + j for this wave's two position blocks
+// (W in LDS, four split blocks per chunk): the 1x1's sums (mma_split32).
 template <int NCH>
-__device__ __forceinline__ void slice_gemm_f32(const u32x4* s_w, const float* bias64, const f32x4 (&u)[2][NCH],
-                                               int col, int grp, f32x4 (&acc)[4][2]) {
+__device__ __forceinline__ void slice_gemm_f32(const u32x4* s_w, const float* bias64, const SplitFrag (&u)[2][NCH],
+                                               int cb0, int lane, int grp, f32x4 (&acc)[2][2]) {
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-        const f32x4 bi = *(const f32x4*)(bias64 + cb * 16 + 4 * grp);
-        acc[cb][0] = bi;
-        acc[cb][1] = bi;
+    for (int j = 0; j < 2; ++j) {
+        const f32x4 bi = *(const f32x4*)(bias64 + (cb0 + j) * 16 + 4 * grp);
+        acc[j][0] = bi;
+        acc[j][1] = bi;
     }
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        // One chunk's 16 weight registers at a time (32 MFMAs cover the LDS latency); without the
-        // fence the compiler hoists every chunk's reads and spills.
+    for (int c = 0; c < NCH; c += 2) {
+        // Opaque copies: the (p0, p2) operand tuples are put together here, not kept for all of u.
+        SplitFrag b0[2] = {u[0][c], u[1][c]}, b1[2] = {u[0][c + 1], u[1][c + 1]};
+        asm volatile("" : "+v"(b0[0].hi), "+v"(b0[1].hi), "+v"(b1[0].hi), "+v"(b1[1].hi));
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            SplitFrag a[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const u32x4* w = s_w + ((c + k) * 4 + cb0 + j) * SPLIT_BLOCK_U;
+                a[k] = SplitFrag{w[lane], ((const u32x2*)(w + 64))[lane]};
+            }
+            mma_split32<2>(acc[j], a[0], a[1], b0, b1, true);
+        }
+        // Two chunks' weight registers at a time: the compiler otherwise hoists every read.
         __builtin_amdgcn_sched_barrier(0);
-        f32x4 a[4];
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb) a[cb] = __builtin_bit_cast(f32x4, s_w[(c * 4 + cb) * 64 + col * 4 + (grp ^ gswz(col))]);
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    acc[cb][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[cb][k], u[i][c][k], acc[cb][i], 0, 0, 0);
     }
 }
 
 }  // namespace
 
 // Feed-forward, f32: as k_ffn, slices of 32 gate pairs (64 p channels). LDS: W_in slice
-// [chunk][4 blocks][16][4] (32 KB at dim 128), p [256 positions][64] (a and b halves swapped on
+// [chunk][4 split blocks] (48 KB at dim 128), p [256 positions][64] (a and b halves swapped on
 // odd positions, 16-byte units XORed with pos & 7 so that the project_in stores of 8
 // neighbouring positions -- one 8-lane ds_write_b128 pass over 128 bytes of banks -- are
-// conflict-free), g [208 positions][32] (units XORed with 2 ((pos >> 1) & 3): conflict-free
-// fragment reads), W_out slice [2 chunks][dim / 16 blocks][16][4], and per slice b_in, the
-// depthwise taps and biases. The weight rows take gswz.
+// conflict-free), g in split form (planes [8 channel quads][208 positions]), and per slice b_in,
+// the depthwise taps and biases. The gate values are first put down as f32 in the W_in buffer
+// (consumed by then; [196 positions][32], 16-byte units XORed with pos & 7), then split four
+// channels at a time. Each wave reads its own W_out rows straight into registers.
 template <int DIM>
 __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
     constexpr int HID = 4 * DIM, C2 = 2 * HID, NS = HID / 32, NCH = DIM / 16;
     constexpr int CB2 = DIM / 16, WPC = 8 / CB2, NPB = (FPB + WPC - 1) / WPC;
-    constexpr int WIN_U = NCH * 4 * 64, P_U = FNP * 16, G_U = FPB * 16 * 8, WO_U = 2 * CB2 * 64;
+    constexpr int WIN_U = NCH * 4 * SPLIT_BLOCK_U, P_U = FNP * 16, GPX = FPB * 16;
+    static_assert(GPX % 32 == 16, "conflict-free planes");
     constexpr int X_U = 11 * 16;  // b_in [64], depthwise taps [9][64], depthwise bias [64] (f32)
-    constexpr int WIN_W = NCH * 4 / 8, WO_W = 2 * CB2 / 8;  // direct loads per wave and slice
-    static_assert(WIN_W * 8 == NCH * 4 && WO_W * 8 == 2 * CB2, "load shapes");
+    constexpr int WIN_W = WIN_U / FTHREADS;  // direct loads per thread and slice
+    static_assert(WIN_W * FTHREADS == WIN_U, "load shapes");
     static_assert(FOP <= FPB * 16 && 2 * 8 * 16 == FNP, "tile shapes");
     // One LDS object per buffer: the compiler then sees that the direct loads into one buffer
     // cannot alias the reads of another and waits for them only where this code does.
-    __shared__ u32x4 s_win[WIN_U];
+    __shared__ u32x4 s_win[WIN_U > FOP * 8 ? WIN_U : FOP * 8];
     __shared__ float s_p[P_U * 4];
-    __shared__ float s_g[G_U * 4];
-    __shared__ u32x4 s_wo[WO_U];
+    __shared__ u32x4 s_g[8 * GPX * 3 / 2];
     __shared__ u32x4 s_x[2 * X_U];
-    __shared__ float s_stat[2 * FNP];
+    float* const s_stat = s_p;  // the LayerNorm statistics, read before p is written
+    u32x2* const s_ghi = (u32x2*)(s_g + 8 * GPX);
+    float* const s_gf = (float*)s_win;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, grp = lane >> 4;
     const int bid = (int)blockIdx.x;
     const int tx = bid % p.gx, ty = (bid / p.gx) % p.gy, b = bid / (p.gx * p.gy);
@@ -814,27 +827,23 @@ __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
     const u32x4* w_out = (const u32x4*)p.w_out;
 
     // Slice s weights. W_in block (c, cb): 16 rows of p channels 32 s + 16 cb (cb < 2) or
-    // hid + 32 s + 16 (cb - 2), K chunk c: one contiguous KB of the packed weight.
-    auto issue_win = [&](int s) {
+    // hid + 32 s + 16 (cb - 2), K chunk c: one contiguous split block of the packed weight.
+    auto issue_win = [&](int s) __attribute__((always_inline)) {
+        const int t = opaque(tid);
 #pragma unroll
         for (int j = 0; j < WIN_W; ++j) {
-            const int blk = wave + 8 * j, c = blk >> 2, cb = blk & 3;
-            const int gb = cb < 2 ? 2 * s + cb : HID / 16 + 2 * s + (cb - 2);
-            lds_dma16(w_in + ((long long)c * p.nblk_in + gb) * 64 + (lane ^ gswz(lane >> 2)), s_win + blk * 64);
-        }
-    };
-    auto issue_wout = [&](int s) {  // K chunks 2 s, 2 s + 1: 2 CB2 contiguous KB
-#pragma unroll
-        for (int j = 0; j < WO_W; ++j) {
-            const int blk = wave + 8 * j;
-            lds_dma16(w_out + ((long long)2 * s * p.nblk_out + blk) * 64 + (lane ^ gswz(lane >> 2)), s_wo + blk * 64);
+            const int u = t + j * FTHREADS, blk = u / SPLIT_BLOCK_U, c = blk >> 2, cb = blk & 3;
+            const int gb = cb < 2 ? cb : HID / 16 + (cb - 2);
+            lds_dma16_at(w_in + (long long)(2 * s) * SPLIT_BLOCK_U,
+                         (unsigned)((c * p.nblk_in + gb) * SPLIT_BLOCK_U + (u - blk * SPLIT_BLOCK_U)) * 16,
+                         s_win + wave * 64 + j * FTHREADS);
         }
     };
     // Unit u of X (176): run u / 8 of 32 floats; runs 0-1 b_in, 2-19 tap (run - 2) / 2, 20-21 the
     // depthwise bias; even runs the first-half channels 32 s .., odd runs hid + 32 s ...
     auto issue_x = [&](int s, int buf) {
         if (wave < 3) {
-            const int u = wave * 64 + lane;
+            const int u = opaque(tid);
             if (u < X_U) {
                 const int run = u >> 3, half = run & 1, q = u & 7;
                 const int ch = (half ? HID : 0) + 32 * s + 4 * q;
@@ -849,7 +858,7 @@ __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
 
     issue_win(0);
     issue_x(0, 0);
-    f32x4 u[2][NCH];
+    SplitFrag u[2][NCH];
     ln_frags_f32<DIM>(xb, p.x, y0, x0, p.h, p.w, p.ln_w, p.ln_b, s_stat, tid, wave, col, grp, u);
 
     const int cb2 = wave % CB2, pw2 = wave / CB2;
@@ -860,32 +869,42 @@ __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
 #pragma unroll
         for (int i = 0; i < NPB; ++i) acc2[i] = bo;
     }
-    // Depthwise role (tid < 448, waves 0-6): gate pair pg of the slice, column dc, all rows.
-    const int pg = tid & 31, dc = (tid >> 5) % FT;
-    const bool dw_thread = tid < 32 * FT;
+    const bool dw_thread = wave < 7;  // the depthwise's 32 x FT threads
+    static_assert(32 * FT == 7 * 64, "whole waves");
 
     for (int s = 0; s < NS; ++s) {
         ffn_wait_vmcnt<0>();
-        __syncthreads();  // W_in(s), X(s) landed; p, g and the W_out buffer free
-        issue_wout(s);
+        __syncthreads();  // W_in(s), X(s) landed; p and g free
+        // This wave's W_out rows, K chunks 2 s and 2 s + 1.
+        SplitFrag wo[2];
+        const int tw = opaque(tid) & 63;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const u32x4* w = w_out + ((long long)(2 * s + k) * p.nblk_out + cb2) * SPLIT_BLOCK_U;
+            wo[k] = SplitFrag{w[tw], ((const u32x2*)(w + 64))[tw]};
+        }
         if (s + 1 < NS) issue_x(s + 1, (s + 1) & 1);
         const float* sx = reinterpret_cast<const float*>(s_x + (s & 1) * X_U);
 
         // a. p slice = b_in + W_in x u for this wave's positions; zero outside the picture.
         {
-            f32x4 acc1[4][2];
-            slice_gemm_f32<NCH>(s_win, sx, u, col, grp, acc1);
+            const int la = opaque(tid) & 63, col = la & 15, grp = la >> 4;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int pos = (2 * wave + i) * 16 + col;
-                const int iy = y0 - 1 + pos / FH, ix = x0 - 1 + pos % FH;
-                const bool inside = iy >= 0 && iy < p.h && ix >= 0 && ix < p.w;
+            for (int cb0 = 0; cb0 < 4; cb0 += 2) {
+                f32x4 acc1[2][2];
+                slice_gemm_f32<NCH>(s_win, sx, u, cb0, la, grp, acc1);
 #pragma unroll
-                for (int cb = 0; cb < 4; ++cb) {
-                    const int half = (cb >> 1) ^ (col & 1);  // pos & 1 == col & 1
-                    const f32x4 v = inside ? acc1[cb][i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                    const int unit = (half * 8 + (cb & 1) * 4 + grp) ^ (col & 7);  // pos & 7 == col & 7
-                    *(f32x4*)(s_p + pos * 64 + unit * 4) = v;
+                for (int i = 0; i < 2; ++i) {
+                    const int pos = (2 * wave + i) * 16 + col;
+                    const int iy = y0 - 1 + pos / FH, ix = x0 - 1 + pos % FH;
+                    const bool inside = iy >= 0 && iy < p.h && ix >= 0 && ix < p.w;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const int cb = cb0 + j, half = (cb >> 1) ^ (col & 1);  // pos & 1 == col & 1
+                        const f32x4 v = inside ? acc1[j][i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                        const int unit = (half * 8 + (cb & 1) * 4 + grp) ^ (col & 7);  // pos & 7 == col & 7
+                        *(f32x4*)(s_p + pos * 64 + unit * 4) = v;
+                    }
                 }
             }
         }
@@ -893,6 +912,8 @@ __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
 
         // b. depthwise 3x3 + ELU gate (k_depthwise3x3's order: bias, then taps (ky, kx) ascending).
         if (dw_thread) {
+            // Gate pair pg of the slice, column dc, all rows.
+            const int td = opaque(tid), pg = td & 31, dc = td >> 5;
             const float* dww = sx + 64;
             float wa[9], wb[9];
             const float ba = dww[576 + pg], bb = dww[576 + 32 + pg];
@@ -938,7 +959,7 @@ __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
                 const float e = cephes_exp(a) - 1.0f;
                 const float elu = a > 0.0f ? a : e;
                 const int o = oy * FT + dc;
-                s_g[o * 32 + (((pg >> 2) ^ (((o >> 1) & 3) << 1)) << 2) + (pg & 3)] = elu * bq;
+                s_gf[o * 32 + (((pg >> 2) ^ (o & 7)) << 2) + (pg & 3)] = elu * bq;
 #pragma unroll
                 for (int kx = 0; kx < 3; ++kx) {
                     xa[0][kx] = xa[1][kx];
@@ -948,35 +969,63 @@ __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
                 }
             }
         }
-        // W_in(s + 1) flies during phase c. W_out(s), issued before it, has landed once at most
-        // WIN_W loads are pending.
-        if (s + 1 < NS) issue_win(s + 1);
-        if (s + 1 < NS) ffn_wait_vmcnt<WIN_W>();
-        else ffn_wait_vmcnt<0>();
-        __syncthreads();  // g ready; W_out(s) landed
-
-        // c. y += W_out(s) x g: K chunks 2 s, 2 s + 1 (channel 16 cc + 4 grp + k of the slice).
+        __syncthreads();  // the gate values are down
+        const int ts = opaque(tid);
 #pragma unroll
-        for (int cc = 0; cc < 2; ++cc) {
-            const f32x4 a = __builtin_bit_cast(f32x4, s_wo[(cc * CB2 + cb2) * 64 + col * 4 + (grp ^ gswz(col))]);
-            // The g swizzle depends on bits 1-2 of the position, i.e. of col: one base address.
-            const float* gq = s_g + (pw2 * 16 + col) * 32 + (((cc * 4 + grp) ^ (((col >> 1) & 3) << 1)) << 2);
-            // Position blocks in groups of GB (fewer live fragment registers).
-            constexpr int GB = 7;
-#pragma unroll
-            for (int i0 = 0; i0 < NPB; i0 += GB) {
-                __builtin_amdgcn_sched_barrier(0);
-                f32x4 bv[GB];
-#pragma unroll
-                for (int j = 0; j < GB; ++j)
-                    if (i0 + j < NPB && pw2 + WPC * (i0 + j) < FPB) bv[j] = *(const f32x4*)(gq + WPC * (i0 + j) * 512);
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-#pragma unroll
-                    for (int j = 0; j < GB; ++j)
-                        if (i0 + j < NPB && pw2 + WPC * (i0 + j) < FPB)
-                            acc2[i0 + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], bv[j][k], acc2[i0 + j], 0, 0, 0);
+        for (int i = 0; i < (FOP * 8 + FTHREADS - 1) / FTHREADS; ++i) {
+            const int v = ts + i * FTHREADS, o = v >> 3, q = v & 7;
+            if (v < FOP * 8) {
+                const SplitFrag f = split_f32(*(const f32x4*)(s_gf + o * 32 + ((q ^ (o & 7)) << 2)));
+                s_g[q * GPX + (o ^ q)] = f.lo;
+                s_ghi[q * GPX + (o ^ q)] = f.hi;
             }
+        }
+        // W_out(s) is in registers before the next direct loads go out (their count would be
+        // waited for with it).
+#pragma unroll
+        for (int k = 0; k < 2; ++k) asm volatile("" : "+v"(wo[k].lo), "+v"(wo[k].hi));
+        __syncthreads();  // g ready, the W_in buffer free: W_in(s + 1) flies during phase c
+        if (s + 1 < NS) issue_win(s + 1);
+
+        // c. y += W_out(s) x g: K chunks 2 s, 2 s + 1 (channel 16 cc + 4 grp + k of the slice),
+        // position blocks in groups of GB (fewer live fragment registers).
+        constexpr int GB = 2;
+        const int lc = opaque(tid) & 63, col = lc & 15, grp = lc >> 4;
+#pragma unroll
+        for (int i0 = 0; i0 < NPB; i0 += GB) {
+            __builtin_amdgcn_sched_barrier(0);
+            SplitFrag bv[2][GB];
+            f32x4 t[GB];
+#pragma unroll
+            for (int j = 0; j < GB; ++j) {
+                if (i0 + j >= NPB) continue;
+                const int pb = min(pw2 + WPC * (i0 + j), FPB - 1);
+                t[j] = acc2[i0 + j];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const int q = 4 * k + grp, a = q * GPX + ((pb * 16 + col) ^ q);
+                    bv[k][j] = SplitFrag{s_g[a], s_ghi[a]};
+                }
+            }
+            if (i0 + GB <= NPB) {
+                mma_split32<GB>(t, wo[0], wo[1], bv[0], bv[1], true);
+            } else {
+                constexpr int R = NPB % GB == 0 ? 1 : NPB % GB;
+                SplitFrag r0[R], r1[R];
+                f32x4 tr[R];
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    r0[j] = bv[0][j];
+                    r1[j] = bv[1][j];
+                    tr[j] = t[j];
+                }
+                mma_split32<R>(tr, wo[0], wo[1], r0, r1, true);
+#pragma unroll
+                for (int j = 0; j < R; ++j) t[j] = tr[j];
+            }
+#pragma unroll
+            for (int j = 0; j < GB; ++j)
+                if (i0 + j < NPB) acc2[i0 + j] = t[j];
         }
     }
 
@@ -1002,19 +1051,17 @@ __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
 // taps of every slice (17 KB at dim 128) are loaded once, with the first slice's weights.
 template <int DIM>
 __global__ void __launch_bounds__(FTHREADS) k_qkv_f32(const QkvArgs p) {
-    // p rows swizzled (16-byte units XORed with pos & 15) at dim 128 only: at dim 64 the
-    // compiler then renamed MFMA accumulator chains closer than the ISA guard allows.
-    constexpr int PSWZ = DIM == 128 ? 15 : 0;
+    constexpr int PSWZ = 15;  // p rows swizzled: 16-byte units XORed with pos & 15
     constexpr int C3 = 3 * DIM, NS = C3 / 64, NCH = DIM / 16;
-    constexpr int W1_U = NCH * 4 * 64, P_U = FNP * 16, X_U = 11 * 16;
-    constexpr int W1_W = NCH * 4 / 8;
-    static_assert(W1_W * 8 == NCH * 4 && C3 % 64 == 0, "load shapes");
+    constexpr int W1_U = NCH * 4 * SPLIT_BLOCK_U, P_U = FNP * 16, X_U = 11 * 16;
+    constexpr int W1_W = W1_U / FTHREADS;
+    static_assert(W1_W * FTHREADS == W1_U && C3 % 64 == 0, "load shapes");
     __shared__ u32x4 s_w1[W1_U];
     __shared__ float s_p[P_U * 4];
     __shared__ u32x4 s_x[NS * X_U];
     __shared__ float s_stat[2 * FNP];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, grp = lane >> 4;
     const int bid = (int)blockIdx.x;
     const int tx = bid % p.gx, ty = (bid / p.gx) % p.gy, b = bid / (p.gx * p.gy);
@@ -1023,12 +1070,16 @@ __global__ void __launch_bounds__(FTHREADS) k_qkv_f32(const QkvArgs p) {
     const u32x4* w1 = (const u32x4*)p.w1;
 
     // Slice s: conv1 output channels 64 s .. 64 s + 63 (blocks 4 s .. 4 s + 3).
+    unsigned woff[W1_W];
+#pragma unroll
+    for (int j = 0; j < W1_W; ++j) {
+        const int u = tid + j * FTHREADS, blk = u / SPLIT_BLOCK_U, c = blk >> 2, cb = blk & 3;
+        woff[j] = (unsigned)((c * p.nblk1 + cb) * SPLIT_BLOCK_U + (u - blk * SPLIT_BLOCK_U)) * 16;
+    }
     auto issue_w1 = [&](int s) {
 #pragma unroll
-        for (int j = 0; j < W1_W; ++j) {
-            const int blk = wave + 8 * j, c = blk >> 2, cb = blk & 3;
-            lds_dma16(w1 + ((long long)c * p.nblk1 + 4 * s + cb) * 64 + (lane ^ gswz(lane >> 2)), s_w1 + blk * 64);
-        }
+        for (int j = 0; j < W1_W; ++j)
+            lds_dma16_at(w1 + (long long)(4 * s) * SPLIT_BLOCK_U, woff[j], s_w1 + wave * 64 + j * FTHREADS);
     };
     // Unit u of slice s's X (176): run u / 16 of 64 floats; run 0 b1, 1-9 tap run - 1, 10 the
     // depthwise bias. Wave w loads 64-unit pieces w, w + 8, ... of all NS * 176 units.
@@ -1046,7 +1097,7 @@ __global__ void __launch_bounds__(FTHREADS) k_qkv_f32(const QkvArgs p) {
         }
     }
     issue_w1(0);
-    f32x4 u[2][NCH];
+    SplitFrag u[2][NCH];
     ln_frags_f32<DIM>(xb, p.x, y0, x0, p.h, p.w, p.ln_w, p.ln_b, s_stat, tid, wave, col, grp, u);
 
     // Depthwise role (tid < 448, waves 0-6): channel pair pg of the slice, column dc, all rows.
@@ -1059,17 +1110,20 @@ __global__ void __launch_bounds__(FTHREADS) k_qkv_f32(const QkvArgs p) {
         __syncthreads();  // W1(s) landed; p free
         const float* sx = reinterpret_cast<const float*>(s_x + s * X_U);
         {
-            f32x4 acc1[4][2];
-            slice_gemm_f32<NCH>(s_w1, sx, u, col, grp, acc1);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int pos = (2 * wave + i) * 16 + col;
-                const int iy = y0 - 1 + pos / FH, ix = x0 - 1 + pos % FH;
-                const bool inside = iy >= 0 && iy < p.h && ix >= 0 && ix < p.w;
+            for (int cb0 = 0; cb0 < 4; cb0 += 2) {
+                f32x4 acc1[2][2];
+                slice_gemm_f32<NCH>(s_w1, sx, u, cb0, lane, grp, acc1);
 #pragma unroll
-                for (int cb = 0; cb < 4; ++cb)  // the row's 16 units XORed with pos & 15 (bank spread)
-                    *(f32x4*)(s_p + pos * 64 + (((cb * 4 + grp) ^ (pos & PSWZ)) << 2)) =
-                        inside ? acc1[cb][i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int i = 0; i < 2; ++i) {
+                    const int pos = (2 * wave + i) * 16 + col;
+                    const int iy = y0 - 1 + pos / FH, ix = x0 - 1 + pos % FH;
+                    const bool inside = iy >= 0 && iy < p.h && ix >= 0 && ix < p.w;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)  // the row's 16 units XORed with pos & 15 (bank spread)
+                        *(f32x4*)(s_p + pos * 64 + ((((cb0 + j) * 4 + grp) ^ (pos & PSWZ)) << 2)) =
+                            inside ? acc1[j][i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
             }
         }
         __syncthreads();  // p ready; W1(s) consumed

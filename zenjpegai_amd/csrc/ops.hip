@@ -4,6 +4,7 @@
 // reference's contract has one). Every kernel covers N batch items (tiles of one shape).
 
 #include "ops.h"
+#include "split.h"
 
 #include <algorithm>
 
@@ -615,7 +616,16 @@ __global__ void k_attention_fold(const float* proj, const float* attn, int dim, 
     for (int i = 0; i < 32; ++i)
         if (i < c) s += (double)pw[i] * (double)av[i];
     const int ch = col / CK, kk = col - ch * CK;
-    wpk[(long long)b * w_bstride + (((long long)ch * nblk + o / 16) * 16 + o % 16) * CK + kk] = from_f32<T>((float)s);
+    if constexpr (sizeof(T) == 4) {  // the split packing (split.h)
+        uint16_t* blk = (uint16_t*)(wpk + (long long)b * w_bstride) + ((long long)ch * nblk + o / 16) * (SPLIT_BLOCK_U * 8);
+        const int lane = (kk >> 2) * 16 + o % 16, k = kk & 3;
+        const SplitFrag f = split_f32(f32x4{(float)s, 0.0f, 0.0f, 0.0f});
+        blk[lane * 8 + k] = (uint16_t)f.lo[0];
+        blk[lane * 8 + 4 + k] = (uint16_t)f.lo[2];
+        blk[512 + lane * 4 + k] = (uint16_t)f.hi[0];
+    } else {
+        wpk[(long long)b * w_bstride + (((long long)ch * nblk + o / 16) * 16 + o % 16) * CK + kk] = from_f32<T>((float)s);
+    }
 }
 
 // Zero fill with vector stores (instead of hipMemsetAsync, which callers capturing the stream

@@ -25,22 +25,11 @@
 
 namespace zjai {
 
-// acc[r] += a . b[r] for N accumulators sharing one A fragment. f32: the four 16x16x4 steps of
-// each accumulator in k order, issued k-outermost so that dependent MFMAs are N instructions
-// apart (the same per-accumulator sums as Mma16<float>::run).
+// acc[r] += a . b[r] for N accumulators sharing one A fragment (16-bit types).
 template <typename T, int N>
 __device__ __forceinline__ void mma_rows(f32x4 (&acc)[N], u32x4 a, const u32x4 (&b)[N]) {
-    if constexpr (sizeof(T) == 4) {
-        const f32x4 af = __builtin_bit_cast(f32x4, a);
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int r = 0; r < N; ++r)
-                acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[k], __builtin_bit_cast(f32x4, b[r])[k], acc[r], 0, 0, 0);
-    } else {
-#pragma unroll
-        for (int r = 0; r < N; ++r) Mma16<T>::run(acc[r], a, b[r]);
-    }
+    for (int r = 0; r < N; ++r) Mma16<T>::run(acc[r], a, b[r]);
 }
 
 template <typename T, int C, int TR>
@@ -80,7 +69,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) k_resau(const Res
     // (16-byte units; lane (col, grp) holds row col, K group grp).
     const u32x4* w1 = (const u32x4*)p.w1 + (long long)gi * 9 * (F32 ? SPLIT_BLOCK_U : 64);
     const u32x4* w2 = (const u32x4*)p.w2;
-    u32x4 a1[F32 ? 1 : 9], a2[NC2];
+    u32x4 a1[F32 ? 1 : 9], a2[F32 ? 1 : NC2];
     SplitFrag an;  // f32: one tap at a time, the next one's loaded ahead
     auto load_tap = [&](int t) __attribute__((always_inline)) {
         const u32x4* w = w1 + t * SPLIT_BLOCK_U;
@@ -93,7 +82,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) k_resau(const Res
         for (int t = 0; t < 9; ++t) a1[t] = w1[(t * 16 + col) * 4 + grp];
     }
 #pragma unroll
-    for (int c = 0; c < (F32 ? 0 : NC2); ++c) a2[c] = w2[((c * p.nblk2 + gi) * 16 + col) * 4 + grp];
+    for (int c = 0; c < (F32 ? 0 : NC2); ++c) a2[F32 ? 0 : c] = w2[((c * p.nblk2 + gi) * 16 + col) * 4 + grp];
 
     // 1. relu6(x) halo. Every load reads a clamped (in-picture) pixel and off-picture ones take
     // zeros afterwards, so all of a thread's loads are in flight together.
@@ -160,10 +149,20 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) k_resau(const Res
             mma_rows<T, NPW>(acc, a1[t], bv);
         }
     }
+    // f32: t in split form, planes [channel quad][TPX positions] as the halo's.
+    constexpr int TPX = (TR * 16 + 15) / 32 * 32 + 16;
+    static_assert(!F32 || UPP * TPX <= UPP * NPX, "t fits the halo's place");
+    u32x2* const s_thi = (u32x2*)(s_h + (F32 ? UPP * TPX : 0));
     // t (channel gi * 16 + 4 grp + k at position (r0 + r) * 16 + col) rounded to the storage type.
 #pragma unroll
     for (int r = 0; r < NPW; ++r) {
         const int pos = (r0 + r) * 16 + col;
+        if constexpr (F32) {
+            const SplitFrag f = split_f32(acc[r]);
+            s_h[(gi * 4 + grp) * TPX + pos] = f.lo;
+            s_thi[(gi * 4 + grp) * TPX + pos] = f.hi;
+            continue;
+        }
         const int ch = gi * 16 + 4 * grp, unit = ch / VEC;
         T* dst = reinterpret_cast<T*>(s_t + pos * UPP + (unit ^ (pos & (UPP - 1)))) + (ch - unit * VEC);
         typedef T t4 __attribute__((ext_vector_type(4)));
@@ -178,15 +177,34 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) k_resau(const Res
     f32x4 acc2[NPW];
 #pragma unroll
     for (int r = 0; r < NPW; ++r) acc2[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll(F32 ? 1 : NC2)
-    for (int c = 0; c < NC2; ++c) {
-        u32x4 bv[NPW];
+    if constexpr (F32) {
+        // Two chunks at a time (mma_split32); the weights are L2-resident.
+#pragma unroll 1
+        for (int c = 0; c < NC2; c += 2) {
+            SplitFrag a[2], bv[2][NPW];
 #pragma unroll
-        for (int r = 0; r < NPW; ++r) {
-            const int pos = (r0 + r) * 16 + col;
-            bv[r] = s_t[pos * UPP + ((c * 4 + grp) ^ (pos & (UPP - 1)))];
+            for (int k = 0; k < 2; ++k) {
+                const u32x4* w = w2 + ((c + k) * p.nblk2 + gi) * SPLIT_BLOCK_U;
+                a[k] = SplitFrag{w[lane], ((const u32x2*)(w + 64))[lane]};
+#pragma unroll
+                for (int r = 0; r < NPW; ++r) {
+                    const int i = ((c + k) * 4 + grp) * TPX + (r0 + r) * 16 + col;
+                    bv[k][r] = SplitFrag{s_h[i], s_thi[i]};
+                }
+            }
+            mma_split32<NPW>(acc2, a[0], a[1], bv[0], bv[1], true);
         }
-        mma_rows<T, NPW>(acc2, F32 ? w2[((c * p.nblk2 + gi) * 16 + col) * 4 + grp] : a2[F32 ? 0 : c], bv);
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC2; ++c) {
+            u32x4 bv[NPW];
+#pragma unroll
+            for (int r = 0; r < NPW; ++r) {
+                const int pos = (r0 + r) * 16 + col;
+                bv[r] = s_t[pos * UPP + ((c * 4 + grp) ^ (pos & (UPP - 1)))];
+            }
+            mma_rows<T, NPW>(acc2, a2[c], bv);
+        }
     }
     T* yb = (T*)p.y.p + (long long)b * p.y.bstride + p.y.c_off;
     const int ch = gi * 16 + 4 * grp;

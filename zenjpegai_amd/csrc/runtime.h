@@ -201,6 +201,9 @@ using LayerP = std::shared_ptr<Layer>;
 
 // Tile shape the implicit-GEMM kernels use for a layer with cout_g outputs per group.
 TileCfg conv_tile_cfg(int cout_g, int kind, int dtype);
+// Tile shape and profile name of an f32 1x1 launch (conv1x1_ring_split).
+TileCfg ring_split_cfg(int nblk, long long positions, int N);
+std::string ring_split_name(TileCfg c);
 
 LayerP make_conv(Context& ctx, int cin, int cout, int kh, int kw, int stride, int pad_h,
                  int pad_w, int groups, const float* weight, const float* bias,

@@ -348,8 +348,7 @@ void Layer::out_size(int h, int w, int* oh, int* ow) const {
 
 // Tile shape of a layer: narrow groups / outputs take 16- or 32-channel tiles; dense stride-1
 // 3x3 layers take the 8-wave 64-channel x 16-row tile (two waves per SIMD from one workgroup hide
-// each other's LDS and barrier waits: +2-3 % on the config-5 picture in every precision); fp32
-// 1x1 layers with >= 256 outputs the 8-wave 128-channel x 8-row tile (+2 % in fp32).
+// each other's LDS and barrier waits: +2-3 % on the config-5 picture in every precision).
 TileCfg conv_tile_cfg(int cout_g, int kind, int dtype) {
     if (conv_is_split(kind, dtype)) {  // the large-map shapes of conv_f32.hip
         const bool wide = cout_g % 128 == 0;
@@ -359,12 +358,12 @@ TileCfg conv_tile_cfg(int cout_g, int kind, int dtype) {
         if (kind == CK_3x3_S2)
             return cout_g <= 16 ? TileCfg{1, 4, 1, 1} : cout_g <= 32 ? TileCfg{1, 4, 2, 1}
                    : wide ? TileCfg{2, 2, 4, 2} : TileCfg{1, 4, 4, 2};
+        if (kind == CK_1x1) return cout_g <= 16 ? TileCfg{1, 4, 1, 2} : cout_g <= 32 ? TileCfg{1, 4, 2, 2} : TileCfg{1, 4, 4, 2};
         return cout_g <= 16 ? TileCfg{1, 8, 1, 1} : cout_g <= 32 ? TileCfg{1, 8, 2, 1} : TileCfg{1, 4, 4, 2};
     }
     if (cout_g <= 16) return TileCfg{1, 4, 1, 2};
     if (cout_g <= 32) return TileCfg{1, 4, 2, 2};
     if (kind == CK_3x3) return TileCfg{2, 4, 2, 4};
-    if (kind == CK_1x1 && dtype == DT_F32 && cout_g >= 256 && cout_g % 128 == 0) return TileCfg{4, 2, 2, 4};
     return TileCfg{2, 2, 2, 4};
 }
 
@@ -599,7 +598,7 @@ static TileCfg split_tile_cfg(const Layer& L, int N, int OH, int OW) {
         return w < 56 ? TileCfg{1, 8, 1, 1} : w < 96 ? TileCfg{1, 4, 1, 2} : w < 200 ? TileCfg{1, 4, 2, 2}
                : w < 384 ? TileCfg{1, 4, 4, 2} : L.cfg;
     }
-    if (nb <= 2) return L.cfg;
+    if (nb <= 2 || L.kind == CK_1x1) return L.cfg;
     const long long w = cols * rows8 * (tiles * nb / 4);
     if (L.kind == CK_3x3_S2) return w < 48 ? TileCfg{1, 4, 1, 1} : w < 160 ? TileCfg{1, 4, 2, 1} : w < 512 ? TileCfg{1, 4, 4, 1} : L.cfg;
     return w < 96 ? TileCfg{1, 8, 1, 1} : w < 384 ? TileCfg{1, 8, 2, 1} : L.cfg;
@@ -651,6 +650,25 @@ static bool convT_merged_fills(const Layer& L, int N, int OH, int OW) {
     const long long wm = (long long)(((OW + 1) / 2 + 15) / 16) * (((OH + 1) / 2 + 15) / 16) * N *
                          (L.nblk_g / TR_MERGED_NB);
     return wm >= 256;
+}
+
+// Tile of an f32 1x1 launch by its number of 64-channel x 128-position workgroups: narrower tiles
+// keep the CUs busy on small maps (us, one launch): 128 -> 512 at 431^2 (11616) 64 ch x 128
+// positions 255, 64 x 64 273, 32 x 64 337; 64 -> 256 at 108^2 (368) 13.9 / 12.4 / 13.8; 128 -> 128
+// at 108^2 (184) 15.3 / 13.0 / 11.9, 16 x 64 13.9; at 51 x 75 (60) 14.1 / 11.6 / 9.1 / 8.9; 160 ->
+// 160 at 45 x 40 (45) 17.6 / 13.7 / 9.7 / 9.4. 128 channels x 128 positions were slower throughout
+// (304 at 431^2: two workgroups per CU instead of three).
+TileCfg ring_split_cfg(int nblk, long long positions, int N) {
+    const long long w4 = (positions + 127) / 128 * N * nblk;  // in quarters of a workgroup
+    if (nblk % 2 || w4 < 4 * 64) return TileCfg{1, 4, 1, 1};
+    if (nblk % 4 || w4 < 4 * 224) return TileCfg{1, 4, 2, 1};
+    return w4 < 4 * 512 ? TileCfg{1, 4, 4, 1} : TileCfg{1, 4, 4, 2};
+}
+
+std::string ring_split_name(TileCfg c) {
+    char buf[64];
+    snprintf(buf, sizeof buf, "conv1x1_ring_split<%d, %d, %d, %d>", c.wc, c.wp, c.cf, c.pf);
+    return buf;
 }
 
 std::string conv_kernel_name(int kind, int dtype, TileCfg c) {
@@ -829,6 +847,12 @@ static TensorP conv_forward_impl(Context& ctx, const Layer& L, const TensorP& x,
         snprintf(name, sizeof name, "conv3x3_m32<%s, %d, %d>", ty[L.dtype], L.mt32, tw);
         LaunchScope sc(ctx, name, 2.0 * macs, bytes);
         ZJAI_HIP(launch_conv3x3_m32(L.dtype, L.mt32, tw, p, ctx.stream));
+        return y;
+    }
+    if (L.kind == CK_1x1 && L.dtype == DT_F32 && !(ctx.top().flags & ZJAI_CTX_IGEMM_CONV1X1) && conv1x1_ring_split_ok(p)) {
+        const TileCfg c = ring_split_cfg(L.nblk_g, (long long)OH * OW, N);
+        LaunchScope sc(ctx, ring_split_name(c), 2.0 * macs, bytes);
+        ZJAI_HIP(launch_conv1x1_ring_split(c, p, ctx.stream));
         return y;
     }
     if (L.kind == CK_1x1 && !(ctx.top().flags & ZJAI_CTX_IGEMM_CONV1X1) && conv1x1_ring_ok(p, L.dtype)) {

@@ -86,6 +86,64 @@ __device__ __forceinline__ void mma_split_rows(f32x4 (&big)[N], f32x4 (&small)[N
     for (int r = 0; r < N; ++r) small[r] = mfma_bf16(ahi, b[r].lo, small[r]);
 }
 
+// 1x1 layers keep one accumulator: the small products of every two K chunks (32 channels; the last
+// chunk of an odd number by itself) are summed from zero and then added to it, which leaves
+// registers for the fused transformer blocks and rounds the full-size sum 9 times per 32 products.
+//
+// The MFMAs are inline assembly, accumulators in place: with a fresh small sum every 32 channels
+// the compiler renames the chains a few instructions apart. It does not know what the block holds,
+// so the block carries its own wait states: two before (an operand written by vector code just
+// before) and 19 after (results of an 8-pass MFMA read or overwritten by vector code).
+#define ZJAI_MF "v_mfma_f32_16x16x32_bf16 "
+#define ZJAI_WAIT "s_nop 15\n\ts_nop 2"
+__device__ __forceinline__ void mma_split32_2(f32x4& c0, f32x4& c1, const SplitFrag& a0, const SplitFrag& a1,
+                                              const SplitFrag& b00, const SplitFrag& b01, const SplitFrag& b10,
+                                              const SplitFrag& b11) {
+    f32x4 s0, s1;
+    asm("s_nop 1\n\t"
+        ZJAI_MF "%2, %4, %9, 0\n\t" ZJAI_MF "%0, %4, %8, %0\n\t" ZJAI_MF "%2, %5, %8, %2\n\t"
+        ZJAI_MF "%3, %4, %13, 0\n\t" ZJAI_MF "%1, %4, %12, %1\n\t" ZJAI_MF "%3, %5, %12, %3\n\t"
+        ZJAI_MF "%2, %6, %11, %2\n\t" ZJAI_MF "%0, %6, %10, %0\n\t" ZJAI_MF "%2, %7, %10, %2\n\t"
+        ZJAI_MF "%3, %6, %15, %3\n\t" ZJAI_MF "%1, %6, %14, %1\n\t" ZJAI_MF "%3, %7, %14, %3\n\t" ZJAI_WAIT
+        : "+v"(c0), "+v"(c1), "=&v"(s0), "=&v"(s1)
+        : "v"(a0.lo), "v"(split_hi(a0)), "v"(a1.lo), "v"(split_hi(a1)), "v"(b00.lo), "v"(split_hi(b00)), "v"(b01.lo),
+          "v"(split_hi(b01)), "v"(b10.lo), "v"(split_hi(b10)), "v"(b11.lo), "v"(split_hi(b11)));
+    c0 += s0;
+    c1 += s1;
+}
+__device__ __forceinline__ void mma_split32_1(f32x4& c0, const SplitFrag& a0, const SplitFrag& a1, const SplitFrag& b0,
+                                              const SplitFrag& b1) {
+    f32x4 s0;
+    asm("s_nop 1\n\t"
+        ZJAI_MF "%1, %2, %7, 0\n\t" ZJAI_MF "%0, %2, %6, %0\n\t" ZJAI_MF "%1, %3, %6, %1\n\t"
+        ZJAI_MF "%1, %4, %9, %1\n\t" ZJAI_MF "%0, %4, %8, %0\n\t" ZJAI_MF "%1, %5, %8, %1\n\t" ZJAI_WAIT
+        : "+v"(c0), "=&v"(s0)
+        : "v"(a0.lo), "v"(split_hi(a0)), "v"(a1.lo), "v"(split_hi(a1)), "v"(b0.lo), "v"(split_hi(b0)), "v"(b1.lo),
+          "v"(split_hi(b1)));
+    c0 += s0;
+}
+__device__ __forceinline__ void mma_split16_1(f32x4& c0, const SplitFrag& a0, const SplitFrag& b0) {
+    f32x4 s0;
+    asm("s_nop 1\n\t"
+        ZJAI_MF "%1, %2, %5, 0\n\t" ZJAI_MF "%0, %2, %4, %0\n\t" ZJAI_MF "%1, %3, %4, %1\n\t" ZJAI_WAIT
+        : "+v"(c0), "=&v"(s0)
+        : "v"(a0.lo), "v"(split_hi(a0)), "v"(b0.lo), "v"(split_hi(b0)));
+    c0 += s0;
+}
+// N accumulators sharing A; chunk 1 is there only if `two` (uniform).
+template <int N>
+__device__ __forceinline__ void mma_split32(f32x4 (&acc)[N], const SplitFrag& a0, const SplitFrag& a1,
+                                            const SplitFrag (&b0)[N], const SplitFrag (&b1)[N], bool two) {
+    if (two) {
+#pragma unroll
+        for (int r = 0; r + 1 < N; r += 2) mma_split32_2(acc[r], acc[r + 1], a0, a1, b0[r], b1[r], b0[r + 1], b1[r + 1]);
+        if (N % 2) mma_split32_1(acc[N - 1], a0, a1, b0[N - 1], b1[N - 1]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < N; ++r) mma_split16_1(acc[r], a0, b0[r]);
+    }
+}
+
 // The sum of a finished pair of accumulators. An infinite full-size sum stays infinite: its small
 // products may have overflowed to either sign.
 __device__ __forceinline__ f32x4 split_sum(f32x4 big, f32x4 small) {
