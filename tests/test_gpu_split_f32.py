@@ -27,6 +27,16 @@ def eng():
 
 
 def _layer(eng, kind, cin, cout, groups, seed):
+    if kind in ("t3", "t4"):  # stride 2, padding 1
+        k = int(kind[1])
+        w = synth.normal(seed, f"split/w{kind}{cin}{cout}", (cin, cout, k, k), 1.0)
+        b = synth.normal(seed, f"split/b{cout}", (cout,), 1.0)
+
+        def ref_t(x, w, b):
+            t = [torch.from_numpy(a).double() for a in (x[None], w, b)]
+            return F.conv_transpose2d(*t, 2, 1, 4 - k)[0].numpy()
+
+        return w, b, lambda w, b: nn.ConvTransposeLayer(nn.ConvTranspose2d(cin, cout, k, 2, 1, 4 - k, w, b), eng), ref_t
     k, stride = {"1x1": (1, 1), "3x3": (3, 1), "s2": (3, 2), "2x2": (2, 1)}[kind]
     w = synth.normal(seed, f"split/w{kind}{cin}{cout}", (cout, cin // groups, k, k), 1.0)
     b = synth.normal(seed, f"split/b{cout}", (cout,), 1.0)
@@ -50,7 +60,9 @@ CASES = [("3x3", 4, 4, 1, 1, 1), ("3x3", 20, 24, 1, 9, 17), ("3x3", 160, 160, 1,
          ("s2", 16, 192, 1, 440, 431), ("2x2", 160, 256, 1, 4, 6), ("2x2", 20, 12, 1, 17, 15), ("2x2", 64, 128, 1, 128, 127),
          ("2x2", 16, 192, 1, 150, 161), ("1x1", 4, 4, 1, 1, 1), ("1x1", 20, 24, 1, 9, 7), ("1x1", 48, 16, 1, 33, 64),
          ("1x1", 160, 160, 1, 8, 15), ("1x1", 128, 64, 1, 128, 127), ("1x1", 96, 128, 1, 150, 130),
-         ("1x1", 32, 256, 1, 171, 190)]
+         ("1x1", 32, 256, 1, 171, 190), ("t3", 20, 12, 1, 1, 1), ("t3", 36, 64, 1, 17, 15), ("t3", 32, 96, 1, 90, 97),
+         ("t3", 16, 128, 1, 130, 33), ("t4", 20, 24, 1, 3, 5), ("t4", 48, 64, 1, 31, 34), ("t4", 16, 160, 1, 70, 65),
+         ("t4", 16, 128, 1, 135, 100)]
 
 
 @pytest.mark.parametrize("kind,cin,cout,groups,h,w", CASES)
@@ -60,22 +72,24 @@ def test_error_against_64_bits(eng, kind, cin, cout, groups, h, w):
     y = make(wt, b).forward(eng, nn.BTensor.from_planar(eng, x)).to_planar()
     want, size = ref(x, wt, b), ref(np.abs(x), np.abs(wt), np.abs(b))
     assert y.shape == want.shape
-    kk = wt[0].size
+    kk = cin * 4 if kind[0] == "t" else wt[0].size  # at most 2 x 2 taps reach an output
     bound = (kk / 4 * (1 + 2.0 ** -7) + 4 + (kk / 32 + 1 if kind == "1x1" else 0)) * 2.0 ** -23 * size
     assert np.all(np.abs(y - want) <= bound), float(np.max(np.abs(y - want) / bound))
 
 
-@pytest.mark.parametrize("kind", ["1x1", "3x3", "s2", "2x2"])
+@pytest.mark.parametrize("kind", ["1x1", "3x3", "s2", "2x2", "t3", "t4"])
 def test_values_that_are_not_finite(eng, kind):
     """Infinities and NaN in the input or the weights reach the outputs that f32 arithmetic sends
     them to, and only those."""
     wt, b, make, ref = _layer(eng, kind, 32, 16, 1, 33)
+    if kind[0] == "t":
+        wt = np.ascontiguousarray(wt.transpose(1, 0, 2, 3))  # outputs first, as the others, for the edits below
     wt[3, 5] = 0.0  # 0 * inf is NaN
     x = synth.normal(34, "split/nf", (32, 24, 40), 1.0)
     for ch, r, c, v in ((0, 2, 3, np.inf), (5, 7, 20, -np.inf), (9, 12, 33, np.nan), (31, 23, 39, np.inf), (5, 18, 8, np.inf), (6, 18, 9, -np.inf)):
         x[ch, r, c] = v
     for w in (wt, np.where(np.arange(16)[:, None, None, None] == 7, np.float32(np.inf), wt)):
-        w = np.ascontiguousarray(w)
+        w = np.ascontiguousarray(w.transpose(1, 0, 2, 3) if kind[0] == "t" else w)
         y = make(w, b).forward(eng, nn.BTensor.from_planar(eng, x)).to_planar()
         want = ref(x, w, b)
         np.testing.assert_array_equal(np.isnan(y), np.isnan(want))

@@ -1,14 +1,14 @@
-// Implicit-GEMM convolution on CDNA4 matrix cores (gfx950).
+// Implicit-GEMM convolution on CDNA4 matrix cores (gfx950), 16-bit storage types (f32:
+// conv_f32.hip), and the narrow transposed convolutions of every type.
 //
 // One workgroup computes TY = WP*PF output rows x 16 output columns x NB = WC*CF blocks of 16
 // output channels. GEMM roles: M = output channels (the weights are the A operand), N = output
 // positions (the input halo is the B operand), K = input channels x taps.
 //
-// Per input-channel chunk (64 bytes of channels per pixel: 16 f32 or 32 f16/bf16) the workgroup
+// Per input-channel chunk (64 bytes of channels per pixel: 32 f16/bf16) the workgroup
 // stages the input halo [HY][HX][64 B] and the packed weights [NB][taps][16][64 B] in LDS, then
-// every wave runs, per tap, one 16-byte LDS read per operand fragment and CF x PF MFMAs:
-//   f32:      4 x v_mfma_f32_16x16x4_f32 (lane group g holds channels 4g..4g+3)
-//   f16/bf16: 1 x v_mfma_f32_16x16x32_{f16,bf16} (lane group g holds channels 8g..8g+7)
+// every wave runs, per tap, one 16-byte LDS read per operand fragment and CF x PF
+// v_mfma_f32_16x16x32_{f16,bf16} (lane group g holds channels 8g..8g+7).
 // A and B fragments use the same lane-group -> channel map, so each MFMA sums matching channels.
 // Accumulators start at the bias; the epilogue applies activation, residual op, pixel shuffle,
 // denormalisation and quantisation, and stores NHWC activations or planar picture samples.
@@ -25,7 +25,7 @@
 
 namespace zjai {
 
-// The 16x16 fragment of mfma.h (Mma16): 4 x 16x16x4 f32 steps or one 16x16x32 16-bit step.
+// The 16x16 fragment of mfma.h (Mma16).
 template <typename T> using Mma = Mma16<T>;
 
 // Staged operands keep 4 16-byte units (one K group each) per row: a halo slot or a weight row,
@@ -293,252 +293,16 @@ conv_igemm(const ConvParams p) {
     }
 }
 
-// ---------------------------------------------------------------------------------------------
-// fp32 pipelined variant of conv_igemm (dense tile shapes): the input halo and the weight blocks
-// of a K stage go global -> LDS with gfx950's direct LDS loads (global_load_lds_dwordx4: lane
-// i's 16 bytes land at the wave's LDS base + 16 i, no VGPR staging), double-buffered, so one
-// barrier per stage separates the loads of stage k + 1 from the MFMAs of stage k. Padding units
-// load from a zeroed device buffer. Numerics are conv_igemm's: bias first, then per K chunk and
-// tap the four k = 0..3 MFMAs of each accumulator in order -- issued k-outermost over the
-// CF x PF accumulators, so that dependent MFMAs are CF x PF instructions apart.
-// ---------------------------------------------------------------------------------------------
+// 64 zero bytes: the source of padding units of direct LDS loads.
 __device__ u32x4 g_zero_units[4];
-
-template <int KH, int KW, int S, bool TR, int WC, int WP, int CF, int PF, int SG>
-__global__ void __launch_bounds__(WC * WP * 64)
-conv_dma_f32(const ConvParams p) {
-    using T = float;
-    constexpr int NT = WC * WP * 64;
-    constexpr int TY = WP * PF;
-    constexpr int HY = (TY - 1) * S + KH;
-    constexpr int HX = 15 * S + KW;
-    constexpr int NTAP = TR ? 4 : KH * KW;
-    constexpr int NB = WC * CF;
-    constexpr int VEC = 4;
-    constexpr int CK = 16;
-    constexpr int HALO_U = HY * HX * 4;
-    constexpr int W_U = NB * NTAP * 64;
-    constexpr int CH_U = HALO_U + W_U;  // one K chunk: halo units, then weight units
-    constexpr int STG_U = SG * CH_U;
-    constexpr int OUT_LD = NB * 16 + 4;
-    constexpr int OUT_U = (TY * 16 * OUT_LD + 3) / 4;
-    // Stride-2 stages (a 17 x 33 halo and 4 x 9 weight blocks, 73 KB) are single-buffered: two
-    // workgroups per CU then overlap each other's loads, where one double-buffered workgroup left
-    // one wave per SIMD.
-    constexpr int NBUF = S == 2 ? 1 : 2;
-    constexpr int LDS_U = (NBUF * STG_U) > OUT_U ? (NBUF * STG_U) : OUT_U;
-    constexpr int HN = (HALO_U + NT - 1) / NT, WN = (W_U + NT - 1) / NT;
-    __shared__ u32x4 s_lds[LDS_U];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wc = wave % WC, wp = wave / WC;
-    const int col = lane & 15, grp = lane >> 4;
-
-    // Workgroup -> tile: the XCD-aware order of conv_igemm.
-    const int nz = p.ntiles * (TR ? 4 : 1);
-    const int total = p.gx * p.gy * p.N * nz;
-    const int bid = (int)blockIdx.x, xj = bid & 7, xk = bid >> 3;
-    const int q8 = total >> 3, r8 = total & 7;
-    const int lid = xj < r8 ? xj * (q8 + 1) + xk : r8 * (q8 + 1) + (xj - r8) * q8 + xk;
-    int rest = lid / nz;
-    const int zl = lid - rest * nz;
-    const int tx = rest % p.gx;
-    rest /= p.gx;
-    const int ty = rest % p.gy, bi = rest / p.gy;
-    const int phase = TR ? (zl & 3) : 0;
-    const int nt = TR ? (zl >> 2) : zl;
-    const int gb = nt * NB;
-    const int g = gb / p.nblk_g, nb0 = gb - g * p.nblk_g;
-    const int ox0 = tx * 16, oy0 = ty * TY;
-
-    int ntap = NTAP;
-    int tdy[NTAP], tdx[NTAP];
-#pragma unroll
-    for (int t = 0; t < NTAP; ++t) {
-        if (TR) {
-            tdy[t] = p.tap_dy[phase][t];
-            tdx[t] = p.tap_dx[phase][t];
-        } else {
-            tdy[t] = t / KW;
-            tdx[t] = t % KW;
-        }
-    }
-    if (TR) ntap = p.ntaps[phase];
-
-    f32x4 acc[CF][PF];
-#pragma unroll
-    for (int cf = 0; cf < CF; ++cf) {
-        const int ocl = (nb0 + wc * CF + cf) * 16 + grp * 4;
-        f32x4 b;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            b[i] = (p.bias && ocl + i < p.cout_g) ? p.bias[g * p.cout_g + ocl + i] : 0.0f;
-#pragma unroll
-        for (int pf = 0; pf < PF; ++pf) acc[cf][pf] = b;
-    }
-
-    const int iy0 = TR ? oy0 - 1 : oy0 * S - p.pad_t;
-    const int ix0 = TR ? ox0 - 1 : ox0 * S - p.pad_l;
-    const T* xg = (const T*)p.x.p + (long long)bi * p.x.bstride;
-    const T* wg = (const T*)p.w + phase * p.phase_stride + (long long)bi * p.w_bstride;
-    const long long xbase = (long long)p.x.c_off + (long long)g * p.cin_g;
-
-    // Halo element offset of each of this thread's units (u = tid + i * NT), -1 in the padding,
-    // and the first channel of the quad it holds. Stride 2: unit q of halo pixel s holds channel
-    // quad q ^ qswz(s); a fragment then reads every other pixel with two lanes per bank quad in
-    // each ds_read_b128 pass instead of four. Stride 1 keeps the plain layout.
-    long long hoff[HN];
-    int hqv[HN];
-#pragma unroll
-    for (int i = 0; i < HN; ++i) {
-        const int u = tid + i * NT, pix = u >> 2, q = u & 3;
-        const int hy = pix / HX, hx = pix - hy * HX;
-        const int iy = iy0 + hy, ix = ix0 + hx;
-        hqv[i] = (S == 2 ? (q ^ qswz(pix)) : q) * VEC;
-        hoff[i] = (u < HALO_U && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W)
-                      ? (long long)iy * p.x.row + (long long)ix * p.x.cs + xbase + hqv[i]
-                      : -1;
-    }
-
-    // Direct LDS loads of stage st into buffer buf. Each wave covers whole 64-unit rows of the
-    // chunk's layout; its M0 base is the row start, lanes past the end are masked off.
-    auto issue = [&](int st, int buf) {
-#pragma unroll
-        for (int s = 0; s < SG; ++s) {
-            const int chunk = st * SG + s;
-            if (chunk >= p.nchunks) break;
-            const int cl0 = chunk * CK;
-            u32x4* dst = s_lds + buf * STG_U + s * CH_U;
-#pragma unroll
-            for (int i = 0; i < HN; ++i) {
-                const int ub = wave * 64 + i * NT;
-                if (ub >= HALO_U) break;
-                if (ub + lane < HALO_U) {
-                    const void* src = (hoff[i] >= 0 && cl0 + hqv[i] < p.cin_g) ? (const void*)(xg + hoff[i] + cl0)
-                                                                              : (const void*)g_zero_units;
-                    lds_dma16(src, dst + ub);
-                }
-            }
-            const u32x4* wsrc = (const u32x4*)(wg + ((long long)(g * p.nchunks + chunk) * p.nblk_g + nb0) *
-                                                        (long long)(NTAP * 16 * CK));
-#pragma unroll
-            for (int i = 0; i < WN; ++i) {
-                const int ub = wave * 64 + i * NT;
-                if (ub >= W_U) break;
-                if (ub + lane < W_U)
-                    lds_dma16(wsrc + ub + lane, dst + HALO_U + ub);
-            }
-        }
-    };
-
-    const int nst = (p.nchunks + SG - 1) / SG;
-    issue(0, 0);
-    for (int st = 0; st < nst; ++st) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads of stage st are in LDS
-        __syncthreads();                     // ... and every other wave's
-        if (NBUF == 2 && st + 1 < nst) issue(st + 1, (st + 1) & 1);
-        const u32x4* sb = s_lds + (NBUF == 2 ? (st & 1) : 0) * STG_U;
-        auto stage = [&](auto relu6) {
-#pragma unroll
-            for (int s = 0; s < SG; ++s) {
-                if (st * SG + s >= p.nchunks) break;
-                const u32x4* s_halo = sb + s * CH_U;
-                const u32x4* s_w = s_halo + HALO_U;
-                for (int t = 0; t < ntap; ++t) {
-                    const int ky = tdy[t], kx = tdx[t];
-                    u32x4 a[CF], b[PF];
-#pragma unroll
-                    for (int cf = 0; cf < CF; ++cf) a[cf] = s_w[((wc * CF + cf) * NTAP + t) * 64 + col * 4 + grp];
-#pragma unroll
-                    for (int pf = 0; pf < PF; ++pf) {
-                        const int hy = (wp * PF + pf) * S + ky, hx = col * S + kx, hs = hy * HX + hx;
-                        b[pf] = s_halo[hs * 4 + (S == 2 ? (grp ^ qswz(hs)) : grp)];
-                        if constexpr (decltype(relu6)::value) b[pf] = relu6_vec<T>(b[pf]);
-                    }
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-#pragma unroll
-                        for (int cf = 0; cf < CF; ++cf)
-#pragma unroll
-                            for (int pf = 0; pf < PF; ++pf)
-                                acc[cf][pf] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                    __builtin_bit_cast(f32x4, a[cf])[k], __builtin_bit_cast(f32x4, b[pf])[k],
-                                    acc[cf][pf], 0, 0, 0);
-                }
-            }
-        };
-        if (p.relu6_in) stage(std::true_type{});
-        else stage(std::false_type{});
-        if (NBUF == 1 && st + 1 < nst) {
-            __syncthreads();  // every wave is done with the buffer
-            issue(st + 1, 0);
-        }
-    }
-
-    if (p.out_mode == OUT_NHWC && p.ps == 1) {
-        __syncthreads();
-        float* so = reinterpret_cast<float*>(s_lds);
-#pragma unroll
-        for (int cf = 0; cf < CF; ++cf)
-#pragma unroll
-            for (int pf = 0; pf < PF; ++pf) {
-                float* d = so + ((wp * PF + pf) * 16 + col) * OUT_LD + (wc * CF + cf) * 16 + grp * 4;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) d[i] = acc[cf][pf][i];
-            }
-        __syncthreads();
-        if (nb0 * 16 + NB * 16 <= p.cout_g) {
-            // 8 channels per thread and step (all of the tile's channels are real).
-            constexpr int QP8 = NB * 2;
-#pragma unroll 4
-            for (int u = tid; u < TY * 16 * QP8; u += NT) {
-                const int pos = u / QP8, c8 = u - pos * QP8;
-                const int r = pos >> 4, cx = pos & 15;
-                const int oy = TR ? 2 * (oy0 + r) + (phase >> 1) : oy0 + r;
-                const int ox = TR ? 2 * (ox0 + cx) + (phase & 1) : ox0 + cx;
-                const f32x4 v0 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8);
-                const f32x4 v1 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8 + 4);
-                if (oy < p.OH && ox < p.OW) epilogue_store8<T>(p, bi, oy, ox, g * p.cout_g + nb0 * 16 + c8 * 8, v0, v1);
-            }
-            return;
-        }
-        constexpr int QP = NB * 4;
-        for (int u = tid; u < TY * 16 * QP; u += NT) {
-            const int pos = u / QP, cq = u - pos * QP;
-            const int r = pos >> 4, cx = pos & 15;
-            const int oy = TR ? 2 * (oy0 + r) + (phase >> 1) : oy0 + r;
-            const int ox = TR ? 2 * (ox0 + cx) + (phase & 1) : ox0 + cx;
-            const int ocl = nb0 * 16 + cq * 4;
-            if (oy >= p.OH || ox >= p.OW || ocl >= p.cout_g) continue;
-            const f32x4 v = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + cq * 4);
-            epilogue_store<T>(p, bi, oy, ox, g * p.cout_g + ocl, min(4, p.cout_g - ocl), v);
-        }
-        return;
-    }
-
-#pragma unroll
-    for (int cf = 0; cf < CF; ++cf) {
-        const int ocl = (nb0 + wc * CF + cf) * 16 + grp * 4;
-        if (ocl >= p.cout_g) continue;
-        const int nvalid = min(4, p.cout_g - ocl);
-#pragma unroll
-        for (int pf = 0; pf < PF; ++pf) {
-            const int r = wp * PF + pf;
-            const int oy = TR ? 2 * (oy0 + r) + (phase >> 1) : oy0 + r;
-            const int ox = TR ? 2 * (ox0 + col) + (phase & 1) : ox0 + col;
-            if (oy >= p.OH || ox >= p.OW) continue;
-            epilogue_store<T>(p, bi, oy, ox, g * p.cout_g + ocl, nvalid, acc[cf][pf]);
-        }
-    }
-}
 
 // ---------------------------------------------------------------------------------------------
 // Stride-2 transposed conv (3x3 kernel) with the four output phases of a tile in one
 // workgroup. The phase-per-workgroup form stages a halo and a weight block per K chunk for
 // 1, 2, 2 or 4 taps; here the 9 taps of all phases share one staged halo and one 9-tap weight
 // block, so a K chunk carries as much matrix work as a 3x3 conv. Each wave accumulates its
-// CF x PF tile for all four phases (acc[4][CF][PF]); the stage pipeline is conv_dma_f32's
-// (direct global -> LDS loads, double-buffered, one barrier per stage), for every storage type.
+// CF x PF tile for all four phases (acc[4][CF][PF]); the stages are direct
+// global -> LDS loads, double-buffered, one barrier per stage (16-bit types; f32: conv_f32.hip).
 // Per output the products are summed exactly as in the phase-per-workgroup kernel: bias, then
 // per K chunk the phase's taps in table order, k ascending within a tap. The phases' tap counts
 // are template parameters (1, 2, 2, 4 for padding 1; 4, 2, 2, 1 for padding 0 or 2), so the tap
@@ -547,10 +311,8 @@ conv_dma_f32(const ConvParams p) {
 template <typename T, int N0, int N1, int N2, int N3>
 __global__ void __launch_bounds__(512)
 conv_tr_merged(const ConvParams p) {
-    // 16-bit weights come packed with unit q of each 16-row block's row r at q ^ qswz(r) (the
-    // launcher's merged packing), so the fragment reads are conflict-free; f32 keeps the plain
-    // layout (under the swizzled addressing the compiler renamed this kernel's f32 MFMA chains).
-    auto wswz = [](int r) __attribute__((always_inline)) { return sizeof(T) == 2 ? qswz(r) : 0; };
+    // The weights come packed with unit q of each 16-row block's row r at q ^ qswz(r) (the
+    // launcher's merged packing), so the fragment reads are conflict-free.
     constexpr int WC = 2, WP = 4, CF = 2, PF = 4;
     constexpr int NT = WC * WP * 64;
     constexpr int TY = WP * PF;
@@ -670,27 +432,15 @@ conv_tr_merged(const ConvParams p) {
                 const int dy = tdy[ph][t], dx = tdx[ph][t];
                 u32x4 a[CF], b[PF];
 #pragma unroll
-                for (int cf = 0; cf < CF; ++cf) a[cf] = s_w[((wc * CF + cf) * NTALL + e) * 64 + col * 4 + (grp ^ wswz(col))];
+                for (int cf = 0; cf < CF; ++cf) a[cf] = s_w[((wc * CF + cf) * NTALL + e) * 64 + col * 4 + (grp ^ qswz(col))];
 #pragma unroll
                 for (int pf = 0; pf < PF; ++pf) {
                     b[pf] = s_halo[((wp * PF + pf + dy) * HX + col + dx) * 4 + grp];
                 }
-                if constexpr (sizeof(T) == 4) {
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
+                for (int cf = 0; cf < CF; ++cf)
 #pragma unroll
-                        for (int cf = 0; cf < CF; ++cf)
-#pragma unroll
-                            for (int pf = 0; pf < PF; ++pf)
-                                acc[ph][cf][pf] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                    __builtin_bit_cast(f32x4, a[cf])[k], __builtin_bit_cast(f32x4, b[pf])[k],
-                                    acc[ph][cf][pf], 0, 0, 0);
-                } else {
-#pragma unroll
-                    for (int cf = 0; cf < CF; ++cf)
-#pragma unroll
-                        for (int pf = 0; pf < PF; ++pf) Mma<T>::run(acc[ph][cf][pf], a[cf], b[pf]);
-                }
+                    for (int pf = 0; pf < PF; ++pf) Mma<T>::run(acc[ph][cf][pf], a[cf], b[pf]);
             }
         };
         phase_taps(std::integral_constant<int, 0>{});
@@ -771,7 +521,6 @@ hipError_t launch_conv_tr_merged(int dtype, const ConvParams& p0, hipStream_t s)
         else hipLaunchKernelGGL((conv_tr_merged<TY, 4, 2, 2, 1>), grid, block, 0, s, p);            \
     } while (0)
     switch (dtype) {
-        case DT_F32: ZJAI_TRM(float); break;
         case DT_F16: ZJAI_TRM(_Float16); break;
         case DT_BF16: ZJAI_TRM(__bf16); break;
         default: return hipErrorInvalidValue;
@@ -1294,14 +1043,6 @@ hipError_t launch_convT_narrow(int dtype, int coutp, const ConvParams& p, const 
 // ---------------------------------------------------------------------------------------------
 // Launch dispatch.
 // ---------------------------------------------------------------------------------------------
-// The fp32 dense tile shapes run the direct-LDS-load kernel (1x1 layers stage two K chunks per
-// barrier); the 16-bit ones and the narrow shapes run conv_igemm.
-template <int WC, int WP, int CF, int PF>
-constexpr bool use_dma_f32() {
-    return (WC == 2 && WP == 2 && CF == 2 && PF == 4) || (WC == 2 && WP == 4 && CF == 2 && PF == 4) ||
-           (WC == 4 && WP == 2 && CF == 2 && PF == 4);
-}
-
 template <typename T, int KH, int KW, int S, bool TR, int WC, int WP, int CF, int PF>
 static hipError_t go(const ConvParams& p0, hipStream_t s) {
     constexpr int SG = (KH * KW == 1 && !TR) ? 4 : 1;
@@ -1314,22 +1055,13 @@ static hipError_t go(const ConvParams& p0, hipStream_t s) {
     p.gy = (gh + TY - 1) / TY;
     const long long total = (long long)p.gx * p.gy * p.N * p.ntiles * (TR ? 4 : 1);
     if (total <= 0 || total > (1ll << 30)) return hipErrorInvalidValue;
-    if constexpr (sizeof(T) == 4 && use_dma_f32<WC, WP, CF, PF>()) {
-        constexpr int SGD = (KH * KW == 1 && !TR) ? 2 : 1;
-        hipLaunchKernelGGL((conv_dma_f32<KH, KW, S, TR, WC, WP, CF, PF, SGD>), dim3((unsigned)total),
-                           dim3(WC * WP * 64), 0, s, p);
-    } else {
-        hipLaunchKernelGGL((conv_igemm<T, KH, KW, S, TR, WC, WP, CF, PF, SG>), dim3((unsigned)total),
-                           dim3(WC * WP * 64), 0, s, p);
-    }
+    hipLaunchKernelGGL((conv_igemm<T, KH, KW, S, TR, WC, WP, CF, PF, SG>), dim3((unsigned)total),
+                       dim3(WC * WP * 64), 0, s, p);
     return hipGetLastError();
 }
 
 template <typename T, int WC, int WP, int CF, int PF>
 static hipError_t go_kind(int kind, const ConvParams& p, hipStream_t s) {
-    if constexpr (sizeof(T) == 4)  // every other kind is launch_conv_split's
-        return kind == CK_T3 ? go<T, 3, 3, 1, true, WC, WP, CF, PF>(p, s) : hipErrorInvalidValue;
-    else
     switch (kind) {
         case CK_1x1: return go<T, 1, 1, 1, false, WC, WP, CF, PF>(p, s);
         case CK_2x2: return go<T, 2, 2, 1, false, WC, WP, CF, PF>(p, s);
@@ -1351,9 +1083,9 @@ static hipError_t go_kind(int kind, const ConvParams& p, hipStream_t s) {
 template <typename T>
 static hipError_t go_cfg(int kind, TileCfg c, const ConvParams& p, hipStream_t s) {
     if (c.wc == 2 && c.wp == 4 && c.cf == 2 && c.pf == 4)
-        return sizeof(T) == 2 && kind == CK_3x3 ? go<std::conditional_t<sizeof(T) == 2, T, __bf16>, 3, 3, 1, false, 2, 4, 2, 4>(p, s) : hipErrorInvalidValue;
+        return kind == CK_3x3 ? go<T, 3, 3, 1, false, 2, 4, 2, 4>(p, s) : hipErrorInvalidValue;
     if (c.wc == 4 && c.wp == 2 && c.cf == 2 && c.pf == 4)
-        return sizeof(T) == 2 && kind == CK_3x3_S2 ? go<std::conditional_t<sizeof(T) == 2, T, __bf16>, 3, 3, 2, false, 4, 2, 2, 4>(p, s) : hipErrorInvalidValue;
+        return kind == CK_3x3_S2 ? go<T, 3, 3, 2, false, 4, 2, 2, 4>(p, s) : hipErrorInvalidValue;
 #define ZJAI_GO(a, b, cc, d) \
     if (c.wc == a && c.wp == b && c.cf == cc && c.pf == d) return go_kind<T, a, b, cc, d>(kind, p, s);
     ZJAI_CFGS(ZJAI_GO)
@@ -1363,7 +1095,6 @@ static hipError_t go_cfg(int kind, TileCfg c, const ConvParams& p, hipStream_t s
 
 hipError_t launch_conv(int kind, int dtype, TileCfg cfg, const ConvParams& p, hipStream_t s) {
     switch (dtype) {
-        case DT_F32: return go_cfg<float>(kind, cfg, p, s);
         case DT_F16: return go_cfg<_Float16>(kind, cfg, p, s);
         case DT_BF16: return go_cfg<__bf16>(kind, cfg, p, s);
     }

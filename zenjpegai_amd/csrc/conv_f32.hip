@@ -19,17 +19,20 @@
 #include "epilogue.h"
 #include "split.h"
 
+#include <type_traits>
+
 namespace zjai {
 
 __device__ u32x4 g_zero_split[1];  // 16 zero bytes: the source of padding units
 
-template <int KH, int KW, int S, int WC, int WP, int CF, int PF, int TS, int NHB, int RW>
+template <int KH, int KW, int S, bool TR, int WC, int WP, int CF, int PF, int TS, int NHB, int RW>
 __global__ void __launch_bounds__(WC * WP * 64, 2)
 conv_igemm_split(const ConvParams p) {
     constexpr int NT = WC * WP * 64;
     constexpr int TY = WP * PF;
     constexpr int HY = (TY - 1) * S + KH, HX = 15 * S + KW, HP = HY * HX;
-    constexpr int NTAP = KH * KW, NST = NTAP / TS;
+    constexpr int NTAP = TR ? 4 : KH * KW, NST = NTAP / TS;
+    static_assert(!TR || (KH == 3 && KW == 3 && S == 1 && TS == 4), "a phase's taps in one stage");
     static_assert(NTAP % TS == 0, "whole stages");
     constexpr int NB = WC * CF;
     constexpr int NPX = (HP + 15) / 32 * 32 + 16;
@@ -49,13 +52,13 @@ conv_igemm_split(const ConvParams p) {
     const int col = lane & 15, grp = lane >> 4;
 
     // Workgroup -> tile: the XCD-aware order of conv_igemm.
-    const int nz = p.ntiles;
+    const int nz = p.ntiles * (TR ? 4 : 1);
     const int total = p.gx * p.gy * p.N * nz;
     const int bid = (int)blockIdx.x, xj = bid & 7, xk = bid >> 3;
     const int q8 = total >> 3, r8 = total & 7;
     const int lid = xj < r8 ? xj * (q8 + 1) + xk : r8 * (q8 + 1) + (xj - r8) * q8 + xk;
     int rest = lid / nz;
-    const int nt = lid - rest * nz;
+    const int zl = lid - rest * nz, phase = TR ? (zl & 3) : 0, nt = TR ? (zl >> 2) : zl;
     const int tx = rest % p.gx;
     rest /= p.gx;
     const int ty = rest % p.gy, bi = rest / p.gy;
@@ -79,7 +82,7 @@ conv_igemm_split(const ConvParams p) {
         }
     }
 
-    const int iy0 = oy0 * S - p.pad_t, ix0 = ox0 * S - p.pad_l;
+    const int iy0 = TR ? oy0 - 1 : oy0 * S - p.pad_t, ix0 = TR ? ox0 - 1 : ox0 * S - p.pad_l;
     const float* xg = (const float*)p.x.p + (long long)bi * p.x.bstride;
     const long long xbase = (long long)p.x.c_off + (long long)g * p.cin_g;
 
@@ -135,7 +138,7 @@ conv_igemm_split(const ConvParams p) {
     // Weight slot of stage (chunk, j): taps j * TS .. of blocks nb0 .. nb0 + NB - 1, loaded RW - 1
     // stages ahead (the slot was last read that many stages ago). The lanes' offsets stay, the
     // uniform base moves.
-    const char* const wg = (const char*)((const u32x4*)((const float*)p.w + bi * p.w_bstride) + ((long long)g * p.nchunks * p.nblk_g + nb0) * (NTAP * SPLIT_BLOCK_U));
+    const char* const wg = (const char*)((const u32x4*)((const float*)p.w + phase * p.phase_stride + bi * p.w_bstride) + ((long long)g * p.nchunks * p.nblk_g + nb0) * (NTAP * SPLIT_BLOCK_U));
     const long long wchunk = (long long)p.nblk_g * (NTAP * SPLIT_BLOCK_U * 16);
     unsigned woff[WN];
 #pragma unroll
@@ -185,7 +188,9 @@ conv_igemm_split(const ConvParams p) {
             nslot = nslot + 1 == RW ? 0 : nslot + 1;
 #pragma unroll
             for (int t = 0; t < TS; ++t) {
-                const int tap = j * TS + t, ky = tap / KW, kx = tap - ky * KW;
+                const int tap = j * TS + t;
+                if (TR && t >= p.ntaps[phase]) break;
+                const int ky = TR ? p.tap_dy[phase][t] : tap / KW, kx = TR ? p.tap_dx[phase][t] : tap - tap / KW * KW;
                 SplitFrag a[CF], b[PF];
 #pragma unroll
                 for (int cf = 0; cf < CF; ++cf) {
@@ -226,13 +231,16 @@ conv_igemm_split(const ConvParams p) {
             *reinterpret_cast<f32x4*>(so + ((wp * PF + pf) * 16 + col) * OUT_LD + (wc * CF + cf) * 16 + grp * 4) =
                 NTAP == 1 ? big[cf][pf] : split_sum(big[cf][pf], small[cf][pf]);
     __syncthreads();
+    // Output row / column of position pos (a phase's are every other one).
+    auto oy_of = [&](int pos) { return TR ? 2 * (oy0 + (pos >> 4)) + (phase >> 1) : oy0 + (pos >> 4); };
+    auto ox_of = [&](int pos) { return TR ? 2 * (ox0 + (pos & 15)) + (phase & 1) : ox0 + (pos & 15); };
     const bool full = nb0 * 16 + NB * 16 <= p.cout_g;  // all of the tile's channels are real
     if (full && epilogue_simple(p)) {
         constexpr int QP8 = NB * 2;  // 8 channels per thread and step
 #pragma unroll 4
         for (int u = tid; u < TY * 16 * QP8; u += NT) {
             const int pos = u / QP8, c8 = u - pos * QP8;
-            const int oy = oy0 + (pos >> 4), ox = ox0 + (pos & 15);
+            const int oy = oy_of(pos), ox = ox_of(pos);
             const f32x4 v0 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8);
             const f32x4 v1 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8 + 4);
             if (oy < p.OH && ox < p.OW) epilogue_store8<float>(p, bi, oy, ox, g * p.cout_g + nb0 * 16 + c8 * 8, v0, v1);
@@ -245,7 +253,7 @@ conv_igemm_split(const ConvParams p) {
         constexpr int QP = NB * 4;
         for (int u = tid; u < TY * 16 * QP; u += NT) {
             const int pos = u / QP, q = u - pos * QP, cq = q % NB, sub = q / NB;
-            const int oy = oy0 + (pos >> 4), ox = ox0 + (pos & 15);
+            const int oy = oy_of(pos), ox = ox_of(pos);
             if (oy >= p.OH || ox >= p.OW) continue;
             const float* v = so + pos * OUT_LD + cq * 16 + sub;
             epilogue_store_ps2<float>(p, bi, oy, ox, sub, (g * p.cout_g + nb0 * 16) / 4 + cq * 4,
@@ -256,11 +264,208 @@ conv_igemm_split(const ConvParams p) {
     constexpr int QP = NB * 4;
     for (int u = tid; u < TY * 16 * QP; u += NT) {
         const int pos = u / QP, cq = u - pos * QP;
-        const int oy = oy0 + (pos >> 4), ox = ox0 + (pos & 15);
+        const int oy = oy_of(pos), ox = ox_of(pos);
         const int ocl = nb0 * 16 + cq * 4;
         if (oy >= p.OH || ox >= p.OW || ocl >= p.cout_g) continue;
         const f32x4 v = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + cq * 4);
         epilogue_store<float>(p, bi, oy, ox, g * p.cout_g + ocl, min(4, p.cout_g - ocl), v);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Stride-2 transposed 3x3 convolution, padding 1, the four output phases of a tile in one
+// workgroup (conv_tr_merged's plan, conv.hip): WC * 2 blocks of 16 channels x WP * 2 rows x 16
+// columns of input positions; each wave accumulates two blocks x two rows for all four phases. A
+// phase reads the 2 x 2 input neighbourhood of a position, so the halo is one row and one column
+// and a chunk's nine taps share its few fragments. Weights (split, phase by phase) go through an
+// LDS ring three taps at a time. Per output the sums are conv_igemm_split's: bias, then per chunk
+// its phase's taps in table order.
+// ---------------------------------------------------------------------------------------------
+template <int WC, int WP>
+__global__ void __launch_bounds__(WC * WP * 64, 2)
+conv_tr_merged_split(const ConvParams p) {
+    constexpr int NT = WC * WP * 64, CF = 2, PF = 2;
+    constexpr int TY = WP * PF, HY = TY + 1, HX = 17, HP = HY * HX;
+    constexpr int NB = WC * CF, TS = 3, NST = 3;
+    constexpr int NPX = (HP + 15) / 32 * 32 + 16;
+    constexpr int HALO_U = 6 * NPX, W_U = NB * TS * SPLIT_BLOCK_U;
+    constexpr int OUT_LD = NB * 16 + 4, OUT_U = (TY * 16 * OUT_LD + 3) / 4;
+    constexpr int RUN_U = HALO_U + 2 * W_U;
+    constexpr int LDS_U = RUN_U > OUT_U ? RUN_U : OUT_U;
+    constexpr int HN = (HP * 4 + NT - 1) / NT, WN = (W_U + NT - 1) / NT;
+    // Taps in packing order: phase (py * 2 + px) and input offset (dy, dx) of each.
+    constexpr int PH[9] = {0, 1, 1, 2, 2, 3, 3, 3, 3};
+    constexpr int DY[9] = {0, 0, 0, 1, 0, 1, 1, 0, 0}, DX[9] = {0, 1, 0, 0, 0, 1, 0, 1, 0};
+    __shared__ u32x4 s_lds[LDS_U];
+    u32x2* const s_hhi = (u32x2*)(s_lds + 4 * NPX);
+    u32x4* const s_w = s_lds + HALO_U;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wc = wave % WC, wp = wave / WC;
+    const int col = lane & 15, grp = lane >> 4;
+
+    const int nz = p.ntiles;
+    const int total = p.gx * p.gy * p.N * nz;
+    const int bid = (int)blockIdx.x, xj = bid & 7, xk = bid >> 3;
+    const int q8 = total >> 3, r8 = total & 7;
+    const int lid = xj < r8 ? xj * (q8 + 1) + xk : r8 * (q8 + 1) + (xj - r8) * q8 + xk;
+    int rest = lid / nz;
+    const int nb0 = (lid - rest * nz) * NB;
+    const int tx = rest % p.gx;
+    rest /= p.gx;
+    const int ty = rest % p.gy, bi = rest / p.gy;
+    const int ox0 = tx * 16, oy0 = ty * TY;
+    if (nb0 * 16 >= p.cout_g) return;  // padding blocks only (uniform)
+
+    f32x4 big[4][CF][PF], small[4][CF][PF];
+#pragma unroll
+    for (int cf = 0; cf < CF; ++cf) {
+        const int ocl = (nb0 + wc * CF + cf) * 16 + grp * 4;
+        f32x4 b;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[i] = (p.bias && ocl + i < p.cout_g) ? p.bias[ocl + i] : 0.0f;
+#pragma unroll
+        for (int ph = 0; ph < 4; ++ph)
+#pragma unroll
+            for (int pf = 0; pf < PF; ++pf) {
+                big[ph][cf][pf] = b;
+                small[ph][cf][pf] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+    }
+
+    const float* xg = (const float*)p.x.p + (long long)bi * p.x.bstride + p.x.c_off;
+    const float* hp[HN];
+    int hstep[HN], hdst[HN];
+#pragma unroll
+    for (int i = 0; i < HN; ++i) {
+        const int u = tid + i * NT, pix = u >> 2, q = u & 3;
+        const int hy = pix / HX, hx = pix - hy * HX;
+        const int iy = oy0 + hy, ix = ox0 + hx;
+        const bool in = u < HP * 4 && iy < p.H && ix < p.W;
+        hp[i] = in ? xg + (long long)iy * p.x.row + (long long)ix * p.x.cs + q * 4 : (const float*)g_zero_split;
+        hstep[i] = in ? 16 : 0;
+        hdst[i] = q * NPX + pix;
+    }
+    const int qv = (tid & 3) * 4;
+    u32x4 rh[HN];
+    auto load_halo = [&](int chunk) __attribute__((always_inline)) {
+        if (chunk * 16 + 16 <= p.cin_g) {
+#pragma unroll
+            for (int i = 0; i < HN; ++i) {
+                rh[i] = *(const u32x4*)hp[i];
+                hp[i] += hstep[i];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < HN; ++i)
+                rh[i] = *(chunk * 16 + qv < p.cin_g ? (const u32x4*)hp[i] : g_zero_split);
+        }
+    };
+    const char* const wg = (const char*)((const u32x4*)p.w + (long long)nb0 * (TR_MERGED_TAPS * SPLIT_BLOCK_U));
+    const long long wchunk = (long long)p.nblk_g * (TR_MERGED_TAPS * SPLIT_BLOCK_U * 16);
+    unsigned woff[WN];
+#pragma unroll
+    for (int i = 0; i < WN; ++i) {
+        const int u = tid + i * NT, nb = u / (TS * SPLIT_BLOCK_U);
+        woff[i] = (unsigned)(nb * (TR_MERGED_TAPS * SPLIT_BLOCK_U) + (u - nb * (TS * SPLIT_BLOCK_U))) * 16;
+    }
+    auto issue_stage = [&](int st, int slot) __attribute__((always_inline)) {
+        const int c = st / NST;
+        const char* src = wg + c * wchunk + (st - c * NST) * (TS * SPLIT_BLOCK_U * 16);
+        u32x4* dst = s_w + slot * W_U;
+#pragma unroll
+        for (int i = 0; i < WN; ++i) {
+            const int ub = wave * 64 + i * NT;
+            if (ub >= W_U) break;
+            if (ub + lane < W_U) lds_dma16_at(src, woff[i], dst + ub);
+        }
+    };
+
+    const int nchunks = p.nchunks, nst = nchunks * NST;
+    load_halo(0);
+    issue_stage(0, 0);
+#pragma unroll 1
+    for (int chunk = 0, st = 0; chunk < nchunks; ++chunk) {
+        auto stage = [&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            if (j == 0) {
+                if (chunk > 0) __syncthreads();  // every wave is done with the last halo
+#pragma unroll
+                for (int i = 0; i < HN; ++i) {
+                    const SplitFrag f = split_f32(__builtin_bit_cast(f32x4, rh[i]));
+                    if (tid + i * NT < HP * 4) {
+                        s_lds[hdst[i]] = f.lo;
+                        s_hhi[hdst[i]] = f.hi;
+                    }
+                }
+            }
+            // This stage's weights have landed; the next chunk's halo loads, issued after them, may
+            // still fly.
+            if (j == 1 && chunk + 1 < nchunks) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(HN) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+            __syncthreads();
+            if (st + 1 < nst) issue_stage(st + 1, (st + 1) & 1);
+            if (j == 0 && chunk + 1 < nchunks) load_halo(chunk + 1);
+            const u32x4* sw = s_w + (st & 1) * W_U;
+            ++st;
+#pragma unroll
+            for (int t = 0; t < TS; ++t) {
+                constexpr int E = j * TS;
+                SplitFrag a[CF], b[PF];
+#pragma unroll
+                for (int cf = 0; cf < CF; ++cf) {
+                    const u32x4* w = sw + ((wc * CF + cf) * TS + t) * SPLIT_BLOCK_U;
+                    a[cf] = SplitFrag{w[lane], ((const u32x2*)(w + 64))[lane]};
+                }
+#pragma unroll
+                for (int pf = 0; pf < PF; ++pf) {
+                    const int i = grp * NPX + (wp * PF + pf + DY[E + t]) * HX + col + DX[E + t];
+                    b[pf] = SplitFrag{s_lds[i], s_hhi[i]};
+                }
+#pragma unroll
+                for (int cf = 0; cf < CF; ++cf)
+#pragma unroll
+                    for (int pf = 0; pf < PF; ++pf)
+                        mma_split(big[PH[E + t]][cf][pf], small[PH[E + t]][cf][pf], a[cf], b[pf]);
+            }
+        };
+        stage(std::integral_constant<int, 0>{});
+        stage(std::integral_constant<int, 1>{});
+        stage(std::integral_constant<int, 2>{});
+    }
+
+    // One phase at a time through the LDS transpose (NHWC output without pixel shuffle).
+    float* so = reinterpret_cast<float*>(s_lds);
+#pragma unroll
+    for (int ph = 0; ph < 4; ++ph) {
+        __syncthreads();
+#pragma unroll
+        for (int cf = 0; cf < CF; ++cf)
+#pragma unroll
+            for (int pf = 0; pf < PF; ++pf)
+                *reinterpret_cast<f32x4*>(so + ((wp * PF + pf) * 16 + col) * OUT_LD + (wc * CF + cf) * 16 + grp * 4) =
+                    split_sum(big[ph][cf][pf], small[ph][cf][pf]);
+        __syncthreads();
+        if (nb0 * 16 + NB * 16 <= p.cout_g) {
+            constexpr int QP8 = NB * 2;
+#pragma unroll 4
+            for (int u = tid; u < TY * 16 * QP8; u += NT) {
+                const int pos = u / QP8, c8 = u - pos * QP8;
+                const int oy = 2 * (oy0 + (pos >> 4)) + (ph >> 1), ox = 2 * (ox0 + (pos & 15)) + (ph & 1);
+                const f32x4 v0 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8);
+                const f32x4 v1 = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + c8 * 8 + 4);
+                if (oy < p.OH && ox < p.OW) epilogue_store8<float>(p, bi, oy, ox, nb0 * 16 + c8 * 8, v0, v1);
+            }
+        } else {
+            constexpr int QP = NB * 4;
+            for (int u = tid; u < TY * 16 * QP; u += NT) {
+                const int pos = u / QP, cq = u - pos * QP, ocl = nb0 * 16 + cq * 4;
+                const int oy = 2 * (oy0 + (pos >> 4)) + (ph >> 1), ox = 2 * (ox0 + (pos & 15)) + (ph & 1);
+                if (oy >= p.OH || ox >= p.OW || ocl >= p.cout_g) continue;
+                const f32x4 v = *reinterpret_cast<const f32x4*>(so + pos * OUT_LD + cq * 4);
+                epilogue_store<float>(p, bi, oy, ox, ocl, min(4, p.cout_g - ocl), v);
+            }
+        }
     }
 }
 
@@ -461,17 +666,17 @@ hipError_t go_1x1_split(const ConvParams& p0, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int KH, int KW, int S, int WC, int WP, int CF, int PF, int TS, int NHB, int RW>
+template <int KH, int KW, int S, bool TR, int WC, int WP, int CF, int PF, int TS, int NHB, int RW>
 hipError_t go_split(const ConvParams& p0, hipStream_t s) {
     constexpr int TY = WP * PF;
     ConvParams p = p0;
     if (p.ntiles != p.groups * p.nblk_g / (WC * CF) || p.nblk_g % (WC * CF) || p.N < 1 || p.N > MAXB)
         return hipErrorInvalidValue;
-    p.gx = (p.OW + 15) / 16;
-    p.gy = (p.OH + TY - 1) / TY;
-    const long long total = (long long)p.gx * p.gy * p.N * p.ntiles;
+    p.gx = ((TR ? (p.OW + 1) / 2 : p.OW) + 15) / 16;
+    p.gy = ((TR ? (p.OH + 1) / 2 : p.OH) + TY - 1) / TY;
+    const long long total = (long long)p.gx * p.gy * p.N * p.ntiles * (TR ? 4 : 1);
     if (total <= 0 || total > (1ll << 30)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((conv_igemm_split<KH, KW, S, WC, WP, CF, PF, TS, NHB, RW>), dim3((unsigned)total),
+    hipLaunchKernelGGL((conv_igemm_split<KH, KW, S, TR, WC, WP, CF, PF, TS, NHB, RW>), dim3((unsigned)total),
                        dim3(WC * WP * 64), 0, s, p);
     return hipGetLastError();
 }
@@ -480,7 +685,7 @@ hipError_t go_split(const ConvParams& p0, hipStream_t s) {
 
 // Instantiated shapes per kind: (wc, wp, cf, pf), taps per weight slot, halo buffers, slots.
 #define ZJAI_SPLIT(KIND, KH, KW, S, A, B, C, D, TS, NHB, RW) \
-    if (kind == KIND && c.wc == A && c.wp == B && c.cf == C && c.pf == D) return go_split<KH, KW, S, A, B, C, D, TS, NHB, RW>(p, s);
+    if (kind == KIND && c.wc == A && c.wp == B && c.cf == C && c.pf == D) return go_split<KH, KW, S, KIND == CK_T3, A, B, C, D, TS, NHB, RW>(p, s);
 
 hipError_t launch_conv_split(int kind, TileCfg c, const ConvParams& p, hipStream_t s) {
     ZJAI_SPLIT(CK_1x1, 1, 1, 1, 1, 4, 4, 2, 1, 1, 2)
@@ -500,6 +705,9 @@ hipError_t launch_conv_split(int kind, TileCfg c, const ConvParams& p, hipStream
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 4, 4, 2, 1, 1, 3)
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 8, 2, 1, 4, 1, 2)
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 8, 1, 1, 4, 1, 2)
+    ZJAI_SPLIT(CK_T3, 3, 3, 1, 1, 4, 4, 2, 4, 1, 2)
+    ZJAI_SPLIT(CK_T3, 3, 3, 1, 1, 8, 2, 1, 4, 1, 2)
+    ZJAI_SPLIT(CK_T3, 3, 3, 1, 1, 8, 1, 1, 4, 1, 2)
     return hipErrorInvalidValue;
 }
 
@@ -519,6 +727,36 @@ hipError_t launch_conv1x1_ring_split(TileCfg c, const ConvParams& p, hipStream_t
     ZJAI_1X1(1, 4, 1, 1)
 #undef ZJAI_1X1
     return hipErrorInvalidValue;
+}
+
+bool conv_tr_merged_split_ok(const ConvParams& p) {
+    // The 3x3 / padding-1 tap table (conv_tr_merged_split's constants, offsets from the input row).
+    static const int n[4] = {1, 2, 2, 4};
+    static const int dy[4][4] = {{1}, {1, 1}, {2, 1}, {2, 2, 1, 1}}, dx[4][4] = {{1}, {2, 1}, {1, 1}, {2, 1, 2, 1}};
+    for (int ph = 0; ph < 4; ++ph) {
+        if (p.ntaps[ph] != n[ph]) return false;
+        for (int t = 0; t < n[ph]; ++t)
+            if (p.tap_dy[ph][t] != dy[ph][t] || p.tap_dx[ph][t] != dx[ph][t]) return false;
+    }
+    return p.groups == 1 && p.nblk_g % TR_MERGED_NB == 0 && p.N >= 1 && p.N <= MAXB && p.out_mode == OUT_NHWC && p.ps == 1 &&
+           !p.relu6_in && !p.w_bstride;
+}
+
+template <int WC, int WP>
+static hipError_t go_merged_split(const ConvParams& p0, hipStream_t s) {
+    ConvParams p = p0;
+    p.ntiles = p.nblk_g / (WC * 2);
+    p.gx = ((p.OW + 1) / 2 + 15) / 16;
+    p.gy = ((p.OH + 1) / 2 + WP * 2 - 1) / (WP * 2);
+    const long long total = (long long)p.gx * p.gy * p.N * p.ntiles;
+    if (p.nblk_g % (WC * 2) || total <= 0 || total > (1ll << 30)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((conv_tr_merged_split<WC, WP>), dim3((unsigned)total), dim3(WC * WP * 64), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_conv_tr_merged_split(const ConvParams& p, hipStream_t s) {
+    if (!conv_tr_merged_split_ok(p)) return hipErrorInvalidValue;
+    return go_merged_split<2, 2>(p, s);
 }
 
 }  // namespace zjai

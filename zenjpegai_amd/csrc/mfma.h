@@ -8,19 +8,10 @@ namespace zjai {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// 16x16 tile, 32 channels of K per instruction for the 16-bit types (four 16x16x4 steps for
-// f32). Lane (i, g) = (lane % 16, lane / 16) supplies row / column i and K group g (8 channels
-// of a 16-bit type, 4 of f32); accumulator register r holds row 4 * g + r of column i.
+// 16x16 tile, 32 channels of K per instruction (16-bit types). Lane (i, g) = (lane % 16, lane / 16)
+// supplies row / column i and K group g (8 channels); accumulator register r holds row 4 * g + r
+// of column i.
 template <typename T> struct Mma16;
-template <> struct Mma16<float> {
-    static __device__ __forceinline__ void run(f32x4& acc, u32x4 a, u32x4 b) {
-        const f32x4 av = __builtin_bit_cast(f32x4, a), bv = __builtin_bit_cast(f32x4, b);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[0], bv[0], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[1], bv[1], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[2], bv[2], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[3], bv[3], acc, 0, 0, 0);
-    }
-};
 template <> struct Mma16<_Float16> {
     static __device__ __forceinline__ void run(f32x4& acc, u32x4 a, u32x4 b) {
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),

@@ -359,6 +359,7 @@ TileCfg conv_tile_cfg(int cout_g, int kind, int dtype) {
             return cout_g <= 16 ? TileCfg{1, 4, 1, 1} : cout_g <= 32 ? TileCfg{1, 4, 2, 1}
                    : wide ? TileCfg{2, 2, 4, 2} : TileCfg{1, 4, 4, 2};
         if (kind == CK_1x1) return cout_g <= 16 ? TileCfg{1, 4, 1, 2} : cout_g <= 32 ? TileCfg{1, 4, 2, 2} : TileCfg{1, 4, 4, 2};
+        // 2x2 and the phases of a transposed convolution
         return cout_g <= 16 ? TileCfg{1, 8, 1, 1} : cout_g <= 32 ? TileCfg{1, 8, 2, 1} : TileCfg{1, 4, 4, 2};
     }
     if (cout_g <= 16) return TileCfg{1, 4, 1, 2};
@@ -482,8 +483,10 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
     const int CK = 64 / dtype_size(dtype);
     L->nblk_g = round_up(ceil_div(cout, 16), NB);
     L->nchunks = ceil_div(cin, CK);
-    L->phase_stride = (long long)L->nchunks * L->nblk_g * 4 * 16 * CK;
-    std::vector<float> pk((size_t)4 * L->phase_stride, 0.0f);
+    const size_t pstride = (size_t)L->nchunks * L->nblk_g * 4 * 16 * CK;  // packed values per phase
+    // In elements of the storage type; a split f32 block takes 1.5 times the room.
+    L->phase_stride = dtype == DT_F32 ? (long long)pstride / 2 * 3 : (long long)pstride;
+    std::vector<float> pk(4 * pstride, 0.0f);
     for (int ph = 0; ph < 4; ++ph) {
         const int py = ph >> 1, px = ph & 1;
         int t = 0;
@@ -493,15 +496,16 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
                 for (int oc = 0; oc < cout; ++oc)
                     for (int ic = 0; ic < cin; ++ic) {
                         const int ch = ic / CK, kk = ic % CK, nb = oc / 16, r = oc % 16;
-                        const size_t dst = (size_t)ph * L->phase_stride +
+                        const size_t dst = (size_t)ph * pstride +
                                            ((((size_t)ch * L->nblk_g + nb) * 4 + t) * 16 + r) * CK + kk;
                         pk[dst] = weight[(((size_t)ic * cout + oc) * k + ky) * k + kx];
                     }
             }
     }
-    L->wpk = upload_as(ctx, pk, dtype, &L->wpk_bytes, &L->dev_bytes);
+    L->wpk = dtype == DT_F32 ? upload_split(pk, &L->wpk_bytes, &L->dev_bytes)
+                             : upload_as(ctx, pk, dtype, &L->wpk_bytes, &L->dev_bytes);
     if (bias) L->bias = upload_f32(bias, cout, &L->dev_bytes);
-    if (k == 3 && cout > 8 && conv_tr_merged_taps_supported(L->ntaps) && L->nblk_g % TR_MERGED_NB == 0) {
+    if (k == 3 && cout > 8 && (dtype != DT_F32 || pad == 1) && conv_tr_merged_taps_supported(L->ntaps) && L->nblk_g % TR_MERGED_NB == 0) {
         // All four phases per workgroup (launch_conv_tr_merged): the nine taps side by side per
         // K chunk and block, phase by phase, each phase's taps in its table order.
         std::vector<float> pm((size_t)L->nchunks * L->nblk_g * TR_MERGED_TAPS * 16 * CK, 0.0f);
@@ -510,7 +514,7 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
                 int e = 0;
                 for (int ph = 0; ph < 4; ++ph)
                     for (int t = 0; t < L->ntaps[ph]; ++t, ++e) {
-                        const float* src = pk.data() + (size_t)ph * L->phase_stride +
+                        const float* src = pk.data() + (size_t)ph * pstride +
                                            (((size_t)ch * L->nblk_g + nb) * 4 + t) * 16 * CK;
                         float* dst = pm.data() + (((size_t)ch * L->nblk_g + nb) * TR_MERGED_TAPS + e) * 16 * CK;
                         if (dtype != DT_F32) {
@@ -525,7 +529,8 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
                         }
                     }
             }
-        L->wpk_m = upload_as(ctx, pm, dtype, &L->wpk_m_bytes, &L->dev_bytes);
+        L->wpk_m = dtype == DT_F32 ? upload_split(pm, &L->wpk_m_bytes, &L->dev_bytes)
+                                   : upload_as(ctx, pm, dtype, &L->wpk_m_bytes, &L->dev_bytes);
     }
     if (cout <= 8) {
         // Narrow layers run on the vector ALUs (launch_convT_narrow) from an f32 copy of the
@@ -587,6 +592,9 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
 //     62 / 48 / 64; 172^2 (132) 58 / 43 / 43; 51 x 75 (24) 54 / 32 / 26, 16 x 4 19.
 //   2x2 160 -> 256: 135 x 240 (1020) 64 ch x 8 rows 74, 32 x 8 (eight waves) 91, 16 x 8 114; 64^2
 //     (128) 29 / 18 / 21; 144 -> 128 at 64^2 (64) 26 / 16 / 14.
+//   transposed, phase by phase (workgroups of all four): k4 160 -> 64 from 135 x 240 (1020) 64 ch x 8
+//     rows 78, 32 x 8 88, 16 x 8 121; 192 -> 128 from 64^2 (256) 37 / 34 / 43; 160 -> 160 from 12 x 20
+//     (48) 30 / 19 / 17.
 //   32-channel groups and outputs: 256^2 (512 of 32 x 8) 32 ch x 8 rows 16.1, 16 x 8 by eight waves
 //     18.0; five groups at 34 x 60 (100) 11.2 / 8.2.
 static TileCfg split_tile_cfg(const Layer& L, int N, int OH, int OW) {
@@ -599,6 +607,10 @@ static TileCfg split_tile_cfg(const Layer& L, int N, int OH, int OW) {
                : w < 384 ? TileCfg{1, 4, 4, 2} : L.cfg;
     }
     if (nb <= 2 || L.kind == CK_1x1) return L.cfg;
+    if (L.kind == CK_T3) {  // per phase
+        const long long w = (long long)(((OW + 1) / 2 + 15) / 16) * (((OH + 1) / 2 + 7) / 8) * (tiles * nb);
+        return w < 64 ? TileCfg{1, 8, 1, 1} : w < 512 ? TileCfg{1, 8, 2, 1} : L.cfg;
+    }
     const long long w = cols * rows8 * (tiles * nb / 4);
     if (L.kind == CK_3x3_S2) return w < 48 ? TileCfg{1, 4, 1, 1} : w < 160 ? TileCfg{1, 4, 2, 1} : w < 512 ? TileCfg{1, 4, 4, 1} : L.cfg;
     return w < 96 ? TileCfg{1, 8, 1, 1} : w < 384 ? TileCfg{1, 8, 2, 1} : L.cfg;
@@ -642,14 +654,16 @@ static TileCfg launch_tile_cfg(const Layer& L, int N, int OH, int OW) {
     return c;
 }
 
-// Transposed 3x3 layers take the merged four-phase kernel when its grid (16 x 16 phase positions
-// x 64 channels per workgroup) has at least 256 workgroups, else the phase-split kernel on a
-// narrow tile: 192 -> 192 from 40^2 runs 119 -> 38 us (fp32), from 80^2 125 -> 88 us; from 160^2
-// the merged kernel is faster (257 vs 304 us).
+// Transposed 3x3 layers take the merged four-phase kernel on maps large enough for its grid, else
+// the phase-split kernel on a narrow tile. 16-bit: at least 256 workgroups of 16 x 16 phase
+// positions x 64 channels. f32 (64 channels x 4 rows of positions per workgroup): from 60
+// tiles of 16 x 8 positions -- 128 -> 128 from 88^2 (66 tiles) merged 36 us, phase-split 44; from 176^2 73 / 111;
+// 64 -> 64 from 108^2 (98) 20.5 / 21.0; below it 160 -> 128 from 64 x 96 (48) 34.6 / 35.2, 128 -> 128
+// from 52 x 76 (35) 28.8 / 27.8 and from 26 x 38 (15) 27 / 17.
 static bool convT_merged_fills(const Layer& L, int N, int OH, int OW) {
-    const long long wm = (long long)(((OW + 1) / 2 + 15) / 16) * (((OH + 1) / 2 + 15) / 16) * N *
-                         (L.nblk_g / TR_MERGED_NB);
-    return wm >= 256;
+    const long long cols = ((OW + 1) / 2 + 15) / 16, rows = (OH + 1) / 2;
+    if (L.dtype == DT_F32) return cols * ((rows + 7) / 8) * N >= 60;
+    return cols * ((rows + 15) / 16) * N * (L.nblk_g / TR_MERGED_NB) >= 256;
 }
 
 // Tile of an f32 1x1 launch by its number of 64-channel x 128-position workgroups: narrower tiles
@@ -680,12 +694,7 @@ std::string conv_kernel_name(int kind, int dtype, TileCfg c) {
         snprintf(buf, sizeof buf, "conv_igemm_split<%s, %d, %d, %d, %d>", geo[kind], c.wc, c.wp, c.cf, c.pf);
         return buf;
     }
-    const bool dma = dtype == DT_F32 && c.cf == 2 && c.pf == 4 &&
-                     ((c.wc == 2 && (c.wp == 2 || c.wp == 4)) || (c.wc == 4 && c.wp == 2));
-    if (dma)  // the fp32 dense shapes run conv_dma_f32 (conv.hip)
-        snprintf(buf, sizeof buf, "conv_dma_f32<%s, %d, %d, %d, %d>", geo[kind], c.wc, c.wp, c.cf, c.pf);
-    else
-        snprintf(buf, sizeof buf, "conv_igemm<%s, %s, %d, %d, %d, %d>", ty[dtype], geo[kind], c.wc, c.wp, c.cf, c.pf);
+    snprintf(buf, sizeof buf, "conv_igemm<%s, %s, %d, %d, %d, %d>", ty[dtype], geo[kind], c.wc, c.wp, c.cf, c.pf);
     return buf;
 }
 static View view_of(const Tensor* t) { return t ? t->v : View{nullptr, 0, 0, 0, 0}; }
@@ -825,7 +834,8 @@ static TensorP conv_forward_impl(Context& ctx, const Layer& L, const TensorP& x,
                            std::to_string(L.ntaps[3]) + ">",
                        2.0 * macs,
                        bytes - (double)L.wpk_bytes + (double)L.wpk_m_bytes);
-        ZJAI_HIP(launch_conv_tr_merged(L.dtype, p, ctx.stream));
+        if (L.dtype == DT_F32) ZJAI_HIP(launch_conv_tr_merged_split(p, ctx.stream));
+        else ZJAI_HIP(launch_conv_tr_merged(L.dtype, p, ctx.stream));
         return y;
     }
     // conv3x3_m32's 256-position tiles carry twice the work of conv_igemm's 64-channel ones: with

@@ -69,8 +69,8 @@ __device__ __forceinline__ f32x4 mfma_bf16(u32x4 a, u32x4 b, f32x4 c) {
 }
 __device__ __forceinline__ u32x4 split_hi(const SplitFrag& f) { return u32x4{f.lo[2], f.lo[3], f.hi[0], f.hi[1]}; }
 __device__ __forceinline__ void mma_split(f32x4& big, f32x4& small, const SplitFrag& a, const SplitFrag& b) {
-    big = mfma_bf16(a.lo, b.lo, big);
     small = mfma_bf16(a.lo, split_hi(b), small);
+    big = mfma_bf16(a.lo, b.lo, big);
     small = mfma_bf16(split_hi(a), b.lo, small);
 }
 
