@@ -66,7 +66,7 @@ TensorP planar_upload(Context& c, const float* data, int ch, int h, int w, int d
     const size_t n = (size_t)ch * h * w;
     float* stage = (float*)c.pool.alloc(n * 4);
     std::shared_ptr<void> keep(stage, [&c](void* q) { c.pool.release(q); });
-    ZJAI_HIP(hipMemcpyAsync(stage, data, n * 4, hipMemcpyHostToDevice, c.stream));
+    c.top().copier.to_device(stage, data, n * 4, c.stream);
     {
         LaunchScope sc(c, kname("k_planar_to_nhwc", dtype), 0.0, (4.0 + dtype_size(dtype)) * n);
         ZJAI_HIP(launch_planar_to_nhwc(stage, ch, h, w, Windows{}, 1, h, w, t->v, dtype, c.stream));
@@ -139,6 +139,7 @@ extern "C" int32_t zjai_ctx_create(int32_t device, uint32_t flags, zjai_ctx** ou
         ZJAI_HIP(hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking));
         ZJAI_HIP(hipEventCreate(&ctx->c.ev0));
         ZJAI_HIP(hipEventCreate(&ctx->c.ev1));
+        ctx->c.copier.create();
     });
     if (rc != ZJAI_OK) {
         delete ctx;
@@ -287,7 +288,7 @@ extern "C" int32_t zjai_tensor_to_planar(zjai_ctx* ctx, const zjai_tensor* t, fl
             LaunchScope sc(ctx->c, kname("k_nhwc_to_planar", x.dtype), 0.0, (4.0 + dtype_size(x.dtype)) * n);
             ZJAI_HIP(launch_nhwc_to_planar(x.v, x.dtype, x.n, x.c, x.h, x.w, stage, ctx->c.stream));
         }
-        ZJAI_HIP(hipMemcpyAsync(data, stage, n * 4, hipMemcpyDeviceToHost, ctx->c.stream));
+        ctx->c.copier.to_host(data, stage, n * 4, ctx->c.stream);
         ZJAI_HIP(hipStreamSynchronize(ctx->c.stream));
     });
 }
@@ -629,7 +630,7 @@ static void run_to_host(zjai_ctx* ctx, const zjai_net* net, const TensorP& a, co
     po.win_w[0] = ow;
     if (primary) primary_forward(ctx->c, *net->n, a, h, w, po);
     else secondary_forward(ctx->c, *net->n, a, b, h, w, po);
-    ZJAI_HIP(hipMemcpyAsync(out, dev, n * 4, hipMemcpyDeviceToHost, ctx->c.stream));
+    ctx->c.copier.to_host(out, dev, n * 4, ctx->c.stream);
     ZJAI_HIP(hipStreamSynchronize(ctx->c.stream));
 }
 
@@ -1008,11 +1009,9 @@ extern "C" int32_t zjai_picture_upload(zjai_ctx* ctx, zjai_picture* pic, const f
     if (!ctx || !pic || !y_hat) return ZJAI_E_INVALID_ARGUMENT;
     return guard(ctx, [&] {
         need(!pic->net_uv || uv_hat, "chroma latent missing");
-        ZJAI_HIP(hipMemcpyAsync(pic->y_hat, y_hat, sizeof(float) * 160 * (size_t)pic->lh * pic->lw,
-                                hipMemcpyHostToDevice, ctx->c.stream));
+        ctx->c.copier.to_device(pic->y_hat, y_hat, sizeof(float) * 160 * (size_t)pic->lh * pic->lw, ctx->c.stream);
         if (pic->net_uv)
-            ZJAI_HIP(hipMemcpyAsync(pic->uv_hat, uv_hat, sizeof(float) * 96 * (size_t)pic->lh * pic->lw,
-                                    hipMemcpyHostToDevice, ctx->c.stream));
+            ctx->c.copier.to_device(pic->uv_hat, uv_hat, sizeof(float) * 96 * (size_t)pic->lh * pic->lw, ctx->c.stream);
         ZJAI_HIP(hipStreamSynchronize(ctx->c.stream));
         pic->uploaded = true;
     });
@@ -1209,13 +1208,12 @@ extern "C" int32_t zjai_picture_download(zjai_ctx* ctx, zjai_picture* pic, void*
     if (!ctx || !pic || !y) return ZJAI_E_INVALID_ARGUMENT;
     return guard(ctx, [&] {
         const size_t sb = pic->sample_bytes();
-        ZJAI_HIP(hipMemcpyAsync(y, pic->out_y, sb * (size_t)pic->out_h * pic->out_w, hipMemcpyDeviceToHost,
-                                ctx->c.stream));
+        ctx->c.copier.to_host(y, pic->out_y, sb * (size_t)pic->out_h * pic->out_w, ctx->c.stream);
         if (pic->net_uv) {
             need(u && v, "chroma outputs missing");
             const size_t n = (size_t)pic->ch() * pic->cw();
-            ZJAI_HIP(hipMemcpyAsync(u, pic->out_uv, sb * n, hipMemcpyDeviceToHost, ctx->c.stream));
-            ZJAI_HIP(hipMemcpyAsync(v, (char*)pic->out_uv + sb * n, sb * n, hipMemcpyDeviceToHost, ctx->c.stream));
+            ctx->c.copier.to_host(u, pic->out_uv, sb * n, ctx->c.stream);
+            ctx->c.copier.to_host(v, (char*)pic->out_uv + sb * n, sb * n, ctx->c.stream);
         }
         ZJAI_HIP(hipStreamSynchronize(ctx->c.stream));
     });
@@ -1248,13 +1246,13 @@ extern "C" int32_t zjai_resize(zjai_ctx* ctx, int32_t mode, const float* src, in
         // Flat f32 scratch from the context's pool: [1][1][n / 8][8] tensors.
         TensorP a = cx.alloc(1, 8, 1, (int)((n_in + 7) / 8), DT_F32);
         TensorP b = cx.alloc(1, 8, 1, (int)((n_out + 7) / 8), DT_F32);
-        ZJAI_HIP(hipMemcpyAsync(a->v.p, src, n_in * 4, hipMemcpyHostToDevice, cx.stream));
+        cx.copier.to_device(a->v.p, src, n_in * 4, cx.stream);
         {
             LaunchScope sc(cx, mode == ZJAI_RESIZE_BICUBIC ? "k_resize_bicubic" : "k_resize_bilinear",
                            0.0, 4.0 * (double)(n_in + n_out));
             ZJAI_HIP(launch_resize(mode, (const float*)a->v.p, c, h, w, (float*)b->v.p, out_h, out_w, cx.stream));
         }
-        ZJAI_HIP(hipMemcpyAsync(dst, b->v.p, n_out * 4, hipMemcpyDeviceToHost, cx.stream));
+        cx.copier.to_host(dst, b->v.p, n_out * 4, cx.stream);
         ZJAI_HIP(hipStreamSynchronize(cx.stream));
     });
 }
@@ -1280,9 +1278,9 @@ extern "C" int32_t zjai_picture_download_rgb(zjai_ctx* ctx, zjai_picture* pic, i
             ZJAI_HIP(launch_picture_rgb((const float*)pic->out_y, pic->out_h, pic->out_w, u, v, ch, cw, bit_depth,
                                         pic->out_rgb, rgb_planes ? pic->out_rgbf : nullptr, cx.stream));
         }
-        ZJAI_HIP(hipMemcpyAsync(rgb, pic->out_rgb, n * 3 * sizeof(uint16_t), hipMemcpyDeviceToHost, cx.stream));
+        cx.copier.to_host(rgb, pic->out_rgb, n * 3 * sizeof(uint16_t), cx.stream);
         if (rgb_planes)
-            ZJAI_HIP(hipMemcpyAsync(rgb_planes, pic->out_rgbf, n * 3 * sizeof(float), hipMemcpyDeviceToHost, cx.stream));
+            cx.copier.to_host(rgb_planes, pic->out_rgbf, n * 3 * sizeof(float), cx.stream);
         ZJAI_HIP(hipStreamSynchronize(cx.stream));
     });
 }
@@ -1349,7 +1347,7 @@ extern "C" int32_t zjai_hyper_decoder_forward(zjai_ctx* ctx, const zjai_net* net
         const size_t zn = (size_t)c * zh * zw;
         void* zdev = cx.pool.alloc(zn);
         std::shared_ptr<void> keep(zdev, [&cx](void* q) { cx.pool.release(q); });
-        ZJAI_HIP(hipMemcpyAsync(zdev, z_hat, zn, hipMemcpyHostToDevice, cx.stream));
+        cx.copier.to_device(zdev, z_hat, zn, cx.stream);
         TensorP z = cx.alloc(1, c, zh, zw, m.dtype);
         {
             LaunchScope sc(cx, kname("k_i8_planar_to_nhwc", m.dtype), 0.0, (1.0 + dtype_size(m.dtype)) * zn);
@@ -1364,7 +1362,7 @@ extern "C" int32_t zjai_hyper_decoder_forward(zjai_ctx* ctx, const zjai_net* net
             LaunchScope sc(cx, kname("k_nhwc_to_planar", m.dtype), 0.0, (4.0 + dtype_size(m.dtype)) * pn);
             ZJAI_HIP(launch_nhwc_to_planar(t->v, m.dtype, 1, 4 * c, out_h, out_w, dev, cx.stream));
         }
-        ZJAI_HIP(hipMemcpyAsync(psi, dev, pn * 4, hipMemcpyDeviceToHost, cx.stream));
+        cx.copier.to_host(psi, dev, pn * 4, cx.stream);
         ZJAI_HIP(hipStreamSynchronize(cx.stream));
     });
 }
@@ -1385,9 +1383,9 @@ extern "C" int32_t zjai_context_decompress(zjai_ctx* ctx, const zjai_net* net, c
         std::shared_ptr<void> keep(rdev, [&cx](void* q) { cx.pool.release(q); });
         float* ydev = (float*)cx.pool.alloc(rn * 4);
         std::shared_ptr<void> keep2(ydev, [&cx](void* q) { cx.pool.release(q); });
-        ZJAI_HIP(hipMemcpyAsync(rdev, residual, rn * 4, hipMemcpyHostToDevice, cx.stream));
+        cx.copier.to_device(rdev, residual, rn * 4, cx.stream);
         latent_decompress(cx, m, rdev, w, (long long)h * w, Windows{}, h, w, ps, ydev);
-        ZJAI_HIP(hipMemcpyAsync(y_hat, ydev, rn * 4, hipMemcpyDeviceToHost, cx.stream));
+        cx.copier.to_host(y_hat, ydev, rn * 4, cx.stream);
         ZJAI_HIP(hipStreamSynchronize(cx.stream));
     });
 }
@@ -1685,7 +1683,7 @@ extern "C" int32_t zjai_analysis_forward(zjai_ctx* ctx, const zjai_net* net, con
         const size_t xn = (size_t)c * h * w;
         float* xdev = (float*)cx.pool.alloc(xn * 4);
         std::shared_ptr<void> keep(xdev, [&cx](void* q) { cx.pool.release(q); });
-        ZJAI_HIP(hipMemcpyAsync(xdev, x, xn * 4, hipMemcpyHostToDevice, cx.stream));
+        cx.copier.to_device(xdev, x, xn * 4, cx.stream);
         TensorP t = analysis_forward(cx, m, xdev, h, w, clip != 0);
         float* dev = (float*)cx.pool.alloc(yn * 4);
         std::shared_ptr<void> keep2(dev, [&cx](void* q) { cx.pool.release(q); });
@@ -1693,7 +1691,7 @@ extern "C" int32_t zjai_analysis_forward(zjai_ctx* ctx, const zjai_net* net, con
             LaunchScope sc(cx, kname("k_nhwc_to_planar", m.dtype), 0.0, (4.0 + dtype_size(m.dtype)) * yn);
             ZJAI_HIP(launch_nhwc_to_planar(t->v, m.dtype, 1, m.chs, t->h, t->w, dev, cx.stream));
         }
-        ZJAI_HIP(hipMemcpyAsync(y, dev, yn * 4, hipMemcpyDeviceToHost, cx.stream));
+        cx.copier.to_host(y, dev, yn * 4, cx.stream);
         ZJAI_HIP(hipStreamSynchronize(cx.stream));
     });
 }

@@ -117,8 +117,17 @@ void reconstruct_latent(Context& ctx, const Net& net, int height, int width, con
     const size_t zn = (size_t)C * zh * zw, rn = (size_t)C * H * W, pn = (size_t)4 * C * ph * pw;
 
     DevBuf zdev(ctx, zn), rdev(ctx, rn * 4), psi(ctx, pn * 4), yhat(ctx, rn * 4);
-    ZJAI_HIP(hipMemcpyAsync(zdev.p, z_hat, zn, hipMemcpyHostToDevice, ctx.stream));
-    ZJAI_HIP(hipMemcpyAsync(rdev.p, residual, rn * 4, hipMemcpyHostToDevice, ctx.stream));
+    // The residual's upload runs beside the hyper-decoder and psi's download beside the context
+    // model, on the copier's stream `side` (a pageable copy holds this thread, not the kernels
+    // already launched). No buffer goes back to the pool while a copy of it is under way.
+    HostCopier& copier = ctx.top().copier;
+    const hipStream_t side = copier.side_stream();
+    std::shared_ptr<void> settle(&copier, [&](void*) {
+        (void)hipStreamSynchronize(side);
+        (void)hipStreamSynchronize(ctx.stream);
+    });
+    copier.to_device(zdev.p, z_hat, zn, ctx.stream);
+    copier.order(ctx.stream, side);
     ZJAI_HIP(launch_zero(psi.p, pn * 4, ctx.stream));
     ZJAI_HIP(launch_zero(yhat.p, rn * 4, ctx.stream));
 
@@ -192,6 +201,10 @@ void reconstruct_latent(Context& ctx, const Net& net, int height, int width, con
                                          pw, core.y, core.x, ctx.stream));
     }
     psi_of.clear();
+    // psi is final here. (The wait is placed behind the upload: `side` runs in order.)
+    copier.to_device(rdev.p, residual, rn * 4, side);
+    copier.order(side, ctx.stream);
+    copier.order(ctx.stream, side);
 
     // 2. y_hat per region (context model on the region's residual and psi windows), merged in
     // raster order: independent regions keep their whole latent area, dependent ones drop one
@@ -251,8 +264,9 @@ void reconstruct_latent(Context& ctx, const Net& net, int height, int width, con
         ZJAI_HIP(launch_assign_planar(src, C, lt.h, lt.w, oy, ox, h, w, yhat.as<float>(), H, W, core.y, core.x,
                                       ctx.stream));
     }
-    ZJAI_HIP(hipMemcpyAsync(psi_out, psi.p, pn * 4, hipMemcpyDeviceToHost, ctx.stream));
-    ZJAI_HIP(hipMemcpyAsync(y_out, yhat.p, rn * 4, hipMemcpyDeviceToHost, ctx.stream));
+    copier.to_host(psi_out, psi.p, pn * 4, side);
+    copier.to_host(y_out, yhat.p, rn * 4, ctx.stream);
+    ZJAI_HIP(hipStreamSynchronize(side));
     ZJAI_HIP(hipStreamSynchronize(ctx.stream));
 }
 

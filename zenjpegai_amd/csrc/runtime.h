@@ -13,6 +13,7 @@
 
 #include "conv.h"
 #include "error.h"
+#include "hostcopy.h"
 #include "ops.h"
 #include "../../include/zjai_hip.h"
 
@@ -128,6 +129,7 @@ struct Context {
     Context* root = nullptr;
     bool owns_stream = false;
     std::vector<std::unique_ptr<Context>> lanes;
+    HostCopier copier;  // the root context's: transfers run on the caller's thread
     Context& lane(int i);
     Context& top() { return root ? *root : *this; }
 
