@@ -471,6 +471,29 @@ def test_narrow_conv_transpose_is_bit_exact(engines, cout, k, op):
     assert np.array_equal(y6, oracle.conv_transpose2d(oracle.relu6(x), w, b, 2, 1, op))
 
 
+# 8 x 8-position tiles: single positions, a tile's edges and one more, several tiles; one to four
+# 32-channel chunks; every output count of the waves' pairs.
+@pytest.mark.parametrize("cin,cout,op,h,w", [(32, 5, 0, 1, 1), (64, 8, 1, 8, 8), (64, 7, 1, 9, 17),
+                                             (96, 6, 0, 7, 40), (128, 8, 1, 33, 5), (48, 8, 1, 9, 9)])
+def test_narrow_conv_transpose_3x3_f32_wide_is_bit_exact(engines, cin, cout, op, h, w):
+    """Five to eight outputs in f32: k_convT3_narrow8 where the channels come in whole 32s, the
+    generic kernel otherwise; both run the oracle's FMA chain, so every bit agrees."""
+    eng = engines["f32"]
+    x = synth.normal(12, "t8/x", (cin, h, w), 1.0)
+    wt = synth.normal(12, "t8/w", (cin, cout, 3, 3), 0.1)
+    b = synth.normal(12, "t8/b", (cout,), 0.1)
+    layer = nn.ConvTransposeLayer(nn.ConvTranspose2d(cin, cout, 3, 2, 1, op, wt, b), eng)
+    xt = nn.BTensor.from_planar(eng, x)
+    eng.sync()
+    eng.profile_begin()
+    y = layer.forward(eng, xt).to_planar()
+    names = [r[0] for r in eng.profile_end()]
+    assert ("k_convT3_narrow8" in names) == (cin % 32 == 0), names
+    assert np.array_equal(y, oracle.conv_transpose2d(x, wt, b, 2, 1, op))
+    y6 = layer.forward_fused(eng, xt, relu6_input=True).to_planar()
+    assert np.array_equal(y6, oracle.conv_transpose2d(oracle.relu6(x), wt, b, 2, 1, op))
+
+
 def _round_storage(a, prec):
     """IEEE round-to-nearest-even of f32 values to the 16-bit storage type, back in f32."""
     a = np.ascontiguousarray(a, np.float32)

@@ -106,10 +106,13 @@ bool conv1x1_ring_ok(const ConvParams& p, int dtype);
 int conv1x1_ring_nb(const ConvParams& p);
 
 // Stride-2 transposed conv with cout <= 8 on the vector ALUs (coutp = cout rounded up to 1, 2, 4
-// or 8); wn is [cin][phase][tap][coutp] f32. Uses p's input view, output geometry, tap tables,
+// or 8); wn is [cin][phase][tap][coutp] f32, for f32 3x3 layers of 5 to 8 outputs and cin % 32 = 0
+// followed by [coutp / 2][cin][9 taps][2] (a tap's place: phase by phase). Uses p's input view, output geometry, tap tables,
 // bias and epilogue fields.
 // convT_narrow_k3: whether launch_convT_narrow takes the 3x3 / padding-1 kernel for p.
+// convT_narrow8_k3: whether it takes the one for 5 to 8 f32 outputs.
 bool convT_narrow_k3(int dtype, const ConvParams& p, int cin);
+bool convT_narrow8_k3(int dtype, const ConvParams& p, int cin);
 hipError_t launch_convT_narrow(int dtype, int coutp, const ConvParams& p, const float* wn, int cin,
                                hipStream_t s);
 // The same layers in f16 / bf16 on 16x16x32 MFMAs when their taps are the 3x3 / padding-1 ones

@@ -787,6 +787,134 @@ k_convT3_narrow(const ConvParams p, const float* __restrict__ wn, int cin) {
     }
 }
 
+// The same layer in f32 with 5 to 8 outputs (HOP chroma 64 -> 8), the outputs split over the waves:
+// a workgroup takes 8 x 8 positions, wave w outputs 2 w and 2 w + 1 of all of them, so a wave's 18
+// weights per input channel are uniform and contiguous (wg: [cin] x 18 per wave, scalar loads) and a
+// thread keeps 8 accumulators. The 9 x 9-pixel halo goes through LDS 32 channels at a time by direct
+// loads, two chunks deep: both of a 64-channel layer's chunks, i.e. all of its input, fly at once, in
+// 21 KB. The generic kernel stages 64 x 4 positions in serial 16-channel rounds, each waiting for its
+// loads, and runs all 32 accumulators per thread from LDS weights; on a small map its few workgroups
+// walk those rounds alone. FMA order per output is the generic kernel's, bit for bit. Bound by the
+// vector ALUs (9 FMAs per position, input channel and output) on a large map, by the scalar weight
+// loads of its 16 rounds on a small one. 64 -> 8 in a 203 x 301 picture 71.5 -> 22.9 us; in the
+// batches of a 4K picture, beside three other lanes, 167 -> 85 us a launch.
+__global__ void __launch_bounds__(256)
+k_convT3_narrow8(const ConvParams p, const float* __restrict__ wg, int cin) {
+    constexpr int TB = 8, HX = TB + 1, HPIX = HX * HX, CPU = 8;
+    constexpr int HALO_U = HPIX * CPU;  // 16-byte units of a chunk: [pixel][CPU swizzled slots]
+    constexpr int HN = (HALO_U + 255) / 256;
+    __shared__ u32x4 s_halo[2 * HALO_U];
+    const int gw = (p.OW + 1) / 2, gh = (p.OH + 1) / 2;
+    const int gx = (gw + TB - 1) / TB, gy = (gh + TB - 1) / TB;
+    // XCD-aware order (k_convT_narrow's): each XCD takes one contiguous band of tiles.
+    int bid = (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
+    if (bid >= gx * gy * p.N) return;
+    const int tx = bid % gx;
+    bid /= gx;
+    const int ty = bid % gy, bi = bid / gy;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane >> 3, c = lane & 7;
+    const int y0 = ty * TB, x0 = tx * TB;
+    const float* xg = (const float*)p.x.p + (long long)bi * p.x.bstride + p.x.c_off;
+
+    float acc[4][2];
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+        const float b = (p.bias && 2 * wave + o < p.cout_g) ? p.bias[2 * wave + o] : 0.0f;
+#pragma unroll
+        for (int ph = 0; ph < 4; ++ph) acc[ph][o] = b;
+    }
+
+    // Slot s of pixel (hy, hx) holds the pixel's 16-byte unit s ^ key(hy, hx). A ds_read_b128 pass
+    // reads 4 neighbouring columns of each of 4 rows: pixels of one parity (one half of the banks)
+    // then differ in their key, for any first row and column.
+    auto key = [](int hy, int hx) { return ((hx >> 1) & 3) | ((hy & 1) << 2); };
+    long long hoff[HN];
+#pragma unroll
+    for (int i = 0; i < HN; ++i) {
+        const int U = tid + i * 256, pix = U >> 3, slot = U & 7;
+        const int hy = pix / HX, hx = pix - hy * HX;
+        const int iy = y0 + hy, ix = x0 + hx;
+        hoff[i] = (U < HALO_U && iy < p.H && ix < p.W)
+                      ? (long long)iy * p.x.row + (long long)ix * p.x.cs + (slot ^ key(hy, hx)) * 4
+                      : -1;
+    }
+    auto issue = [&](int chunk) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < HN; ++i) {
+            const int ub = wave * 64 + i * 256;
+            if (ub >= HALO_U) break;
+            if (ub + lane < HALO_U) {
+                const void* src = hoff[i] >= 0 ? (const void*)(xg + hoff[i] + chunk * 32) : (const void*)g_zero_unitsT;
+                lds_dma16(src, s_halo + (chunk & 1) * HALO_U + ub);
+            }
+        }
+    };
+    int nbase[4], nkey[4];  // neighbours (y' + a, x' + b), index 2a + b
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        const int hy = r + (n >> 1), hx = c + (n & 1);
+        nbase[n] = (hy * HX + hx) * CPU;
+        nkey[n] = key(hy, hx);
+    }
+
+    const int nch = cin / 32;
+    const float* wp = wg + (long long)wave * cin * 18;
+    issue(0);
+    if (nch > 1) issue(1);
+    for (int ch = 0; ch < nch; ++ch) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads are in LDS
+        __syncthreads();                     // ... and every other wave's
+        const u32x4* hb = s_halo + (ch & 1) * HALO_U;
+#pragma unroll 1
+        for (int q = 0; q < CPU; ++q) {
+            float x[4][4];
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                unpack16<float>(hb[nbase[n] + (q ^ nkey[n])], x[n]);
+                if (p.relu6_in) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float e = x[n][i];
+                        e = e < 0.0f ? 0.0f : e;
+                        x[n][i] = e > 6.0f ? 6.0f : e;
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i, wp += 18) {
+                // Taps as in k_convT3_narrow, two outputs each.
+#pragma unroll
+                for (int o = 0; o < 2; ++o) {
+                    acc[0][o] = fmaf(wp[0 + o], x[0][i], acc[0][o]);
+                    acc[1][o] = fmaf(wp[2 + o], x[1][i], acc[1][o]);
+                    acc[1][o] = fmaf(wp[4 + o], x[0][i], acc[1][o]);
+                    acc[2][o] = fmaf(wp[6 + o], x[2][i], acc[2][o]);
+                    acc[2][o] = fmaf(wp[8 + o], x[0][i], acc[2][o]);
+                    acc[3][o] = fmaf(wp[10 + o], x[3][i], acc[3][o]);
+                    acc[3][o] = fmaf(wp[12 + o], x[2][i], acc[3][o]);
+                    acc[3][o] = fmaf(wp[14 + o], x[1][i], acc[3][o]);
+                    acc[3][o] = fmaf(wp[16 + o], x[0][i], acc[3][o]);
+                }
+            }
+        }
+        if (ch + 2 < nch) {
+            __syncthreads();  // every wave is done with this chunk's buffer
+            issue(ch + 2);
+        }
+    }
+    if (2 * wave >= p.cout_g) return;
+    const int yq = y0 + r, xq = x0 + c;
+#pragma unroll
+    for (int ph = 0; ph < 4; ++ph) {
+        const int oy = 2 * yq + (ph >> 1), ox = 2 * xq + (ph & 1);
+        if (oy >= p.OH || ox >= p.OW) continue;
+        epilogue_store<float>(p, bi, oy, ox, 2 * wave, min(2, p.cout_g - 2 * wave),
+                              f32x4{acc[ph][0], acc[ph][1], 0.0f, 0.0f});
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // 16-bit 3x3 stride-2 transposed convs with at most 8 outputs and 64 or 128 input channels (the
 // last synthesis layers: HOP luma 128 -> 1, HOP chroma 64 -> 8) on the matrix cores. Output phase
@@ -969,6 +1097,12 @@ bool convT_narrow_k3(int dtype, const ConvParams& p, int cin) {
            p.x.c_off % vec == 0 && p.x.row % vec == 0 && p.x.bstride % vec == 0;
 }
 
+// Five to eight f32 outputs: k_convT3_narrow8, on any map (16-bit nets take k_convT3_mfma).
+bool convT_narrow8_k3(int dtype, const ConvParams& p, int cin) {
+    return dtype == DT_F32 && p.cout_g > 4 && p.cout_g <= 8 && taps_are_k3p1(p) && cin % 32 == 0 &&
+           p.x.cs % 4 == 0 && p.x.c_off % 4 == 0 && p.x.row % 4 == 0 && p.x.bstride % 4 == 0;
+}
+
 bool convT_mfma_k3(int dtype, const ConvParams& p, int cin) {
     return dtype != DT_F32 && taps_are_k3p1(p) && (cin == 64 || cin == 128) && p.x.cs % 8 == 0 &&
            p.x.c_off % 8 == 0 && p.x.row % 8 == 0 && p.x.bstride % 8 == 0;
@@ -1024,6 +1158,14 @@ static hipError_t go_narrow(int coutp, const ConvParams& p, const float* wn, int
 
 hipError_t launch_convT_narrow(int dtype, int coutp, const ConvParams& p, const float* wn, int cin,
                                hipStream_t s) {
+    if (convT_narrow8_k3(dtype, p, cin)) {
+        const int gw = (p.OW + 1) / 2, gh = (p.OH + 1) / 2;
+        const long long blocks = ((long long)((gw + 7) / 8) * ((gh + 7) / 8) * p.N + 7) / 8 * 8;
+        if (blocks <= 0 || blocks > (1ll << 30) || p.N < 1 || p.N > MAXB || coutp != 8) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(k_convT3_narrow8, dim3((unsigned)blocks), dim3(256), 0, s, p,
+                           wn + (size_t)16 * cin * coutp, cin);
+        return hipGetLastError();
+    }
     if (convT_narrow_k3(dtype, p, cin)) {
         switch (dtype) {
             case DT_F32: return go_narrow3<float>(coutp, p, wn, cin, s);

@@ -549,6 +549,14 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
                                 storage_value(weight[(((size_t)ic * cout + oc) * k + ky) * k + kx], dtype);
                 }
         }
+        if (dtype == DT_F32 && k == 3 && L->coutp == 8 && cin % 32 == 0) {  // k_convT3_narrow8's order
+            for (int pair = 0; pair < 4; ++pair)
+                for (int ic = 0; ic < cin; ++ic)
+                    for (int ph = 0; ph < 4; ++ph)
+                        for (int t = 0; t < nky[ph >> 1] * nky[ph & 1]; ++t)
+                            for (int o = 0; o < 2; ++o)
+                                wn.push_back(wn[((size_t)ic * 16 + ph * 4 + t) * 8 + 2 * pair + o]);
+        }
         L->wn = upload_f32(wn.data(), wn.size(), &L->dev_bytes);
         if (dtype != DT_F32 && k == 3 && (cin == 64 || cin == 128)) {
             // The MFMA form (launch_convT3_mfma): row R = phase * coutp + output of 16-row block
@@ -817,8 +825,9 @@ static TensorP conv_forward_impl(Context& ctx, const Layer& L, const TensorP& x,
     if (L.wn && !e.w_batch) {
         static const char* ty[] = {"float", "_Float16", "__bf16"};
         char name[64];
-        snprintf(name, sizeof name, "%s<%s, %d>", convT_narrow_k3(L.dtype, p, L.cin) ? "k_convT3_narrow" : "k_convT_narrow",
-                 ty[L.dtype], L.coutp);
+        if (convT_narrow8_k3(L.dtype, p, L.cin)) snprintf(name, sizeof name, "k_convT3_narrow8");
+        else snprintf(name, sizeof name, "%s<%s, %d>", convT_narrow_k3(L.dtype, p, L.cin) ? "k_convT3_narrow" : "k_convT_narrow",
+                      ty[L.dtype], L.coutp);
         LaunchScope sc(ctx, name, 2.0 * macs, bytes);
         ZJAI_HIP(launch_convT_narrow(L.dtype, L.coutp, p, L.wn, L.cin, ctx.stream));
         return y;
