@@ -730,6 +730,11 @@ k_convT3_narrow(const ConvParams p, const float* __restrict__ wn, int cin) {
 
     const int nch = cin / (CPU * VEC);
     issue(0, 0);
+    // Every 128-byte line of the weights touched once, beside the first halo (as k_convT3_narrow8):
+    // 128 -> 1 in a 203 x 301 picture 36.8 -> 23.7 us.
+    unsigned warm = 0;
+    for (int u = tid * 32; u < cin * 16 * COUT; u += 256 * 32) warm |= *(const unsigned*)(wn + u);
+    asm volatile("" : : "v"(warm));
     for (int ch = 0; ch < nch; ++ch) {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads of chunk ch are in LDS
         __syncthreads();                     // ... and every other wave's
@@ -796,7 +801,8 @@ k_convT3_narrow(const ConvParams p, const float* __restrict__ wn, int cin) {
 // loads, and runs all 32 accumulators per thread from LDS weights; on a small map its few workgroups
 // walk those rounds alone. FMA order per output is the generic kernel's, bit for bit. Bound by the
 // vector ALUs (9 FMAs per position, input channel and output) on a large map, by the scalar weight
-// loads of its 16 rounds on a small one. 64 -> 8 in a 203 x 301 picture 71.5 -> 22.9 us; in the
+// loads of its 16 rounds on a small one. 64 -> 8 in a 203 x 301 picture 71.5 -> 22.9 us, 16.2 with the
+// weight lines touched beside the halo; in the
 // batches of a 4K picture, beside three other lanes, 167 -> 85 us a launch.
 __global__ void __launch_bounds__(256)
 k_convT3_narrow8(const ConvParams p, const float* __restrict__ wg, int cin) {
@@ -863,6 +869,11 @@ k_convT3_narrow8(const ConvParams p, const float* __restrict__ wg, int cin) {
     const float* wp = wg + (long long)wave * cin * 18;
     issue(0);
     if (nch > 1) issue(1);
+    // The scalar loads below would each miss L2 in turn on a workgroup's first pass: every 128-byte
+    // line of the weights is touched here, together with the halo (one word a thread).
+    unsigned warm = 0;
+    for (int u = tid * 32; u < cin * 72; u += 256 * 32) warm |= *(const unsigned*)(wg + u);
+    asm volatile("" : : "v"(warm));
     for (int ch = 0; ch < nch; ++ch) {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads are in LDS
         __syncthreads();                     // ... and every other wave's

@@ -663,8 +663,8 @@ __global__ void __launch_bounds__(FTHREADS) k_qkv(const QkvArgs p) {
 // c), and every wave computes all channels of a slice for its 32 positions. The weights of each
 // slice arrive by direct global -> LDS loads issued one phase ahead. The arithmetic is the f32
 // unfused kernels' instruction for instruction: LayerNorm as k_layer_norm (f64 sums in channel
-// order per position), the 1x1 convs as conv1x1_ring (bias, then v_mfma_f32_16x16x4_f32 over K
-// chunks of 16 channels in ascending order), the depthwise 3x3 and gate as k_depthwise3x3, so the
+// order per position), the 1x1 convs as conv1x1_ring_split (bias, then mma_split32 over pairs
+// of 16-channel K chunks in ascending order), the depthwise 3x3 and gate as k_depthwise3x3, so the
 // fused and unfused f32 paths agree bit for bit.
 
 namespace {

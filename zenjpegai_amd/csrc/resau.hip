@@ -10,7 +10,7 @@
 //      with the pixel index so that 16 consecutive pixels' same unit hits different banks);
 //   2. wave w computes t for group w % G (G = C / 16) and rows (w / G) * NPW .. : per output,
 //      bias-free, the 9 taps in (ky, kx) order, one K chunk of 16 channels (f32:
-//      4 x v_mfma_f32_16x16x4_f32; f16 / bf16: one 16x16x32 MFMA whose upper 16 K lanes are the
+//      the piece products of mma_split; f16 / bf16: one 16x16x32 MFMA whose upper 16 K lanes are the
 //      zero padding the unfused kernel also multiplies) -- conv_igemm's instruction sequence for
 //      this layer; t is rounded to the storage type into LDS, as the unfused kernel stores it;
 //   3. the 1x1 over t for output block w % G on the same rows: K chunks in ascending order, the
