@@ -43,7 +43,7 @@ extern "C" {
 #define ZJAI_E_DEVICE (-6)           /* HIP runtime / device failure */
 
 /* Precision of a layer / net: storage type of weights and activations. Accumulation is f32. */
-#define ZJAI_F32 0  /* fp32 MFMA parity path */
+#define ZJAI_F32 0  /* fp32 parity path */
 #define ZJAI_F16 1  /* f16 inputs, fp32 accumulate */
 #define ZJAI_BF16 2 /* bf16 inputs, fp32 accumulate */
 
