@@ -240,11 +240,10 @@ ZJAI_API int32_t zjai_channel_attention(zjai_ctx* ctx, const zjai_tensor* qkv, i
  * out are caller-owned device buffers, 16-byte aligned, NHWC dense in `precision`: qkv
  * [h][w][channels] (channels = 3 * dim: q, k, v), out [h][w][dim]; temperature is a device array
  * of `heads` floats. The work is enqueued on the context's stream (zjai_sync waits for it) and
- * allocates nothing: its scratch (Gram partial sums, attention matrix, folded weight) is one
- * static device array of ZJAI_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends and
- * shared by every call on that GPU, so calls that overlap on one GPU (contexts on different
- * streams) race. A map that needs more scratch (with dim 128 and 4 heads: more than ~240k
- * positions) returns ZJAI_E_LIMIT before anything is launched. */
+ * allocates nothing: its scratch (Gram partial sums, attention matrix, folded weight) is an array
+ * of ZJAI_NOALLOC_SCRATCH_BYTES (and 1 MiB beside it) that zjai_ctx_create allocates for the
+ * context, so calls on several contexts may overlap on one GPU. A map that needs more scratch (with
+ * dim 128 and 4 heads: more than ~240k positions) returns ZJAI_E_LIMIT before anything is launched. */
 #define ZJAI_NOALLOC_SCRATCH_BYTES (16u << 20)
 ZJAI_API int32_t zjai_channel_attention_noalloc(zjai_ctx* ctx, const void* qkv, int32_t channels,
                                                 int32_t h, int32_t w, int32_t heads,

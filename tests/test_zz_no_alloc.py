@@ -1,8 +1,9 @@
 """GPU: the allocation-free entry point ``zjai_channel_attention_noalloc`` against
 ``zjai_channel_attention`` (src/nn/fast/math.rs:512-603), through the C-ABI, bit for bit: two
-calls in a row with the second on a smaller map (the shared scratch then holds the first call's
-larger contents), in f32, f16 and bf16, dims 128 and 64 and a dim of 8 whose folded weight has
-padded rows and columns. A map beyond the scratch returns LimitExceeded before any launch.
+calls in a row with the second on a smaller map (the scratch then holds the first call's larger
+contents), in f32, f16 and bf16, dims 128 and 64 and a dim of 8 whose folded weight has
+padded rows and columns; and calls of several contexts in flight together, each with its own
+result. A map beyond the scratch returns LimitExceeded before any launch.
 
 The caller-owned device buffers come from the HIP runtime the library itself links
 (libamdhip64.so.7, via ctypes)."""
@@ -105,6 +106,45 @@ def test_noalloc_attention_equals_the_allocating_entry_point(prec, dim, heads):
         assert np.isfinite(want).all()
         assert np.array_equal(got, want), (prec, dim, h, w, float(np.max(np.abs(got - want))))
     eng.close()
+
+
+@pytest.mark.parametrize("prec", ["f32", "f16", "bf16"])
+def test_noalloc_attention_of_several_contexts_in_flight_together(prec):
+    """Nothing orders the streams of two contexts, so their calls overlap: each must keep its
+    scratch to itself. q = +-k by head, so that the attention matrix of another context's map (other
+    signs) would change every output."""
+    hip = _hip()
+    dim, heads, h, w = 128, 4, 64, 80
+    es = 4 if prec == "f32" else 2
+    engs = [nn.Engine(0, prec) for _ in range(3)]
+    bufs, calls, want = [], [], []
+    try:
+        for i, eng in enumerate(engs):
+            x = synth.normal(40 + i, "noalloc/ctx", (3 * dim, h, w), 1.0)
+            x[:dim] = x[dim:2 * dim] * np.where(np.arange(dim) // 32 == i, -1.0, 1.0).astype(np.float32)[:, None, None]
+            x, raw = _storage_exact(x, prec)
+            temp = np.full(heads, 2.0, np.float32)
+            want.append(nn.channel_attention(eng, nn.BTensor.from_planar(eng, x), heads, temp).to_planar())
+            q, t, o = DevBuf(hip, 3 * dim * h * w * es), DevBuf(hip, heads * 4), DevBuf(hip, dim * h * w * es)
+            bufs += [q, t, o]
+            q.put(np.ascontiguousarray(raw.transpose(1, 2, 0)))
+            t.put(temp)
+            calls.append((eng, q, t, o))
+        assert hip.hipDeviceSynchronize() == 0
+        for _ in range(20):
+            for _ in range(3):  # three rounds of calls that nothing waits between
+                for eng, q, t, o in calls:
+                    assert _lib.lib().zjai_channel_attention_noalloc(eng.handle, q.p, 3 * dim, h, w, heads, t.p,
+                                                                     _lib.PRECISIONS[prec], o.p) == _lib.OK
+            assert hip.hipDeviceSynchronize() == 0
+            for (_, _, _, o), y in zip(calls, want):
+                dt = np.float32 if prec == "f32" else np.float16 if prec == "f16" else np.uint16
+                np.testing.assert_array_equal(_to_f32(o.get(dt, (h, w, dim)), prec).transpose(2, 0, 1), y)
+    finally:
+        for b in bufs:
+            b.free()
+        for eng in engs:
+            eng.close()
 
 
 def test_noalloc_attention_rejects_a_map_beyond_the_scratch():

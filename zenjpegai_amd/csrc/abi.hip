@@ -77,41 +77,13 @@ TensorP planar_upload(Context& c, const float* data, int ch, int h, int w, int d
 
 }  // namespace
 
-// ---------------------------------------------------------------- allocation-free scratch
-// Scratch of zjai_channel_attention_noalloc: each GPU holds its own copy of this array until the
-// process ends. In host code `scratch` is a host-side stand-in, not device memory: the array's
-// address on a device comes from hipGetSymbolAddress (scratch_setup, called by zjai_ctx_create
-// with that device current) and only that address is passed to kernels.
-// The bytes past ZJAI_NOALLOC_SCRATCH_BYTES hold the third bf16 piece of an f32 call's folded
-// weight (half its f32 size; dim <= 639 by the Gram kernel's LDS stage), so that maps up to the
-// documented size fit as they do in f32 form.
-constexpr size_t SCRATCH_PIECE_BYTES = 1u << 20;
-static __device__ __align__(256) unsigned char scratch[ZJAI_NOALLOC_SCRATCH_BYTES + SCRATCH_PIECE_BYTES];
-
-namespace {
-
-constexpr int SCRATCH_DEVICES = 64;
-std::mutex g_scratch_mu;
-void* g_scratch_dev[SCRATCH_DEVICES] = {};
-
-void scratch_setup(int device) {
-    std::lock_guard<std::mutex> g(g_scratch_mu);
-    if (device < 0 || device >= SCRATCH_DEVICES) throw Error(ZJAI_E_UNSUPPORTED, "device index beyond the scratch table");
-    if (g_scratch_dev[device]) return;
-    void* p = nullptr;
-    ZJAI_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-    if (!p) throw Error(ZJAI_E_DEVICE, "hipGetSymbolAddress: no address for the scratch array");
-    g_scratch_dev[device] = p;
-}
-
-unsigned char* scratch_of(int device) {
-    std::lock_guard<std::mutex> g(g_scratch_mu);
-    return device >= 0 && device < SCRATCH_DEVICES ? (unsigned char*)g_scratch_dev[device] : nullptr;
-}
-
-size_t round_up256(size_t n) { return (n + 255) / 256 * 256; }
-
-}  // namespace
+// Scratch of zjai_channel_attention_noalloc, one per context: every launch of a call runs on the
+// context's stream, so calls on one context follow each other, and calls on several contexts (whose
+// streams nothing orders) share nothing. The bytes past ZJAI_NOALLOC_SCRATCH_BYTES hold the third
+// bf16 piece of an f32 call's folded weight (half its f32 size; dim <= 639 by the Gram kernel's LDS
+// stage), so that maps up to the documented size fit as they do in f32 form.
+static constexpr size_t SCRATCH_PIECE_BYTES = 1u << 20;
+static size_t round_up256(size_t n) { return (n + 255) / 256 * 256; }
 
 // ------------------------------------------------------------------------------- context
 extern "C" int32_t zjai_ctx_create(int32_t device, uint32_t flags, zjai_ctx** out) {
@@ -133,16 +105,16 @@ extern "C" int32_t zjai_ctx_create(int32_t device, uint32_t flags, zjai_ctx** ou
         if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0)
             throw Error(ZJAI_E_UNSUPPORTED, std::string("kernels are built for gfx950, device is ") + prop.gcnArchName);
         ZJAI_HIP(hipSetDevice(device));
-        scratch_setup(device);
         ctx->c.device = device;
         ctx->c.flags = flags;
         ZJAI_HIP(hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking));
         ZJAI_HIP(hipEventCreate(&ctx->c.ev0));
         ZJAI_HIP(hipEventCreate(&ctx->c.ev1));
+        ZJAI_HIP(hipMalloc(&ctx->c.attention_scratch, ZJAI_NOALLOC_SCRATCH_BYTES + SCRATCH_PIECE_BYTES));
         ctx->c.copier.create();
     });
     if (rc != ZJAI_OK) {
-        delete ctx;
+        (void)zjai_ctx_destroy(ctx);
         return rc;
     }
     *out = ctx;
@@ -505,8 +477,7 @@ extern "C" int32_t zjai_channel_attention_noalloc(zjai_ctx* ctx, const void* qkv
         const size_t attn_off = round_up256(part_bytes), w_off = round_up256(attn_off + (size_t)dim * c * 4);
         if (w_off + w_plain > ZJAI_NOALLOC_SCRATCH_BYTES || w_bytes - w_plain > SCRATCH_PIECE_BYTES)
             throw Error(ZJAI_E_LIMIT, "attention: the map needs more than the allocation-free scratch");
-        unsigned char* base = scratch_of(ctx->c.device);
-        if (!base) throw Error(ZJAI_E_DEVICE, "allocation-free scratch not set up for this device");
+        unsigned char* base = (unsigned char*)ctx->c.attention_scratch;
         float* partial = (float*)base;
         float* attn = (float*)(base + attn_off);
         void* wfold = base + w_off;

@@ -113,6 +113,7 @@ struct Context {
     std::string last_error;
     volatile int stop = 0;
     uint64_t mem_limit = 0;  // zjai_ctx_set_memory_limit: device bytes a picture may need (0: none)
+    void* attention_scratch = nullptr;  // zjai_channel_attention_noalloc's (root context)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.0f;
     long long launches = 0;

@@ -136,6 +136,7 @@ Context::~Context() {
     }
     for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
     if (range_slots) (void)hipFree(range_slots);
+    if (attention_scratch) (void)hipFree(attention_scratch);
 }
 
 void range_slots_init(Context& ctx) {
