@@ -157,7 +157,7 @@ typedef struct zjai_prof_record {
 ZJAI_API int32_t zjai_profile_begin(zjai_ctx* ctx);
 ZJAI_API int32_t zjai_profile_end(zjai_ctx* ctx, zjai_prof_record* out, int32_t cap, int32_t* n);
 /* Returns cached pool blocks to the device (`release_buffers`, src/nn/fast/tensor.rs:122), the
- * lanes' included, and starts a new pool_peak. The pool figures of zjai_get_stats cover the
+ * lanes' included, and the buffer that f32 weights of new layers go through, and starts a new pool_peak. The pool figures of zjai_get_stats cover the
  * context's own pool and every lane's (pool_peak: the sum of the pools' high-water marks). */
 ZJAI_API int32_t zjai_release_buffers(zjai_ctx* ctx);
 

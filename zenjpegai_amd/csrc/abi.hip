@@ -220,6 +220,7 @@ extern "C" int32_t zjai_release_buffers(zjai_ctx* ctx) {
         ZJAI_HIP(hipStreamSynchronize(ctx->c.stream));
         ctx->c.pool.trim();
         ctx->c.pool.reset_peak();
+        ctx->c.release_weight_stage();
         for (const auto& l : ctx->c.lanes) {
             ZJAI_HIP(hipStreamSynchronize(l->stream));
             l->pool.trim();

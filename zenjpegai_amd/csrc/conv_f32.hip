@@ -653,6 +653,23 @@ conv1x1_ring_split(const ConvParams p) {
     }
 }
 
+// Weight blocks [16 outputs][16 channels] to split blocks (split.h), a lane's four channels per
+// thread.
+__global__ void __launch_bounds__(256) k_split_weights(const float* src, u32x4* dst, long long nblk) {
+    const long long t = (long long)blockIdx.x * 256 + threadIdx.x, b = t >> 6;
+    if (b >= nblk) return;
+    const int lane = (int)t & 63;
+    const SplitFrag f = split_f32(*(const f32x4*)(src + b * 256 + (lane & 15) * 16 + (lane >> 4) * 4));
+    dst[b * SPLIT_BLOCK_U + lane] = f.lo;
+    ((u32x2*)(dst + b * SPLIT_BLOCK_U + 64))[lane] = f.hi;
+}
+
+hipError_t launch_split_weights(const float* src, void* dst, long long nblk, hipStream_t s) {
+    if (nblk <= 0 || nblk > (1ll << 28)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_split_weights, dim3((unsigned)((nblk + 3) / 4)), dim3(256), 0, s, src, (u32x4*)dst, nblk);
+    return hipGetLastError();
+}
+
 namespace {
 
 template <int WC, int WP, int CF, int PF>

@@ -114,6 +114,8 @@ struct Context {
     volatile int stop = 0;
     uint64_t mem_limit = 0;  // zjai_ctx_set_memory_limit: device bytes a picture may need (0: none)
     void* attention_scratch = nullptr;  // zjai_channel_attention_noalloc's (root context)
+    void* weight_stage = nullptr;  // f32 weights on their way to the split form (root context)
+    size_t weight_stage_bytes = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.0f;
     long long launches = 0;
@@ -138,6 +140,7 @@ struct Context {
     TensorP alloc(int n, int c, int h, int w, int dtype);
     void check_stop();
     hipEvent_t take_event();
+    void release_weight_stage();
     ~Context();
 };
 

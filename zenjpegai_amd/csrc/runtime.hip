@@ -137,6 +137,13 @@ Context::~Context() {
     for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
     if (range_slots) (void)hipFree(range_slots);
     if (attention_scratch) (void)hipFree(attention_scratch);
+    release_weight_stage();
+}
+
+void Context::release_weight_stage() {
+    if (weight_stage) (void)hipFree(weight_stage);
+    weight_stage = nullptr;
+    weight_stage_bytes = 0;
 }
 
 void range_slots_init(Context& ctx) {
@@ -214,9 +221,6 @@ static uint16_t f32_to_bf16_bits(float v) {
     return (uint16_t)(r >> 16);
 }
 
-// Largest f32 that rounds to a finite bf16 (SPLIT_MAX of split.h).
-static constexpr float SPLIT_MAX_HOST = 3.39531337e38f;
-
 // The f32 value of a storage-dtype weight (f16 / bf16 upcasts are exact).
 static float storage_value(float v, int dtype) {
     if (dtype == DT_F32) return v;
@@ -267,54 +271,26 @@ static void* upload_as(Context& ctx, const std::vector<float>& host, int dtype, 
 }
 
 // A packed f32 weight ([..][16 outputs][16 channels] blocks) as three bf16 pieces per value in
-// the fragment order of split.h: per block the 64 lanes' (p1 x4, p0 x4), then their p2 x4, lane =
-// 16 * (channel / 4) + output. A value that is not finite as bf16 is kept whole in p2.
-static void* upload_split(const std::vector<float>& host, size_t* bytes_out, size_t* total) {
-    // Round to nearest even; v is finite as bf16 or NaN / infinite (whose low bits do not round up).
-    auto rne = [](float v) {
-        uint32_t b;
-        std::memcpy(&b, &v, 4);
-        const bool nan = (b & 0x7fffffff) > 0x7f800000;
-        const uint32_t r = (b + 0x7fff + ((b >> 16) & 1)) & 0xffff0000u;
-        return nan ? (b | 0x400000u) & 0xffff0000u : r;
-    };
-    auto f = [](uint32_t b) {
-        float v;
-        std::memcpy(&v, &b, 4);
-        return v;
-    };
-    const size_t nblk = host.size() / 256;
-    std::unique_ptr<uint16_t[]> h(new uint16_t[nblk * 768]);
-    for (size_t b = 0; b < nblk; ++b) {
-        uint16_t* lo = h.get() + b * 768;
-        uint16_t* hi = lo + 512;
-        for (int r = 0; r < 16; ++r) {
-            const float* src = host.data() + b * 256 + r * 16;
-            uint16_t p0[16], p1[16], p2[16];
-            for (int c = 0; c < 16; ++c) {  // one row of 16 channels, branch-free
-                const float v = src[c];
-                const bool fin = std::fabs(v) <= SPLIT_MAX_HOST;
-                const uint32_t b0 = rne(fin ? v : 0.0f);
-                const float r1 = v - f(b0);
-                const uint32_t b1 = rne(fin ? r1 : 0.0f);
-                p0[c] = (uint16_t)(b0 >> 16);
-                p1[c] = (uint16_t)(b1 >> 16);
-                p2[c] = (uint16_t)(rne(r1 - f(b1)) >> 16);
-            }
-            for (int q = 0; q < 4; ++q) {
-                const int lane = q * 16 + r;
-                std::memcpy(lo + lane * 8, p1 + 4 * q, 8);
-                std::memcpy(lo + lane * 8 + 4, p0 + 4 * q, 8);
-                std::memcpy(hi + lane * 4, p2 + 4 * q, 8);
-            }
-        }
+// the fragment order of split.h, split on the device: on the host a HOP luma net's weights took
+// 4 ms of its 9 ms. The f32 copy goes through a buffer that the context keeps (the largest layer's
+// size), on the null stream as the plain uploads.
+static void* upload_split(Context& ctx, const std::vector<float>& host, size_t* bytes_out, size_t* total) {
+    Context& c = ctx.top();
+    const size_t n = host.size() * 4, bytes = n / 2 * 3;
+    if (c.weight_stage_bytes < n) {
+        c.release_weight_stage();
+        ZJAI_HIP(hipMalloc(&c.weight_stage, std::max(n, size_t(4) << 20)));
+        c.weight_stage_bytes = std::max(n, size_t(4) << 20);
     }
-    const size_t bytes = nblk * 1536;
+    ZJAI_HIP(hipMemcpy(c.weight_stage, host.data(), n, hipMemcpyHostToDevice));
     void* dev = nullptr;
     ZJAI_HIP(hipMalloc(&dev, bytes));
-    ZJAI_HIP(hipMemcpy(dev, h.get(), bytes, hipMemcpyHostToDevice));
+    std::unique_ptr<void, hipError_t (*)(void*)> keep(dev, hipFree);
+    ZJAI_HIP(launch_split_weights((const float*)c.weight_stage, dev, (long long)(host.size() / 256), nullptr));
+    ZJAI_HIP(hipStreamSynchronize(nullptr));
+    keep.release();
     *bytes_out = bytes;
-    *total += *bytes_out;
+    *total += bytes;
     return dev;
 }
 
@@ -419,7 +395,7 @@ LayerP make_conv(Context& ctx, int cin, int cout, int kh, int kw, int stride, in
                 const float* src = weight + ((size_t)(g * cout_g + ocl) * cin_g + icl) * T;
                 for (int t = 0; t < T; ++t) dst[(size_t)t * 16 * CK] = src[t];
             }
-    L->wpk = conv_is_split(L->kind, dtype) ? upload_split(pk, &L->wpk_bytes, &L->dev_bytes)
+    L->wpk = conv_is_split(L->kind, dtype) ? upload_split(ctx, pk, &L->wpk_bytes, &L->dev_bytes)
                                            : upload_as(ctx, pk, dtype, &L->wpk_bytes, &L->dev_bytes);
     if (dtype != DT_F32 && L->kind == CK_3x3 && groups == 1 && (cin == 64 || cin == 128) && cout % 64 == 0 && no_extra &&
         pad_h == 1 && pad_w == 1) {
@@ -503,7 +479,7 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
                     }
             }
     }
-    L->wpk = dtype == DT_F32 ? upload_split(pk, &L->wpk_bytes, &L->dev_bytes)
+    L->wpk = dtype == DT_F32 ? upload_split(ctx, pk, &L->wpk_bytes, &L->dev_bytes)
                              : upload_as(ctx, pk, dtype, &L->wpk_bytes, &L->dev_bytes);
     if (bias) L->bias = upload_f32(bias, cout, &L->dev_bytes);
     if (k == 3 && cout > 8 && (dtype != DT_F32 || pad == 1) && conv_tr_merged_taps_supported(L->ntaps) && L->nblk_g % TR_MERGED_NB == 0) {
@@ -530,7 +506,7 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
                         }
                     }
             }
-        L->wpk_m = dtype == DT_F32 ? upload_split(pm, &L->wpk_m_bytes, &L->dev_bytes)
+        L->wpk_m = dtype == DT_F32 ? upload_split(ctx, pm, &L->wpk_m_bytes, &L->dev_bytes)
                                    : upload_as(ctx, pm, dtype, &L->wpk_m_bytes, &L->dev_bytes);
     }
     if (cout <= 8) {
