@@ -14,7 +14,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from zenjpegai_amd import nn, synth
+from zenjpegai_amd import _lib, nn, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -97,3 +97,66 @@ def test_values_that_are_not_finite(eng, kind):
         np.testing.assert_array_equal(y[inf], want[inf])
         fin = np.isfinite(want)
         assert np.isfinite(y[fin]).all() and np.allclose(y[fin], want[fin], rtol=1e-4, atol=1e-3)
+
+
+@pytest.fixture(scope="module")
+def eng_igemm():
+    e = nn.Engine(0, "f32", flags=_lib.CTX_IGEMM_CONV1X1)
+    yield e
+    e.close()
+
+
+# (kind, cin, cout, channel, columns between values): single chunks, whole and odd pairs of chunks, wide and
+# narrow tiles, the transposed layers phase by phase and (at 1280 columns) merged.
+ONE_CHANNEL = [("1x1", 4, 64, 2, 4), ("1x1", 32, 64, 21, 4), ("1x1", 48, 16, 40, 4), ("1x1", 160, 160, 70, 4),
+               ("3x3", 4, 128, 1, 4), ("3x3", 64, 64, 50, 4), ("s2", 20, 128, 17, 4), ("2x2", 36, 64, 33, 4),
+               ("t3", 20, 64, 7, 4), ("t3", 32, 128, 30, 32), ("t4", 32, 32, 11, 4)]
+N_VALUES = 40
+
+
+def _products(e, kind, cin, cout, ch, step, xv, wv):
+    """wv[o] * xv[i] as the layer computes them, [o][i]: the input is zero but for channel ch of every
+    step-th column, the weights but for the tap of that channel on the output's own position."""
+    x = np.zeros((cin, 1, step * len(xv)), np.float32)
+    x[ch, 0, ::step] = xv
+    if kind[0] == "t":
+        k = int(kind[1])
+        w = np.zeros((cin, cout, k, k), np.float32)
+        w[ch, :, 1, 1] = wv
+        layer = nn.ConvTransposeLayer(nn.ConvTranspose2d(cin, cout, k, 2, 1, 4 - k, w, np.zeros(cout, np.float32)), e)
+        scale = 2
+    else:
+        k, stride = {"1x1": (1, 1), "3x3": (3, 1), "s2": (3, 2), "2x2": (2, 1)}[kind]
+        pad, ext = {"1x1": ((0, 0), (0, 0, 0, 0)), "2x2": ((0, 0), (0, 0, 1, 1))}.get(kind, ((1, 1), (0, 0, 0, 0)))
+        w = np.zeros((cout, cin, k, k), np.float32)
+        w[:, ch, (k - 1) // 2, (k - 1) // 2] = wv
+        layer = nn.ConvLayer(nn.Conv2d(cin, cout, (k, k), stride, pad, 1, w, np.zeros(cout, np.float32)), e, extra_pad=ext)
+        scale = 1 / stride
+    y = layer.forward(e, nn.BTensor.from_planar(e, x)).to_planar()
+    return y[:, 0, ::int(step * scale)][:, :len(xv)]
+
+
+def _cycle(values, n):
+    return np.resize(np.asarray(values, np.float32), n)
+
+
+F32 = np.finfo(np.float32)
+# Around 0x7f7f7fff, the largest f32 that rounds to a finite bf16, and up to f32's own largest.
+TOP = np.array([0x7f7f7fff, 0x7f7f8000, 0x7f7f8001, 0x7f7fffff, 0x7f7fffa5, 0x7f7e1234, 0x7f7f6f43, 0x7f6fffff],
+               np.uint32).view(np.float32)
+
+
+@pytest.mark.parametrize("kind,cin,cout,ch,step", ONE_CHANNEL)
+@pytest.mark.parametrize("weights", [False, True])
+def test_the_largest_finite_values(eng, eng_igemm, kind, cin, cout, ch, step, weights):
+    """Finite values above bf16's largest are three pieces like any other: times zero and the powers of
+    two up to one every bit is there, times other values the six products' 2^-22."""
+    top, other = np.concatenate([TOP, -TOP]), [0.0, 1.0, -1.0, 0.5, -2.0 ** -20, 2.0 ** -100, 0.3, -0.7123456]
+    xv, wv = (_cycle(other, N_VALUES), _cycle(top, cout)) if weights else (_cycle(top, N_VALUES), _cycle(other, cout))
+    want = wv[:, None] * xv
+    exact = np.frexp(np.abs(wv[:, None] if not weights else xv[None]))[0] * np.ones_like(want)
+    exact = (exact == 0.5) | (exact == 0)
+    for e in (eng, eng_igemm) if kind == "1x1" else (eng,):
+        y = _products(e, kind, cin, cout, ch, step, xv, wv)
+        np.testing.assert_array_equal(y[exact], want[exact])
+        np.testing.assert_allclose(y[~exact], want[~exact], rtol=2.0 ** -22)

@@ -19,10 +19,12 @@
 // times where the f32 MFMA rounds it K times (K = 1152, against 64-bit sums: 3e-7 relative
 // instead of 4-6e-7).
 //
-// A value that is not finite (or above bf16's largest, 3.395e38) keeps its whole in p2, which
-// only ever meets b0: infinities and NaN then reach the result as in f32 arithmetic. Values below
-// 2^-110 lose low bits (the pieces become subnormal).
+// A finite value too large to round to bf16 takes bf16's largest for p0; p1 and p2 then hold the rest
+// exactly. A value that is not finite is kept whole in p2, which only ever meets b0. Values below 2^-110
+// lose low bits (the pieces become subnormal).
 #pragma once
+
+#include <cfloat>
 
 #include "mfma.h"
 
@@ -31,8 +33,8 @@ namespace zjai {
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// Largest f32 that rounds to a finite bf16.
-constexpr float SPLIT_MAX = 3.39531337e38f;
+// The largest f32 that rounds to a finite bf16 (0x7f7f7fff).
+constexpr float SPLIT_MAX = 0x1.fefffep127f;
 
 struct SplitFrag {
     u32x4 lo;  // p1 of channels 0..3, p0 of channels 0..3
@@ -51,8 +53,9 @@ __device__ __forceinline__ SplitFrag split_f32(f32x4 v) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const float x = v[2 * h], y = v[2 * h + 1];
-        const bool fx = __builtin_fabsf(x) <= SPLIT_MAX, fy = __builtin_fabsf(y) <= SPLIT_MAX;
-        const unsigned p0 = pack_bf16(fx ? x : 0.0f, fy ? y : 0.0f);
+        const bool fx = __builtin_fabsf(x) <= FLT_MAX, fy = __builtin_fabsf(y) <= FLT_MAX;
+        const unsigned p0 = pack_bf16(fx ? __builtin_amdgcn_fmed3f(x, -SPLIT_MAX, SPLIT_MAX) : 0.0f,
+                                      fy ? __builtin_amdgcn_fmed3f(y, -SPLIT_MAX, SPLIT_MAX) : 0.0f);
         const float rx = x - __builtin_bit_cast(float, p0 << 16);
         const float ry = y - __builtin_bit_cast(float, p0 & 0xffff0000u);
         const unsigned p1 = pack_bf16(fx ? rx : 0.0f, fy ? ry : 0.0f);
