@@ -160,3 +160,18 @@ def test_the_largest_finite_values(eng, eng_igemm, kind, cin, cout, ch, step, we
         y = _products(e, kind, cin, cout, ch, step, xv, wv)
         np.testing.assert_array_equal(y[exact], want[exact])
         np.testing.assert_allclose(y[~exact], want[~exact], rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize("kind,cin,cout,ch,step", ONE_CHANNEL)
+def test_single_values_that_are_not_finite(eng, eng_igemm, kind, cin, cout, ch, step):
+    """Every pairing of infinities, NaN, zeros, values of one, two and three pieces and the largest ones,
+    one product an output: what f32 gives, infinity times infinity among it."""
+    v = [np.inf, -np.inf, np.nan, 0.0, 1.0, -1.0 - 2.0 ** -9, 0.3, F32.max, -F32.max, 1e-30]
+    xv, wv = _cycle(v, N_VALUES), _cycle(np.repeat(v, 2), cout)
+    with np.errstate(all="ignore"):
+        want = wv[:, None] * xv
+    for e in (eng, eng_igemm) if kind == "1x1" else (eng,):
+        y = _products(e, kind, cin, cout, ch, step, xv, wv)
+        fin = np.isfinite(want)
+        np.testing.assert_array_equal(y[~fin], want[~fin])
+        np.testing.assert_allclose(y[fin], want[fin], rtol=2.0 ** -22)

@@ -214,7 +214,7 @@ conv_igemm_split(const ConvParams p) {
                 for (int cf = 0; cf < CF; ++cf)
 #pragma unroll
                     for (int pf = 0; pf < PF; ++pf) {
-                        big[cf][pf] += small[cf][pf];
+                        big[cf][pf] = split_sum(big[cf][pf], small[cf][pf]);
                         small[cf][pf] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                     }
             }

@@ -20,8 +20,10 @@
 // instead of 4-6e-7).
 //
 // A finite value too large to round to bf16 takes bf16's largest for p0; p1 and p2 then hold the rest
-// exactly. A value that is not finite is kept whole in p2, which only ever meets b0. Values below 2^-110
-// lose low bits (the pieces become subnormal).
+// exactly. An infinity or NaN is p0, with p1 = 0 and p2 NaN: a0 b0 then goes to infinity or NaN as the
+// f32 product does, and the full-size sum with it, while the small products, which zero pieces turn
+// into NaN, no longer count (split_sum). Values below 2^-110 lose low bits (the pieces become
+// subnormal). A product within 2^-7 of overflow may overflow: its a0 b0 can be that much larger.
 #pragma once
 
 #include <cfloat>
@@ -54,8 +56,8 @@ __device__ __forceinline__ SplitFrag split_f32(f32x4 v) {
     for (int h = 0; h < 2; ++h) {
         const float x = v[2 * h], y = v[2 * h + 1];
         const bool fx = __builtin_fabsf(x) <= FLT_MAX, fy = __builtin_fabsf(y) <= FLT_MAX;
-        const unsigned p0 = pack_bf16(fx ? __builtin_amdgcn_fmed3f(x, -SPLIT_MAX, SPLIT_MAX) : 0.0f,
-                                      fy ? __builtin_amdgcn_fmed3f(y, -SPLIT_MAX, SPLIT_MAX) : 0.0f);
+        const unsigned p0 = pack_bf16(fx ? __builtin_amdgcn_fmed3f(x, -SPLIT_MAX, SPLIT_MAX) : x,
+                                      fy ? __builtin_amdgcn_fmed3f(y, -SPLIT_MAX, SPLIT_MAX) : y);
         const float rx = x - __builtin_bit_cast(float, p0 << 16);
         const float ry = y - __builtin_bit_cast(float, p0 & 0xffff0000u);
         const unsigned p1 = pack_bf16(fx ? rx : 0.0f, fy ? ry : 0.0f);
@@ -89,6 +91,15 @@ __device__ __forceinline__ void mma_split_rows(f32x4 (&big)[N], f32x4 (&small)[N
     for (int r = 0; r < N; ++r) small[r] = mfma_bf16(ahi, b[r].lo, small[r]);
 }
 
+// The sum of a pair of accumulators, the small one made finite: where the full-size sum is infinite or
+// NaN, which it then stays, the small products may be NaN or have overflowed to the other sign. (The
+// median of a NaN and two numbers is the smaller number.)
+__device__ __forceinline__ f32x4 split_sum(f32x4 big, f32x4 small) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) small[i] = __builtin_amdgcn_fmed3f(small[i], -FLT_MAX, FLT_MAX);
+    return big + small;
+}
+
 // 1x1 layers keep one accumulator: the small products of every two K chunks (32 channels; the last
 // chunk of an odd number by itself) are summed from zero and then added to it, which leaves
 // registers for the fused transformer blocks and rounds the full-size sum 9 times per 32 products.
@@ -111,8 +122,8 @@ __device__ __forceinline__ void mma_split32_2(f32x4& c0, f32x4& c1, const SplitF
         : "+v"(c0), "+v"(c1), "=&v"(s0), "=&v"(s1)
         : "v"(a0.lo), "v"(split_hi(a0)), "v"(a1.lo), "v"(split_hi(a1)), "v"(b00.lo), "v"(split_hi(b00)), "v"(b01.lo),
           "v"(split_hi(b01)), "v"(b10.lo), "v"(split_hi(b10)), "v"(b11.lo), "v"(split_hi(b11)));
-    c0 += s0;
-    c1 += s1;
+    c0 = split_sum(c0, s0);
+    c1 = split_sum(c1, s1);
 }
 __device__ __forceinline__ void mma_split32_1(f32x4& c0, const SplitFrag& a0, const SplitFrag& a1, const SplitFrag& b0,
                                               const SplitFrag& b1) {
@@ -123,7 +134,7 @@ __device__ __forceinline__ void mma_split32_1(f32x4& c0, const SplitFrag& a0, co
         : "+v"(c0), "=&v"(s0)
         : "v"(a0.lo), "v"(split_hi(a0)), "v"(a1.lo), "v"(split_hi(a1)), "v"(b0.lo), "v"(split_hi(b0)), "v"(b1.lo),
           "v"(split_hi(b1)));
-    c0 += s0;
+    c0 = split_sum(c0, s0);
 }
 __device__ __forceinline__ void mma_split16_1(f32x4& c0, const SplitFrag& a0, const SplitFrag& b0) {
     f32x4 s0;
@@ -131,7 +142,7 @@ __device__ __forceinline__ void mma_split16_1(f32x4& c0, const SplitFrag& a0, co
         ZJAI_MF "%1, %2, %5, 0\n\t" ZJAI_MF "%0, %2, %4, %0\n\t" ZJAI_MF "%1, %3, %4, %1\n\t" ZJAI_WAIT
         : "+v"(c0), "=&v"(s0)
         : "v"(a0.lo), "v"(split_hi(a0)), "v"(b0.lo), "v"(split_hi(b0)));
-    c0 += s0;
+    c0 = split_sum(c0, s0);
 }
 // N accumulators sharing A; chunk 1 is there only if `two` (uniform).
 template <int N>
@@ -145,15 +156,6 @@ __device__ __forceinline__ void mma_split32(f32x4 (&acc)[N], const SplitFrag& a0
 #pragma unroll
         for (int r = 0; r < N; ++r) mma_split16_1(acc[r], a0, b0[r]);
     }
-}
-
-// The sum of a finished pair of accumulators. An infinite full-size sum stays infinite: its small
-// products may have overflowed to either sign.
-__device__ __forceinline__ f32x4 split_sum(f32x4 big, f32x4 small) {
-    f32x4 r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = __builtin_isinf(big[i]) ? big[i] : big[i] + small[i];
-    return r;
 }
 
 // A packed 16 x 16 weight block (16 outputs x 16 input channels) in split form: 96 16-byte
