@@ -175,3 +175,17 @@ def test_single_values_that_are_not_finite(eng, eng_igemm, kind, cin, cout, ch, 
         fin = np.isfinite(want)
         np.testing.assert_array_equal(y[~fin], want[~fin])
         np.testing.assert_allclose(y[fin], want[fin], rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize("kind,cin,cout,ch,step", ONE_CHANNEL)
+@pytest.mark.parametrize("igemm", [False, True])
+def test_products_that_overflow(eng, eng_igemm, kind, cin, cout, ch, step, igemm):
+    """A finite product past f32's largest is infinite, of its own sign, although its small piece
+    products may have overflowed to the other one."""
+    n = N_VALUES
+    xv = synth.uniform(35, "split/ovx", (n,), 1.0, 2.0) * _cycle([-1e30, 1e30], n)
+    wv = synth.uniform(36, f"split/ovw{cout}", (cout,), 1.0, 2.0) * _cycle([-1e30, 1e30, 1e30], cout)
+    with np.errstate(over="ignore"):
+        want = wv[:, None] * xv
+    assert np.isinf(want).all()
+    np.testing.assert_array_equal(_products(eng_igemm if igemm else eng, kind, cin, cout, ch, step, xv, wv), want)

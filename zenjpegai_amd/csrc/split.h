@@ -19,11 +19,13 @@
 // times where the f32 MFMA rounds it K times (K = 1152, against 64-bit sums: 3e-7 relative
 // instead of 4-6e-7).
 //
-// A finite value too large to round to bf16 takes bf16's largest for p0; p1 and p2 then hold the rest
-// exactly. An infinity or NaN is p0, with p1 = 0 and p2 NaN: a0 b0 then goes to infinity or NaN as the
-// f32 product does, and the full-size sum with it, while the small products, which zero pieces turn
-// into NaN, no longer count (split_sum). Values below 2^-110 lose low bits (the pieces become
-// subnormal). A product within 2^-7 of overflow may overflow: its a0 b0 can be that much larger.
+// From 2^15 on p0 is cut off instead of rounded, so that p1 has the value's sign: where a0 b0 overflows,
+// a1 b1, which shares its accumulator, can then only overflow to the same infinity (it overflows only if
+// both operands are that large). FLT_MAX's p0 is finite for the same reason. An infinity or NaN is p0,
+// with p1 = 0 and p2 NaN: a0 b0 goes to infinity or NaN as the f32 product does, and the full-size sum
+// with it, while the small products, which zero pieces turn into NaN, no longer count (split_sum).
+// Values below 2^-110 lose low bits (the pieces become subnormal). A product within 2^-7 of overflow may
+// overflow: its a0 b0 can be that much larger.
 #pragma once
 
 #include <cfloat>
@@ -35,8 +37,8 @@ namespace zjai {
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// The largest f32 that rounds to a finite bf16 (0x7f7f7fff).
-constexpr float SPLIT_MAX = 0x1.fefffep127f;
+// From here on a value's p0 is cut off instead of rounded.
+constexpr float SPLIT_CUT = 0x1p15f;
 
 struct SplitFrag {
     u32x4 lo;  // p1 of channels 0..3, p0 of channels 0..3
@@ -50,14 +52,19 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
     return __builtin_bit_cast(unsigned, r);
 }
 
+// What rounds to v's p0 (`fin`: v is finite).
+__device__ __forceinline__ float split_p0(float v, bool fin) {
+    const float cut = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) & 0xffff0000u);
+    return __builtin_fabsf(v) < SPLIT_CUT ? v : fin ? cut : v;
+}
+
 __device__ __forceinline__ SplitFrag split_f32(f32x4 v) {
     SplitFrag f;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const float x = v[2 * h], y = v[2 * h + 1];
         const bool fx = __builtin_fabsf(x) <= FLT_MAX, fy = __builtin_fabsf(y) <= FLT_MAX;
-        const unsigned p0 = pack_bf16(fx ? __builtin_amdgcn_fmed3f(x, -SPLIT_MAX, SPLIT_MAX) : x,
-                                      fy ? __builtin_amdgcn_fmed3f(y, -SPLIT_MAX, SPLIT_MAX) : y);
+        const unsigned p0 = pack_bf16(split_p0(x, fx), split_p0(y, fy));
         const float rx = x - __builtin_bit_cast(float, p0 << 16);
         const float ry = y - __builtin_bit_cast(float, p0 & 0xffff0000u);
         const unsigned p1 = pack_bf16(fx ? rx : 0.0f, fy ? ry : 0.0f);
