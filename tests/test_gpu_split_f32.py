@@ -14,7 +14,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from zenjpegai_amd import _lib, nn, synth
+from zenjpegai_amd import _lib, model, nn, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -189,3 +189,38 @@ def test_products_that_overflow(eng, eng_igemm, kind, cin, cout, ch, step, igemm
         want = wv[:, None] * xv
     assert np.isinf(want).all()
     np.testing.assert_array_equal(_products(eng_igemm if igemm else eng, kind, cin, cout, ch, step, xv, wv), want)
+
+
+@pytest.mark.parametrize("op,comp", [("sop", "y"), ("hop", "y"), ("hop", "uv")])
+def test_fused_blocks_split_large_values_as_the_single_layers_do(op, comp):
+    """Every fifth gate value of the feed-forward halves and channel inside the ResAUs past the size from
+    which a p0 is cut off (taken back by the next weights): waves of the fused kernels then split both
+    kinds, to the same bits as the layers by themselves."""
+    p = {k: np.array(v) for k, v in synth.random_params(op, comp, seed=41, gain=0.5).items()}
+    big = np.float32(2.0 ** 18)
+    n = 0
+    for k in p:
+        if k.endswith("ffn.dwconv.weight"):
+            hid = p[k].shape[0] // 2
+            p[k][hid::5] *= big
+            p[k.replace("dwconv", "project_out")][:, ::5] /= big
+            n += 1
+        elif k.endswith(".conv2.weight") and k.replace("conv2", "conv") in p and p[k].shape[2] == 1:
+            p[k.replace("conv2", "conv")][::5] *= big
+            p[k][:, ::5] /= big
+            n += 1
+    assert n >= 2, n
+    lh, lw = 7, 9
+    y, uv = synth.latent(41, "big/y", 160, lh, lw), synth.latent(41, "big/uv", 96, lh, lw)
+    outs = []
+    for flags in (0, _lib.CTX_UNFUSED_BLOCKS):
+        e = nn.Engine(0, "f32", flags=flags)
+        yt = nn.BTensor.from_planar(e, y)
+        if comp == "y":
+            outs.append(model.SynthesisPrimary.load(p, op, e).forward(e, yt, 16 * lh, 16 * lw))
+        else:
+            net = model.SynthesisSecondary.load(p, op, e)
+            outs.append(net.forward(e, yt, nn.BTensor.from_planar(e, uv), 16 * lh, 16 * lw))
+        e.close()
+    assert np.isfinite(outs[0]).all() and len(np.unique(outs[0])) > 1000
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))

@@ -26,7 +26,7 @@ namespace zjai {
 __device__ u32x4 g_zero_split[1];  // 16 zero bytes: the source of padding units
 
 template <int KH, int KW, int S, bool TR, int WC, int WP, int CF, int PF, int TS, int NHB, int RW>
-__global__ void __launch_bounds__(WC * WP * 64, 2)
+__global__ void __launch_bounds__(WC * WP * 64, S == 1 && CF * PF == 4 ? 4 : 2)  // 4: as LDS allows, in 128 registers
 conv_igemm_split(const ConvParams p) {
     constexpr int NT = WC * WP * 64;
     constexpr int TY = WP * PF;
@@ -124,16 +124,15 @@ conv_igemm_split(const ConvParams p) {
     auto store_halo = [&](int chunk) __attribute__((always_inline)) {
         u32x4* dst = s_lds + (NHB == 2 ? (chunk & 1) * HALO_U : 0);
         u32x2* hi = (u32x2*)(dst + 4 * NPX);
+        f32x4 v[HN];
 #pragma unroll
-        for (int i = 0; i < HN; ++i) {
-            u32x4 v = rh[i];
-            if (p.relu6_in) v = relu6_vec<float>(v);
-            const SplitFrag f = split_f32(__builtin_bit_cast(f32x4, v));
+        for (int i = 0; i < HN; ++i) v[i] = __builtin_bit_cast(f32x4, p.relu6_in ? relu6_vec<float>(rh[i]) : rh[i]);
+        split_each<HN>(v, [&](int i, const SplitFrag& f) __attribute__((always_inline)) {
             if (tid + i * NT < HP * 4) {
                 dst[hdst[i]] = f.lo;
                 hi[hdst[i]] = f.hi;
             }
-        }
+        });
     };
     // Weight slot of stage (chunk, j): taps j * TS .. of blocks nb0 .. nb0 + NB - 1, loaded RW - 1
     // stages ahead (the slot was last read that many stages ago). The lanes' offsets stay, the
@@ -390,14 +389,15 @@ conv_tr_merged_split(const ConvParams p) {
             constexpr int j = decltype(jc)::value;
             if (j == 0) {
                 if (chunk > 0) __syncthreads();  // every wave is done with the last halo
+                f32x4 v[HN];
 #pragma unroll
-                for (int i = 0; i < HN; ++i) {
-                    const SplitFrag f = split_f32(__builtin_bit_cast(f32x4, rh[i]));
+                for (int i = 0; i < HN; ++i) v[i] = __builtin_bit_cast(f32x4, rh[i]);
+                split_each<HN>(v, [&](int i, const SplitFrag& f) __attribute__((always_inline)) {
                     if (tid + i * NT < HP * 4) {
                         s_lds[hdst[i]] = f.lo;
                         s_hhi[hdst[i]] = f.hi;
                     }
-                }
+                });
             }
             // This stage's weights have landed; the next chunk's halo loads, issued after them, may
             // still fly.
@@ -482,7 +482,7 @@ conv_tr_merged_split(const ConvParams p) {
 // MFMA) once the products run on the bf16 matrix cores.
 // ---------------------------------------------------------------------------------------------
 template <int WC, int WP, int CF, int PF>
-__global__ void __launch_bounds__(WC * WP * 64, 2)
+__global__ void __launch_bounds__(WC * WP * 64, 3)  // three workgroups per CU, as LDS allows, in 168 registers
 conv1x1_ring_split(const ConvParams p) {
     constexpr int NT = WC * WP * 64;
     constexpr int NB = WC * CF, MP = WP * PF * 16;
@@ -576,12 +576,13 @@ conv1x1_ring_split(const ConvParams p) {
 #pragma unroll 1
     for (int st = 0; st < nst; ++st) {
         if (st > 0) __syncthreads();  // every wave is done with the last stage's positions
+        f32x4 v[XN];
 #pragma unroll
-        for (int i = 0; i < XN; ++i) {
-            const SplitFrag f = split_f32(__builtin_bit_cast(f32x4, rx[i]));
+        for (int i = 0; i < XN; ++i) v[i] = __builtin_bit_cast(f32x4, rx[i]);
+        split_each<XN>(v, [&](int i, const SplitFrag& f) __attribute__((always_inline)) {
             s_lds[xdst[i]] = f.lo;
             s_xhi[xdst[i]] = f.hi;
-        }
+        });
         asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // this wave's weights of the stage
         __syncthreads();
         if (st + 1 < nst) {

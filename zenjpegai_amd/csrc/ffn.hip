@@ -971,15 +971,20 @@ __global__ void __launch_bounds__(FTHREADS) k_ffn_f32(const FfnArgs p) {
         }
         __syncthreads();  // the gate values are down
         const int ts = opaque(tid);
+        constexpr int GN = (FOP * 8 + FTHREADS - 1) / FTHREADS;
+        f32x4 gv[GN];
 #pragma unroll
-        for (int i = 0; i < (FOP * 8 + FTHREADS - 1) / FTHREADS; ++i) {
+        for (int i = 0; i < GN; ++i) {
+            const int v = min(ts + i * FTHREADS, FOP * 8 - 1), o = v >> 3, q = v & 7;
+            gv[i] = *(const f32x4*)(s_gf + o * 32 + ((q ^ (o & 7)) << 2));
+        }
+        split_each<GN>(gv, [&](int i, const SplitFrag& f) __attribute__((always_inline)) {
             const int v = ts + i * FTHREADS, o = v >> 3, q = v & 7;
             if (v < FOP * 8) {
-                const SplitFrag f = split_f32(*(const f32x4*)(s_gf + o * 32 + ((q ^ (o & 7)) << 2)));
                 s_g[q * GPX + (o ^ q)] = f.lo;
                 s_ghi[q * GPX + (o ^ q)] = f.hi;
             }
-        }
+        });
         // W_out(s) is in registers before the next direct loads go out (their count would be
         // waited for with it).
 #pragma unroll

@@ -96,20 +96,23 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) k_resau(const Res
     }
 #pragma unroll
     for (int i = 0; i < HIT; ++i) {
-        const int u = tid + i * 256;
-        if (u >= HU) break;
-        const int pix = u / UPP, q = u - pix * UPP;
+        const int u = tid + i * 256, pix = u / UPP, q = u - pix * UPP;
         const int hy = pix / HX, hx = pix - hy * HX;
         const int iy = y0 - 1 + hy, ix = x0 - 1 + hx;
         const bool in = iy >= 0 && iy < p.h && ix >= 0 && ix < p.w;
-        const u32x4 v = in ? relu6_vec<T>(hv[i]) : u32x4{0u, 0u, 0u, 0u};
-        if constexpr (F32) {
-            const SplitFrag f = split_f32(__builtin_bit_cast(f32x4, v));
+        hv[i] = in ? relu6_vec<T>(hv[i]) : u32x4{0u, 0u, 0u, 0u};
+        if (!F32 && u < HU) s_h[pix * UPP + (q ^ (pix & (UPP - 1)))] = hv[i];
+    }
+    if constexpr (F32) {
+        f32x4 v[HIT];
+#pragma unroll
+        for (int i = 0; i < HIT; ++i) v[i] = __builtin_bit_cast(f32x4, hv[i]);
+        split_each<HIT>(v, [&](int i, const SplitFrag& f) __attribute__((always_inline)) {
+            const int u = tid + i * 256, pix = u / UPP, q = u - pix * UPP;
+            if (u >= HU) return;
             s_h[q * NPX + pix] = f.lo;
             s_hhi[q * NPX + pix] = f.hi;
-        } else {
-            s_h[pix * UPP + (q ^ (pix & (UPP - 1)))] = v;
-        }
+        });
     }
     __syncthreads();
 
@@ -154,15 +157,15 @@ __global__ void __launch_bounds__(256, sizeof(T) == 4 ? 2 : 1) k_resau(const Res
     static_assert(!F32 || UPP * TPX <= UPP * NPX, "t fits the halo's place");
     u32x2* const s_thi = (u32x2*)(s_h + (F32 ? UPP * TPX : 0));
     // t (channel gi * 16 + 4 grp + k at position (r0 + r) * 16 + col) rounded to the storage type.
+    if constexpr (F32)
+        split_each<NPW>(acc, [&](int r, const SplitFrag& f) __attribute__((always_inline)) {
+            const int i = (gi * 4 + grp) * TPX + (r0 + r) * 16 + col;
+            s_h[i] = f.lo;
+            s_thi[i] = f.hi;
+        });
 #pragma unroll
-    for (int r = 0; r < NPW; ++r) {
+    for (int r = 0; r < (F32 ? 0 : NPW); ++r) {
         const int pos = (r0 + r) * 16 + col;
-        if constexpr (F32) {
-            const SplitFrag f = split_f32(acc[r]);
-            s_h[(gi * 4 + grp) * TPX + pos] = f.lo;
-            s_thi[(gi * 4 + grp) * TPX + pos] = f.hi;
-            continue;
-        }
         const int ch = gi * 16 + 4 * grp, unit = ch / VEC;
         T* dst = reinterpret_cast<T*>(s_t + pos * UPP + (unit ^ (pos & (UPP - 1)))) + (ch - unit * VEC);
         typedef T t4 __attribute__((ext_vector_type(4)));

@@ -58,13 +58,15 @@ __device__ __forceinline__ float split_p0(float v, bool fin) {
     return __builtin_fabsf(v) < SPLIT_CUT ? v : fin ? cut : v;
 }
 
+// ORDINARY: all four values are finite and below SPLIT_CUT (the same pieces without a test).
+template <bool ORDINARY = false>
 __device__ __forceinline__ SplitFrag split_f32(f32x4 v) {
     SplitFrag f;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const float x = v[2 * h], y = v[2 * h + 1];
-        const bool fx = __builtin_fabsf(x) <= FLT_MAX, fy = __builtin_fabsf(y) <= FLT_MAX;
-        const unsigned p0 = pack_bf16(split_p0(x, fx), split_p0(y, fy));
+        const bool fx = ORDINARY || __builtin_fabsf(x) <= FLT_MAX, fy = ORDINARY || __builtin_fabsf(y) <= FLT_MAX;
+        const unsigned p0 = ORDINARY ? pack_bf16(x, y) : pack_bf16(split_p0(x, fx), split_p0(y, fy));
         const float rx = x - __builtin_bit_cast(float, p0 << 16);
         const float ry = y - __builtin_bit_cast(float, p0 & 0xffff0000u);
         const unsigned p1 = pack_bf16(fx ? rx : 0.0f, fy ? ry : 0.0f);
@@ -73,6 +75,24 @@ __device__ __forceinline__ SplitFrag split_f32(f32x4 v) {
         f.hi[h] = pack_bf16(rx - __builtin_bit_cast(float, p1 << 16), ry - __builtin_bit_cast(float, p1 & 0xffff0000u));
     }
     return f;
+}
+
+// store(i, split_f32(v[i])) for each of a lane's N vectors: the maximum over them (NaN if one is) costs
+// half an instruction a value, the tests that it spares a wave of ordinary values five of their eleven.
+template <int N, typename F>
+__device__ __forceinline__ void split_each(const f32x4 (&v)[N], F store) {
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m = __builtin_elementwise_maximum(m, __builtin_fabsf(v[i][k]));
+    if (__builtin_amdgcn_ballot_w64(!(m < SPLIT_CUT)) == 0) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) store(i, split_f32<true>(v[i]));
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) store(i, split_f32(v[i]));
+    }
 }
 
 // big += lo . lo, small += the other two MFMAs (16 channels of K).
@@ -114,9 +134,10 @@ __device__ __forceinline__ f32x4 split_sum(f32x4 big, f32x4 small) {
 // The MFMAs are inline assembly, accumulators in place: with a fresh small sum every 32 channels
 // the compiler renames the chains a few instructions apart. It does not know what the block holds,
 // so the block carries its own wait states: two before (an operand written by vector code just
-// before) and 19 after (results of an 8-pass MFMA read or overwritten by vector code).
+// before) and eight after (results read or overwritten by vector code), as the compiler puts them
+// around the builtin.
 #define ZJAI_MF "v_mfma_f32_16x16x32_bf16 "
-#define ZJAI_WAIT "s_nop 15\n\ts_nop 2"
+#define ZJAI_WAIT "s_nop 7"
 __device__ __forceinline__ void mma_split32_2(f32x4& c0, f32x4& c1, const SplitFrag& a0, const SplitFrag& a1,
                                               const SplitFrag& b00, const SplitFrag& b01, const SplitFrag& b10,
                                               const SplitFrag& b11) {
