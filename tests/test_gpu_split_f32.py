@@ -57,7 +57,9 @@ CASES = [("3x3", 4, 4, 1, 1, 1), ("3x3", 20, 24, 1, 9, 17), ("3x3", 160, 160, 1,
          ("3x3", 16, 128, 1, 260, 250), ("3x3", 64, 64, 4, 33, 31), ("3x3", 64, 64, 4, 150, 161),
          ("3x3", 128, 128, 4, 15, 16), ("3x3", 128, 128, 4, 150, 161), ("s2", 20, 16, 1, 1, 7), ("s2", 64, 64, 1, 35, 33),
          ("s2", 24, 32, 1, 66, 64), ("s2", 64, 64, 1, 175, 177), ("s2", 16, 128, 1, 255, 257), ("s2", 16, 128, 1, 440, 431),
-         ("s2", 16, 192, 1, 440, 431), ("2x2", 160, 256, 1, 4, 6), ("2x2", 20, 12, 1, 17, 15), ("2x2", 64, 128, 1, 128, 127),
+         ("s2", 16, 192, 1, 440, 431), ("s2", 16, 16, 1, 500, 431), ("s2", 20, 12, 1, 450, 515),
+         ("2x2", 160, 256, 1, 4, 6), ("2x2", 20, 12, 1, 17, 15), ("2x2", 64, 128, 1, 128, 127),
+         ("2x2", 16, 16, 1, 210, 201), ("2x2", 20, 12, 1, 300, 130),
          ("2x2", 16, 192, 1, 150, 161), ("1x1", 4, 4, 1, 1, 1), ("1x1", 20, 24, 1, 9, 7), ("1x1", 48, 16, 1, 33, 64),
          ("1x1", 160, 160, 1, 8, 15), ("1x1", 128, 64, 1, 128, 127), ("1x1", 96, 128, 1, 150, 130),
          ("1x1", 32, 256, 1, 171, 190), ("t3", 20, 12, 1, 1, 1), ("t3", 36, 64, 1, 17, 15), ("t3", 32, 96, 1, 90, 97),

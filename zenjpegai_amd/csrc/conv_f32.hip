@@ -719,9 +719,11 @@ hipError_t launch_conv_split(int kind, TileCfg c, const ConvParams& p, hipStream
     ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 4, 4, 2, 1, 1, 2)
     ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 4, 4, 1, 3, 1, 2)
     ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 4, 2, 1, 3, 1, 2)
+    ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 8, 1, 1, 3, 1, 2)
     ZJAI_SPLIT(CK_3x3_S2, 3, 3, 2, 1, 4, 1, 1, 9, 1, 2)
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 4, 4, 2, 1, 1, 3)
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 8, 2, 1, 4, 1, 2)
+    ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 4, 1, 2, 4, 1, 2)
     ZJAI_SPLIT(CK_2x2, 2, 2, 1, 1, 8, 1, 1, 4, 1, 2)
     ZJAI_SPLIT(CK_T3, 3, 3, 1, 1, 4, 4, 2, 4, 1, 2)
     ZJAI_SPLIT(CK_T3, 3, 3, 1, 1, 8, 2, 1, 4, 1, 2)

@@ -333,11 +333,11 @@ TileCfg conv_tile_cfg(int cout_g, int kind, int dtype) {
             return cout_g <= 16 ? TileCfg{1, 4, 1, 2} : cout_g <= 32 ? TileCfg{1, 4, 2, 2}
                    : wide ? TileCfg{2, 2, 4, 4} : TileCfg{1, 4, 4, 4};
         if (kind == CK_3x3_S2)
-            return cout_g <= 16 ? TileCfg{1, 4, 1, 1} : cout_g <= 32 ? TileCfg{1, 4, 2, 1}
+            return cout_g <= 16 ? TileCfg{1, 8, 1, 1} : cout_g <= 32 ? TileCfg{1, 4, 2, 1}
                    : wide ? TileCfg{2, 2, 4, 2} : TileCfg{1, 4, 4, 2};
         if (kind == CK_1x1) return cout_g <= 16 ? TileCfg{1, 4, 1, 2} : cout_g <= 32 ? TileCfg{1, 4, 2, 2} : TileCfg{1, 4, 4, 2};
         // 2x2 and the phases of a transposed convolution
-        return cout_g <= 16 ? TileCfg{1, 8, 1, 1} : cout_g <= 32 ? TileCfg{1, 8, 2, 1} : TileCfg{1, 4, 4, 2};
+        return cout_g <= 16 ? (kind == CK_2x2 ? TileCfg{1, 4, 1, 2} : TileCfg{1, 8, 1, 1}) : cout_g <= 32 ? TileCfg{1, 8, 2, 1} : TileCfg{1, 4, 4, 2};
     }
     if (cout_g <= 16) return TileCfg{1, 4, 1, 2};
     if (cout_g <= 32) return TileCfg{1, 4, 2, 2};
@@ -582,6 +582,9 @@ LayerP make_conv_transpose(Context& ctx, int cin, int cout, int k, int stride, i
 //     (48) 30 / 19 / 17.
 //   32-channel groups and outputs: 256^2 (512 of 32 x 8) 32 ch x 8 rows 16.1, 16 x 8 by eight waves
 //     18.0; five groups at 34 x 60 (100) 11.2 / 8.2.
+//   16 outputs, stride 2 (of 16 x 8): from 350^2 (242) 16 ch x 4 rows 8.6, x 8 rows by eight waves 9.2,
+//     from 500^2 (512) 13.7 / 11.4, from 900^2 36 / 28; 2x2: at 100^2 (91) x 8 rows by eight waves 6.4, by
+//     four 6.5, at 180^2 (276) 7.5 / 7.0, at 500^2 (2016) 17.4 / 14.4.
 static TileCfg split_tile_cfg(const Layer& L, int N, int OH, int OW) {
     const int nb = L.cfg.wc * L.cfg.cf;
     const long long cols = (OW + 15) / 16, rows8 = (OH + 7) / 8, tiles = L.groups * (long long)(L.nblk_g / nb) * N;
@@ -591,6 +594,8 @@ static TileCfg split_tile_cfg(const Layer& L, int N, int OH, int OW) {
         return w < 56 ? TileCfg{1, 8, 1, 1} : w < 96 ? TileCfg{1, 4, 1, 2} : w < 200 ? TileCfg{1, 4, 2, 2}
                : w < 384 ? TileCfg{1, 4, 4, 2} : L.cfg;
     }
+    if (nb == 1 && L.kind == CK_3x3_S2) return cols * rows8 * tiles < 400 ? TileCfg{1, 4, 1, 1} : L.cfg;
+    if (nb == 1 && L.kind == CK_2x2) return cols * rows8 * tiles < 256 ? TileCfg{1, 8, 1, 1} : L.cfg;
     if (nb <= 2 || L.kind == CK_1x1) return L.cfg;
     if (L.kind == CK_T3) {  // per phase
         const long long w = (long long)(((OW + 1) / 2 + 15) / 16) * (((OH + 1) / 2 + 7) / 8) * (tiles * nb);
