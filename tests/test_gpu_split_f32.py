@@ -62,7 +62,8 @@ CASES = [("3x3", 4, 4, 1, 1, 1), ("3x3", 20, 24, 1, 9, 17), ("3x3", 160, 160, 1,
          ("2x2", 16, 16, 1, 210, 201), ("2x2", 20, 12, 1, 300, 130),
          ("2x2", 16, 192, 1, 150, 161), ("1x1", 4, 4, 1, 1, 1), ("1x1", 20, 24, 1, 9, 7), ("1x1", 48, 16, 1, 33, 64),
          ("1x1", 160, 160, 1, 8, 15), ("1x1", 128, 64, 1, 128, 127), ("1x1", 96, 128, 1, 150, 130),
-         ("1x1", 32, 256, 1, 171, 190), ("t3", 20, 12, 1, 1, 1), ("t3", 36, 64, 1, 17, 15), ("t3", 32, 96, 1, 90, 97),
+         ("1x1", 32, 256, 1, 171, 190), ("1x1", 16, 12, 1, 240, 251), ("1x1", 12, 36, 1, 301, 260),
+         ("1x1", 8, 200, 1, 130, 129), ("t3", 20, 12, 1, 1, 1), ("t3", 36, 64, 1, 17, 15), ("t3", 32, 96, 1, 90, 97),
          ("t3", 16, 128, 1, 130, 33), ("t4", 20, 24, 1, 3, 5), ("t4", 48, 64, 1, 31, 34), ("t4", 16, 160, 1, 70, 65),
          ("t4", 16, 128, 1, 135, 100)]
 

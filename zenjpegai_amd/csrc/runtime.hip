@@ -656,6 +656,15 @@ static bool convT_merged_fills(const Layer& L, int N, int OH, int OW) {
     return cols * ((rows + 15) / 16) * N * (L.nblk_g / TR_MERGED_NB) >= 256;
 }
 
+// Layers of one 16-channel chunk leave half of conv1x1_ring_split's stages empty: on large maps
+// conv_igemm_split (the same bits) is faster (us, ring / implicit GEMM, by 16-channel x 128-position
+// blocks): 16 -> 16 at 180^2 (254) 6.4 / 6.6, 250^2 (489) 7.4 / 7.1, 500^2 14.8 / 12.2, 900^2 34 / 25;
+// 8 -> 200 at 120^2 (1808) 11.8 / 12.2, 200^2 (5008) 22.6 / 21.1; 16 -> 64 at 180^2 (1016) 9.0 / 9.8, 4 ->
+// 64 at 300^2 (2816) 13.5 / 12.9, 16 -> 96 at 540^2 57 / 53.
+static bool ring_split_pays(const Layer& L, long long positions, int N) {
+    return L.nchunks > 1 || (positions + 127) / 128 * N * L.nblk_g < (L.nblk_g == 1 ? 400 : 2048);
+}
+
 // Tile of an f32 1x1 launch by its number of 64-channel x 128-position workgroups: narrower tiles
 // keep the CUs busy on small maps (us, one launch): 128 -> 512 at 431^2 (11616) 64 ch x 128
 // positions 255, 64 x 64 273, 32 x 64 337; 64 -> 256 at 108^2 (368) 13.9 / 12.4 / 13.8; 128 -> 128
@@ -850,7 +859,8 @@ static TensorP conv_forward_impl(Context& ctx, const Layer& L, const TensorP& x,
         ZJAI_HIP(launch_conv3x3_m32(L.dtype, L.mt32, tw, p, ctx.stream));
         return y;
     }
-    if (L.kind == CK_1x1 && L.dtype == DT_F32 && !(ctx.top().flags & ZJAI_CTX_IGEMM_CONV1X1) && conv1x1_ring_split_ok(p)) {
+    if (L.kind == CK_1x1 && L.dtype == DT_F32 && !(ctx.top().flags & ZJAI_CTX_IGEMM_CONV1X1) && conv1x1_ring_split_ok(p) &&
+        ring_split_pays(L, (long long)OH * OW, N)) {
         const TileCfg c = ring_split_cfg(L.nblk_g, (long long)OH * OW, N);
         LaunchScope sc(ctx, ring_split_name(c), 2.0 * macs, bytes);
         ZJAI_HIP(launch_conv1x1_ring_split(c, p, ctx.stream));
