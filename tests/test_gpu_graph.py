@@ -201,7 +201,7 @@ def test_merged_phase_transposed_convs_are_bit_identical_to_phase_split(prec, co
         outs.append(out)
     n_tr = 4 if comp == "y" else 2
     for ns in names:
-        assert not any(n.startswith("conv_tr_merged<") for n in ns)
+        assert not any(n.startswith("conv_tr_merged") for n in ns)
         assert sum(n.startswith("conv_") and "3, 3, 1, true," in n for n in ns) == n_tr
     assert np.isfinite(outs[0]).all()
     np.testing.assert_array_equal(outs[0], outs[1])

@@ -273,17 +273,16 @@ conv_igemm_split(const ConvParams p) {
 
 // ---------------------------------------------------------------------------------------------
 // Stride-2 transposed 3x3 convolution, padding 1, the four output phases of a tile in one
-// workgroup (conv_tr_merged's plan, conv.hip): WC * 2 blocks of 16 channels x WP * 2 rows x 16
-// columns of input positions; each wave accumulates two blocks x two rows for all four phases. A
+// workgroup (conv_tr_merged's plan, conv.hip): four blocks of 16 channels x four rows x 16 columns of
+// input positions; each wave accumulates two blocks x two rows for all four phases. A
 // phase reads the 2 x 2 input neighbourhood of a position, so the halo is one row and one column
 // and a chunk's nine taps share its few fragments. Weights (split, phase by phase) go through an
 // LDS ring three taps at a time. Per output the sums are conv_igemm_split's: bias, then per chunk
 // its phase's taps in table order.
 // ---------------------------------------------------------------------------------------------
-template <int WC, int WP>
-__global__ void __launch_bounds__(WC * WP * 64, 2)
+__global__ void __launch_bounds__(256, 2)
 conv_tr_merged_split(const ConvParams p) {
-    constexpr int NT = WC * WP * 64, CF = 2, PF = 2;
+    constexpr int WC = 2, WP = 2, CF = 2, PF = 2, NT = WC * WP * 64;
     constexpr int TY = WP * PF, HY = TY + 1, HX = 17, HP = HY * HX;
     constexpr int NB = WC * CF, TS = 3, NST = 3;
     constexpr int NPX = (HP + 15) / 32 * 32 + 16;
@@ -762,21 +761,16 @@ bool conv_tr_merged_split_ok(const ConvParams& p) {
            !p.relu6_in && !p.w_bstride;
 }
 
-template <int WC, int WP>
-static hipError_t go_merged_split(const ConvParams& p0, hipStream_t s) {
+hipError_t launch_conv_tr_merged_split(const ConvParams& p0, hipStream_t s) {
+    if (!conv_tr_merged_split_ok(p0)) return hipErrorInvalidValue;
     ConvParams p = p0;
-    p.ntiles = p.nblk_g / (WC * 2);
+    p.ntiles = p.nblk_g / TR_MERGED_NB;
     p.gx = ((p.OW + 1) / 2 + 15) / 16;
-    p.gy = ((p.OH + 1) / 2 + WP * 2 - 1) / (WP * 2);
+    p.gy = ((p.OH + 1) / 2 + 3) / 4;
     const long long total = (long long)p.gx * p.gy * p.N * p.ntiles;
-    if (p.nblk_g % (WC * 2) || total <= 0 || total > (1ll << 30)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((conv_tr_merged_split<WC, WP>), dim3((unsigned)total), dim3(WC * WP * 64), 0, s, p);
+    if (total <= 0 || total > (1ll << 30)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(conv_tr_merged_split, dim3((unsigned)total), dim3(256), 0, s, p);
     return hipGetLastError();
-}
-
-hipError_t launch_conv_tr_merged_split(const ConvParams& p, hipStream_t s) {
-    if (!conv_tr_merged_split_ok(p)) return hipErrorInvalidValue;
-    return go_merged_split<2, 2>(p, s);
 }
 
 }  // namespace zjai

@@ -828,12 +828,11 @@ static TensorP conv_forward_impl(Context& ctx, const Layer& L, const TensorP& x,
         static const char* ty[] = {"float", "_Float16", "__bf16"};
         p.w = L.wpk_m;
         p.ntiles = L.nblk_g / TR_MERGED_NB;
-        LaunchScope sc(ctx,
-                       std::string("conv_tr_merged<") + ty[L.dtype] + ", " + std::to_string(L.ntaps[0]) + ", " +
-                           std::to_string(L.ntaps[1]) + ", " + std::to_string(L.ntaps[2]) + ", " +
-                           std::to_string(L.ntaps[3]) + ">",
-                       2.0 * macs,
-                       bytes - (double)L.wpk_bytes + (double)L.wpk_m_bytes);
+        const std::string name = L.dtype == DT_F32 ? std::string("conv_tr_merged_split")
+                                                   : std::string("conv_tr_merged<") + ty[L.dtype] + ", " + std::to_string(L.ntaps[0]) +
+                                                         ", " + std::to_string(L.ntaps[1]) + ", " + std::to_string(L.ntaps[2]) + ", " +
+                                                         std::to_string(L.ntaps[3]) + ">";
+        LaunchScope sc(ctx, name, 2.0 * macs, bytes - (double)L.wpk_bytes + (double)L.wpk_m_bytes);
         if (L.dtype == DT_F32) ZJAI_HIP(launch_conv_tr_merged_split(p, ctx.stream));
         else ZJAI_HIP(launch_conv_tr_merged(L.dtype, p, ctx.stream));
         return y;
