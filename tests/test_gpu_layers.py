@@ -245,6 +245,7 @@ def test_conv1x1_kernels_are_bit_identical(engines, prec, cin, cout, h, w, op, c
 SMALL_GRID_CASES = [
     ("3x3", 192, 192, 24, 40, 256, "conv_igemm"),
     ("3x3", 192, 192, 80, 96, 256, "conv_igemm"),
+    ("3x3", 160, 256, 24, 40, 256, "conv_igemm"),  # f32 large map: 128-channel tiles
     ("s2", 192, 192, 48, 80, 256, "conv_igemm"),
     ("s2", 128, 128, 48, 80, 384, "conv_igemm"),  # 16-bit large map: 128-channel tiles
     ("convT", 192, 192, 20, 24, 160, "conv_igemm"),

@@ -1,13 +1,19 @@
 """GPU: the f32 convolutions that run on the bf16 matrix cores (three bf16 pieces per value, six
-piece products, csrc/split.h) against 64-bit sums, at the edges of their tiles and on values that
-are not finite.
+piece products, csrc/split.h) against 64-bit sums, at the edges of their tiles, on values that are not
+finite, at both ends of f32's range, and the fused blocks against the single layers.
 
-Bound: the matrix core rounds its f32 accumulator once per 8 products; the full-size accumulator
-takes 16 of the K products per 4 such roundings, its partner's are 2^-8 smaller, the pieces drop
-2^-26 of a product, and bias, final sum and store add three roundings; a 1x1 layer adds the two
-accumulators every 32 products. Every rounding is at most 2^-23 (it may truncate) of a partial sum,
-itself at most S = |b| + sum |x w|, so |err| <= (K / 4 * (1 + 2^-7) + 4 + [1x1] (K / 32 + 1)) *
-2^-23 * S."""
+Worst case: the matrix core rounds its f32 accumulator once per 8 products; the full-size accumulator
+takes 16 of the K products per 4 such roundings, its partner twice as many of sums 2^-7 as large, the
+dropped products are 2^-24 of a product, and bias, final sum and store add three roundings; a 1x1 layer
+adds the two accumulators every 32 products. Every rounding is at most 2^-23 (it may truncate) of a
+partial sum, itself at most S = |b| + sum |x w|, so |err| <= (K / 4 * (1 + 2^-6) + 4.5 + [1x1] (K / 32 +
+1)) * 2^-23 * S.
+
+That bound grows past the third pieces' part of a result, so that of random products (rms_bound) is held
+too: roundings to nearest are at most 2^-24 of a partial sum and independent, so that the rms of err / S2,
+S2^2 = b^2 + sum (x w)^2, stays below (sqrt(K / 7) + 2) * 2^-24: K / 4 + K / 32 roundings of partial sums
+of half the mean square, and the rest. A missing piece product leaves 2.7e-6 at least, whatever K is
+(tests/test_split_bounds.py)."""
 
 import numpy as np
 import pytest
@@ -24,6 +30,10 @@ def eng():
     e = nn.Engine(0, "f32")
     yield e
     e.close()
+
+
+def rms_bound(k):
+    return ((k / 7) ** 0.5 + 2) * 2.0 ** -24
 
 
 def _layer(eng, kind, cin, cout, groups, seed):
@@ -76,8 +86,11 @@ def test_error_against_64_bits(eng, kind, cin, cout, groups, h, w):
     want, size = ref(x, wt, b), ref(np.abs(x), np.abs(wt), np.abs(b))
     assert y.shape == want.shape
     kk = cin * 4 if kind[0] == "t" else wt[0].size  # at most 2 x 2 taps reach an output
-    bound = (kk / 4 * (1 + 2.0 ** -7) + 4 + (kk / 32 + 1 if kind == "1x1" else 0)) * 2.0 ** -23 * size
+    bound = (kk / 4 * (1 + 2.0 ** -6) + 4.5 + (kk / 32 + 1 if kind == "1x1" else 0)) * 2.0 ** -23 * size
     assert np.all(np.abs(y - want) <= bound), float(np.max(np.abs(y - want) / bound))
+    if y.size >= 1000:
+        rms = float(np.sqrt(np.mean((y - want) ** 2 / ref(x * x, wt * wt, b * b))))
+        assert rms <= rms_bound(kk), (rms, rms_bound(kk))
 
 
 @pytest.mark.parametrize("kind", ["1x1", "3x3", "s2", "2x2", "t3", "t4"])
@@ -227,3 +240,19 @@ def test_fused_blocks_split_large_values_as_the_single_layers_do(op, comp):
         e.close()
     assert np.isfinite(outs[0]).all() and len(np.unique(outs[0])) > 1000
     np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind,cin,cout,ch,step", ONE_CHANNEL)
+@pytest.mark.parametrize("weights", [False, True])
+def test_the_smallest_values(eng, kind, cin, cout, ch, step, weights):
+    """Below 2^-110 the pieces run out of bf16's exponents: what is left of an operand is within 2^-134 (half
+    of the smallest bf16) of it, and the rest as for any other product."""
+    n = N_VALUES
+    tiny = synth.uniform(37, "split/tiny", (n,), 1.0, 2.0) * (2.0 ** -np.linspace(100, 149, n)).astype(np.float32)
+    tiny, other = np.concatenate([tiny[::2], -tiny[1::2]]).astype(np.float32), [1.0, -0.3, 2.0 ** 60, 1.2345e37, 0.0]
+    xv, wv = (_cycle(other, n), _cycle(tiny, cout)) if weights else (tiny, _cycle(other, cout))
+    want = wv[:, None].astype(np.float64) * xv
+    left = np.abs(_cycle(other, n)[None] if weights else _cycle(other, cout)[:, None]) * 2.0 ** -134
+    y = _products(eng, kind, cin, cout, ch, step, xv, wv)
+    bound = left * (1 + 2.0 ** -7) + 2.0 ** -22 * np.abs(want) + 2.0 ** -149
+    assert np.all(np.abs(y - want) <= bound), float(np.max(np.abs(y - want) / bound))
