@@ -14,7 +14,8 @@ def test_planar_round_trip_is_exact_on_both_sides_of_the_slot_size(w, locked):
 
     eng = nn.Engine(0, "f32")
     rng = np.random.default_rng(w)
-    # More uploads than there are slots, none waited for before the next begins.
+    # Every slot in turn and the first ones again. (Each call waits for its own copy, so no slot is taken
+    # while it is still being read.)
     xs = [torch.from_numpy(rng.standard_normal((4, 1, w)).astype(np.float32)) for _ in range(7)]
     if locked:
         xs = [x.pin_memory() for x in xs]
@@ -22,3 +23,4 @@ def test_planar_round_trip_is_exact_on_both_sides_of_the_slot_size(w, locked):
     ts = [nn.BTensor.from_planar(eng, x) for x in xs]
     for x, t in zip(xs, ts):
         np.testing.assert_array_equal(t.to_planar(), x)
+    eng.close()

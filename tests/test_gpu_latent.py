@@ -157,6 +157,37 @@ def test_reconstruct_latent_16bit_storage(prec):
         e.close()
 
 
+# 64 x 48: every copy fits a page-locked slot; 704 x 512: none of residual, psi and y_hat does.
+@pytest.mark.parametrize("height,width,regions", [(64, 48, None), (704, 512, geo.Regions(2, 2, True)),
+                                                  (704, 512, geo.Regions(2, 2, False, 1, 4))])
+@pytest.mark.parametrize("inputs,outputs", [("pageable", "locked"), ("locked", "pageable"), ("locked", "locked"),
+                                            ("locked", "in place"), ("pageable", "in place")])
+def test_reconstruct_latent_from_and_to_page_locked_arrays(eng, height, width, regions, inputs, outputs):
+    """The residual's upload and psi's download run on a second stream, asynchronously where the caller's
+    array is page-locked: whatever the arrays are, y_hat in the residual's place included, the results are
+    those of ordinary ones, call after call."""
+    c = synth.LATENT_CHANNELS[0]
+    h, w, zh, zw = _sizes(0, height, width)
+    m = model.LatentModel.load(synth.random_latent_params(0, seed=29, gain=1.0), 0, eng)
+
+    def array(shape, dtype, kind):
+        return eng.host_array(shape, dtype) if kind == "locked" else np.empty(shape, dtype)
+
+    zd, rd = array((c, zh, zw), np.int8, inputs), array((c, h, w), np.float32, inputs)
+    psi = array((4 * c, _ceil(h, 2), _ceil(w, 2)), np.float32, outputs)
+    y = rd if outputs == "in place" else array((c, h, w), np.float32, outputs)
+    _keep, rp = model._regions_ptr(_mr(regions))
+    for seed in (1, 2, 3):
+        z, r = synth.hyper_latent(seed, "pl/z", c, zh, zw), synth.normal(seed, "pl/r", (c, h, w), 0.5)
+        want_psi, want_y = m.reconstruct(height, width, _mr(regions), z, r)
+        zd[...], rd[...] = z, r
+        psi[...] = np.nan
+        _lib.check(_lib.lib().zjai_reconstruct_latent(eng.handle, m._h, height, width, rp, zd.ctypes.data, zh, zw,
+                                                      model._fp(rd), h, w, model._fp(psi), model._fp(y)), eng.handle)
+        np.testing.assert_array_equal(psi, want_psi)
+        np.testing.assert_array_equal(y, want_y)
+
+
 def test_latent_errors_are_invalid_arguments(eng):
     p = synth.random_latent_params(1, seed=27)
     m = model.LatentModel.load(p, 1, eng)

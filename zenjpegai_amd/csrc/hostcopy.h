@@ -15,7 +15,8 @@ public:
     static constexpr size_t SLOT = 256u << 10;
     static constexpr int SLOTS = 4;
     void create();
-    // Returns once `src` may be reused; the device side is in stream order.
+    // In stream order on the device. A pageable `src` may be reused on return; a page-locked one is read in
+    // stream order too, and stays until `s` has got there.
     void to_device(void* dst, const void* src, size_t n, hipStream_t s);
     // Page-locked `dst`: in stream order. Pageable `dst`: holds the bytes on return.
     void to_host(void* dst, const void* src, size_t n, hipStream_t s);
