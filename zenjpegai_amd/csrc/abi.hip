@@ -471,7 +471,7 @@ extern "C" int32_t zjai_channel_attention_noalloc(zjai_ctx* ctx, const void* qkv
         const TileCfg cfg = conv_tile_cfg(dim, CK_1x1, precision);
         const int nblk = round_up(ceil_div(dim, 16), cfg.wc * cfg.cf), nchunks = ceil_div(dim, CK);
         const size_t w_plain = (size_t)nchunks * nblk * 16 * CK * es;
-        const size_t w_bytes = conv_is_split(CK_1x1, precision) ? w_plain / 2 * 3 : w_plain;
+        const size_t w_bytes = conv_is_split(precision) ? w_plain / 2 * 3 : w_plain;
         // Scratch layout: Gram partials [nchunk][heads][c*c + 2c] f32 | attn [dim][c] f32 | weight.
         const int nchunk = attention_gram_chunks(h, w);
         const size_t part_bytes = (size_t)nchunk * heads * (c * c + 2 * c) * 4;
@@ -526,7 +526,7 @@ extern "C" int32_t zjai_channel_attention_noalloc(zjai_ctx* ctx, const void* qkv
         p.out_mode = OUT_NHWC;
         p.sv = p.sh = 1;
         const double flops = 2.0 * n * dim * dim, bytes = es * 2.0 * n * dim + (double)w_bytes;
-        if (conv_is_split(CK_1x1, precision)) {  // views of a dim % 8 == 0 map on 16-byte buffers: always aligned
+        if (conv_is_split(precision)) {  // views of a dim % 8 == 0 map on 16-byte buffers: always aligned
             const TileCfg c1 = ring_split_cfg(nblk, (long long)h * w, 1);
             LaunchScope sc(C, ring_split_name(c1), flops, bytes);
             ZJAI_HIP(launch_conv1x1_ring_split(c1, p, C.stream));

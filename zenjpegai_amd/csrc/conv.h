@@ -66,9 +66,9 @@ struct TileCfg {
 
 enum ConvKind : int { CK_1x1 = 0, CK_2x2 = 1, CK_3x3 = 2, CK_3x3_S2 = 3, CK_T3 = 4 };
 
-// f32 layers of these kinds run on the bf16 matrix cores from weights packed in split form
-// (conv_f32.hip, split.h); everything else goes through launch_conv.
-inline bool conv_is_split(int kind, int dtype) { return dtype == DT_F32 && kind <= CK_T3; }
+// f32 layers of every kind run on the bf16 matrix cores from weights packed in split form
+// (conv_f32.hip, split.h), 16-bit ones go through launch_conv.
+inline bool conv_is_split(int dtype) { return dtype == DT_F32; }
 // nblk blocks of [16 outputs][16 channels] f32 weights into split.h's blocks.
 hipError_t launch_split_weights(const float* src, void* dst, long long nblk, hipStream_t s);
 hipError_t launch_conv_split(int kind, TileCfg cfg, const ConvParams& p, hipStream_t s);

@@ -25,9 +25,10 @@ template <> struct Mma16<__bf16> {
     }
 };
 
-// 32x32 tile, 16 channels of K per instruction (16-bit types only): v_mfma_f32_32x32x16 runs
-// at twice the rate of the 16x16x32 form on gfx950 (measured 2.36 vs 1.33 PF/s on register
-// operands). Lane (j, h) = (lane % 32, lane / 32) supplies row / column j and channels
+// 32x32 tile, 16 channels of K per instruction (16-bit types only): half the LDS fragment reads
+// per FLOP of the 16x16x32 form. On registers (independent chains, two waves per SIMD) it runs 1.84
+// PFLOP/s on random operands and 2.46 on zeros, 16x16x32 2.07 and 2.36: the chip's power sets the
+// rate, not the form. Lane (j, h) = (lane % 32, lane / 32) supplies row / column j and channels
 // 8h..8h+7 of the 16-channel step; accumulator register r holds row 8 * (r / 4) + 4 * h + r % 4
 // of column j.
 template <typename T> struct Mma32;

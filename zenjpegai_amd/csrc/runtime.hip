@@ -327,7 +327,7 @@ void Layer::out_size(int h, int w, int* oh, int* ow) const {
 // 3x3 layers take the 8-wave 64-channel x 16-row tile (two waves per SIMD from one workgroup hide
 // each other's LDS and barrier waits: +2-3 % on the config-5 picture in every precision).
 TileCfg conv_tile_cfg(int cout_g, int kind, int dtype) {
-    if (conv_is_split(kind, dtype)) {  // the large-map shapes of conv_f32.hip
+    if (conv_is_split(dtype)) {  // the large-map shapes of conv_f32.hip
         const bool wide = cout_g % 128 == 0;
         if (kind == CK_3x3)
             return cout_g <= 16 ? TileCfg{1, 4, 1, 2} : cout_g <= 32 ? TileCfg{1, 4, 2, 2}
@@ -395,7 +395,7 @@ LayerP make_conv(Context& ctx, int cin, int cout, int kh, int kw, int stride, in
                 const float* src = weight + ((size_t)(g * cout_g + ocl) * cin_g + icl) * T;
                 for (int t = 0; t < T; ++t) dst[(size_t)t * 16 * CK] = src[t];
             }
-    L->wpk = conv_is_split(L->kind, dtype) ? upload_split(ctx, pk, &L->wpk_bytes, &L->dev_bytes)
+    L->wpk = conv_is_split(dtype) ? upload_split(ctx, pk, &L->wpk_bytes, &L->dev_bytes)
                                            : upload_as(ctx, pk, dtype, &L->wpk_bytes, &L->dev_bytes);
     if (dtype != DT_F32 && L->kind == CK_3x3 && groups == 1 && (cin == 64 || cin == 128) && cout % 64 == 0 && no_extra &&
         pad_h == 1 && pad_w == 1) {
@@ -616,7 +616,7 @@ static TileCfg split_tile_cfg(const Layer& L, int N, int OH, int OW) {
 // (512 tiles) the 16-row tile stays fastest.
 static TileCfg launch_tile_cfg(const Layer& L, int N, int OH, int OW) {
     const TileCfg c = L.cfg;
-    if (conv_is_split(L.kind, L.dtype)) return split_tile_cfg(L, N, OH, OW);
+    if (conv_is_split(L.dtype)) return split_tile_cfg(L, N, OH, OW);
     if (L.groups != 1) return c;
     const long long nt4 = L.nblk_g / 4;
     if (L.kind == CK_3x3 && c.wc == 2 && c.wp == 4 && c.cf == 2 && c.pf == 4) {
@@ -647,9 +647,10 @@ static TileCfg launch_tile_cfg(const Layer& L, int N, int OH, int OW) {
 // Transposed 3x3 layers take the merged four-phase kernel on maps large enough for its grid, else
 // the phase-split kernel on a narrow tile. 16-bit: at least 256 workgroups of 16 x 16 phase
 // positions x 64 channels. f32 (64 channels x 4 rows of positions per workgroup): from 60
-// tiles of 16 x 8 positions -- 128 -> 128 from 88^2 (66 tiles) merged 36 us, phase-split 44; from 176^2 73 / 111;
-// 64 -> 64 from 108^2 (98) 20.5 / 21.0; below it 160 -> 128 from 64 x 96 (48) 34.6 / 35.2, 128 -> 128
-// from 52 x 76 (35) 28.8 / 27.8 and from 26 x 38 (15) 27 / 17.
+// tiles of 16 x 8 positions, for any number of outputs, which adds to both grids alike -- 128 -> 128
+// from 88^2 (66 tiles) merged 36 us, phase-split 44; from 176^2 73 / 111; 64 -> 64 from 108^2 (98)
+// 20.5 / 21.0; below it 160 -> 128 from 64 x 96 (48) 34.6 / 35.2, 128 -> 128 from 52 x 76 (35) 28.8 /
+// 27.8 and from 26 x 38 (15) 27 / 17.
 static bool convT_merged_fills(const Layer& L, int N, int OH, int OW) {
     const long long cols = ((OW + 1) / 2 + 15) / 16, rows = (OH + 1) / 2;
     if (L.dtype == DT_F32) return cols * ((rows + 7) / 8) * N >= 60;
@@ -689,7 +690,7 @@ std::string conv_kernel_name(int kind, int dtype, TileCfg c) {
                                 "3, 3, 1, true"};
     static const char* ty[] = {"float", "_Float16", "__bf16"};
     char buf[128];
-    if (conv_is_split(kind, dtype)) {
+    if (conv_is_split(dtype)) {
         snprintf(buf, sizeof buf, "conv_igemm_split<%s, %d, %d, %d, %d>", geo[kind], c.wc, c.wp, c.cf, c.pf);
         return buf;
     }
@@ -876,7 +877,7 @@ static TensorP conv_forward_impl(Context& ctx, const Layer& L, const TensorP& x,
     const TileCfg cfg = launch_tile_cfg(L, N, OH, OW);
     p.ntiles = L.groups * L.nblk_g / (cfg.wc * cfg.cf);
     LaunchScope sc(ctx, conv_kernel_name(L.kind, L.dtype, cfg), 2.0 * macs, bytes);
-    if (conv_is_split(L.kind, L.dtype)) ZJAI_HIP(launch_conv_split(L.kind, cfg, p, ctx.stream));
+    if (conv_is_split(L.dtype)) ZJAI_HIP(launch_conv_split(L.kind, cfg, p, ctx.stream));
     else ZJAI_HIP(launch_conv(L.kind, L.dtype, cfg, p, ctx.stream));
     return y;
 }

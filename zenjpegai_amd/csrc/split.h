@@ -1,12 +1,13 @@
 // f32 products on the bf16 matrix cores (gfx950).
 //
 // An f32 value is the exact sum of three bf16 pieces, v = p0 + p1 + p2 (8 significant bits each,
-// rounded to nearest, so |p1| <= 2^-9 |v| and |p2| <= 2^-18 |v|). Of the nine piece products of
-// a * b the six largest carry everything down to 2^-26 of the product -- below half an ulp of the
-// f32 product -- so a sum of products takes six bf16 multiply-adds per f32 one, at sixteen times
-// the rate: v_mfma_f32_16x16x32_bf16 measured 1.95 PFLOP/s on registers, i.e. 325 TFLOP/s of f32
-// products, against 136-150 TFLOP/s for v_mfma_f32_16x16x4_f32, and unlike the f32 form it runs
-// beside vector work.
+// rounded to nearest, so |p1| <= 2^-8 |v| and |p2| <= 2^-17 |v|). Of the nine piece products of
+// a * b the six largest are summed; the others are at most 2^-24 of the product, 2^-27.5 in the mean
+// square (Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", ARITH 2019). A sum of products takes six bf16 multiply-adds per f32
+// one, at sixteen times the rate: v_mfma_f32_16x16x32_bf16 runs 1.95 PFLOP/s on registers (random
+// operands, eight chains, one wave per SIMD), i.e. 325 TFLOP/s of f32 products, against 137-142 for
+// v_mfma_f32_16x16x4_f32, and unlike the f32 form it runs beside vector work.
 //
 // A lane holds four channels of an operand as six registers [p1 x4 | p0 x4 | p2 x4]: its first
 // four (`lo`) are the pieces (p1, p0), its last four (`hi`) the pieces (p0, p2), each the eight K
