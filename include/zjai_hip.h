@@ -317,8 +317,9 @@ ZJAI_API int32_t zjai_picture_upload(zjai_ctx* ctx, zjai_picture* pic, const flo
  *     out), >= live_bytes.
  * live and pool are models calibrated on measured pool use that bound it from above (bytes per
  * sample of each tile batch's 16 x latent window, +8 %). The nets' own bytes
- * (zjai_net_device_bytes) and the buffers of zjai_picture_download_rgb (6 bytes per displayed
- * pixel, 18 with float planes) are not included. */
+ * (zjai_net_device_bytes), the buffers of zjai_picture_download_rgb (6 bytes per displayed
+ * pixel, 18 with float planes) and what a context holds by itself (17 MiB of attention scratch, and
+ * 4 MiB or the largest f32 layer once f32 layers were made) are not included. */
 typedef struct zjai_memory_estimate {
     uint64_t picture_bytes;
     uint64_t live_bytes;
