@@ -157,7 +157,7 @@ typedef struct zjai_prof_record {
 ZJAI_API int32_t zjai_profile_begin(zjai_ctx* ctx);
 ZJAI_API int32_t zjai_profile_end(zjai_ctx* ctx, zjai_prof_record* out, int32_t cap, int32_t* n);
 /* Returns cached pool blocks to the device (`release_buffers`, src/nn/fast/tensor.rs:122), the
- * lanes' included, and the buffer that f32 weights of new layers go through, and starts a new pool_peak. The pool figures of zjai_get_stats cover the
+ * lanes' included, and starts a new pool_peak. The pool figures of zjai_get_stats cover the
  * context's own pool and every lane's (pool_peak: the sum of the pools' high-water marks). */
 ZJAI_API int32_t zjai_release_buffers(zjai_ctx* ctx);
 
@@ -241,8 +241,8 @@ ZJAI_API int32_t zjai_channel_attention(zjai_ctx* ctx, const zjai_tensor* qkv, i
  * [h][w][channels] (channels = 3 * dim: q, k, v), out [h][w][dim]; temperature is a device array
  * of `heads` floats. The work is enqueued on the context's stream (zjai_sync waits for it) and
  * allocates nothing: its scratch (Gram partial sums, attention matrix, folded weight) is an array
- * of ZJAI_NOALLOC_SCRATCH_BYTES (and 1 MiB beside it) that zjai_ctx_create allocates for the
- * context, so calls on several contexts may overlap on one GPU. A map that needs more scratch (with
+ * of ZJAI_NOALLOC_SCRATCH_BYTES (and 1 MiB beside it) that zjai_ctx_create takes for the context
+ * (new, or the one that the last destroyed context of the device left), so calls on several contexts may overlap on one GPU. A map that needs more scratch (with
  * dim 128 and 4 heads: more than ~240k positions) returns ZJAI_E_LIMIT before anything is launched. */
 #define ZJAI_NOALLOC_SCRATCH_BYTES (16u << 20)
 ZJAI_API int32_t zjai_channel_attention_noalloc(zjai_ctx* ctx, const void* qkv, int32_t channels,
@@ -318,8 +318,8 @@ ZJAI_API int32_t zjai_picture_upload(zjai_ctx* ctx, zjai_picture* pic, const flo
  * live and pool are models calibrated on measured pool use that bound it from above (bytes per
  * sample of each tile batch's 16 x latent window, +8 %). The nets' own bytes
  * (zjai_net_device_bytes), the buffers of zjai_picture_download_rgb (6 bytes per displayed
- * pixel, 18 with float planes) and what a context holds by itself (17 MiB of attention scratch, and
- * 4 MiB or the largest f32 layer once f32 layers were made) are not included. */
+ * pixel, 18 with float planes) and what a context holds by itself (17 MiB of scratch) are not
+ * included. */
 typedef struct zjai_memory_estimate {
     uint64_t picture_bytes;
     uint64_t live_bytes;

@@ -147,6 +147,26 @@ def test_noalloc_attention_of_several_contexts_in_flight_together(prec):
             eng.close()
 
 
+def test_contexts_made_and_destroyed_in_turn_and_together():
+    """The scratch a destroyed context leaves serves the next one; contexts alive together have their own.
+    Each makes an f32 layer (its weights go through the scratch) between two attention calls."""
+    hip = _hip()
+    w = synth.normal(50, "noalloc/w", (64, 64, 1, 1), 0.1)
+    x = synth.normal(51, "noalloc/x", (64, 9, 7), 1.0)
+    first = nn.Engine(0, "f32")
+    want = nn.ConvLayer(nn.Conv2d(64, 64, (1, 1), 1, (0, 0), 1, w), first).forward(first, nn.BTensor.from_planar(first, x)).to_planar()
+    for k in range(3):
+        engs = [nn.Engine(0, "f32") for _ in range(1 + k)]
+        for i, eng in enumerate(engs):
+            assert np.array_equal(*_run_both(eng, hip, 64, 4, 30 + k, 20, "f32", 60 + i))
+            layer = nn.ConvLayer(nn.Conv2d(64, 64, (1, 1), 1, (0, 0), 1, w), eng)
+            assert np.array_equal(*_run_both(eng, hip, 128, 4, 12, 11, "f32", 70 + i))
+            assert np.array_equal(layer.forward(eng, nn.BTensor.from_planar(eng, x)).to_planar(), want)
+        for eng in engs:
+            eng.close()
+    first.close()
+
+
 def test_noalloc_attention_rejects_a_map_beyond_the_scratch():
     """Checked on the host before any launch: 1024 x 1024 positions at dim 128 need ~71 MB of
     Gram partials, more than the 16 MiB scratch; dim 640 exceeds the Gram kernel's LDS stage.

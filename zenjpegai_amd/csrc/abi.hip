@@ -77,12 +77,9 @@ TensorP planar_upload(Context& c, const float* data, int ch, int h, int w, int d
 
 }  // namespace
 
-// Scratch of zjai_channel_attention_noalloc, one per context: every launch of a call runs on the
+// zjai_channel_attention_noalloc works in its context's scratch: every launch of a call runs on the
 // context's stream, so calls on one context follow each other, and calls on several contexts (whose
-// streams nothing orders) share nothing. The bytes past ZJAI_NOALLOC_SCRATCH_BYTES hold the third
-// bf16 piece of an f32 call's folded weight (half its f32 size; dim <= 639 by the Gram kernel's LDS
-// stage), so that maps up to the documented size fit as they do in f32 form.
-static constexpr size_t SCRATCH_PIECE_BYTES = 1u << 20;
+// streams nothing orders) share nothing.
 static size_t round_up256(size_t n) { return (n + 255) / 256 * 256; }
 
 // ------------------------------------------------------------------------------- context
@@ -110,7 +107,7 @@ extern "C" int32_t zjai_ctx_create(int32_t device, uint32_t flags, zjai_ctx** ou
         ZJAI_HIP(hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking));
         ZJAI_HIP(hipEventCreate(&ctx->c.ev0));
         ZJAI_HIP(hipEventCreate(&ctx->c.ev1));
-        ZJAI_HIP(hipMalloc(&ctx->c.attention_scratch, ZJAI_NOALLOC_SCRATCH_BYTES + SCRATCH_PIECE_BYTES));
+        ctx->c.scratch = take_scratch(device);
         ctx->c.copier.create();
     });
     if (rc != ZJAI_OK) {
@@ -220,7 +217,6 @@ extern "C" int32_t zjai_release_buffers(zjai_ctx* ctx) {
         ZJAI_HIP(hipStreamSynchronize(ctx->c.stream));
         ctx->c.pool.trim();
         ctx->c.pool.reset_peak();
-        ctx->c.release_weight_stage();
         for (const auto& l : ctx->c.lanes) {
             ZJAI_HIP(hipStreamSynchronize(l->stream));
             l->pool.trim();
@@ -478,7 +474,7 @@ extern "C" int32_t zjai_channel_attention_noalloc(zjai_ctx* ctx, const void* qkv
         const size_t attn_off = round_up256(part_bytes), w_off = round_up256(attn_off + (size_t)dim * c * 4);
         if (w_off + w_plain > ZJAI_NOALLOC_SCRATCH_BYTES || w_bytes - w_plain > SCRATCH_PIECE_BYTES)
             throw Error(ZJAI_E_LIMIT, "attention: the map needs more than the allocation-free scratch");
-        unsigned char* base = (unsigned char*)ctx->c.attention_scratch;
+        unsigned char* base = (unsigned char*)ctx->c.scratch;
         float* partial = (float*)base;
         float* attn = (float*)(base + attn_off);
         void* wfold = base + w_off;

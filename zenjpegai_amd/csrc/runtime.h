@@ -113,9 +113,9 @@ struct Context {
     std::string last_error;
     volatile int stop = 0;
     uint64_t mem_limit = 0;  // zjai_ctx_set_memory_limit: device bytes a picture may need (0: none)
-    void* attention_scratch = nullptr;  // zjai_channel_attention_noalloc's (root context)
-    void* weight_stage = nullptr;  // f32 weights on their way to the split form (root context)
-    size_t weight_stage_bytes = 0;
+    // Root context: CONTEXT_SCRATCH_BYTES for zjai_channel_attention_noalloc and for f32 weights on their
+    // way to the split form, both in stream order.
+    void* scratch = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float last_ms = 0.0f;
     long long launches = 0;
@@ -140,9 +140,19 @@ struct Context {
     TensorP alloc(int n, int c, int h, int w, int dtype);
     void check_stop();
     hipEvent_t take_event();
-    void release_weight_stage();
     ~Context();
 };
+
+// The bytes past ZJAI_NOALLOC_SCRATCH_BYTES hold the third bf16 piece of an f32 attention call's folded
+// weight (half its f32 size; dim <= 639 by the Gram kernel's LDS stage), so that maps up to the
+// documented size fit as they do in f32 form.
+constexpr size_t SCRATCH_PIECE_BYTES = 1u << 20;
+constexpr size_t CONTEXT_SCRATCH_BYTES = ZJAI_NOALLOC_SCRATCH_BYTES + SCRATCH_PIECE_BYTES;
+// A context's scratch on the current device. The last one given back stays for the next context of its
+// device (one array per device, until the process ends): a program that makes a context per picture would
+// otherwise pay for the allocation, and for what freeing 17 MiB costs the allocations after it, each time.
+void* take_scratch(int device);
+void give_scratch(int device, void* p);  // nothing in flight uses it
 
 // Brackets one kernel launch: counts it and, while profiling, records events around it.
 class LaunchScope {

@@ -4,6 +4,7 @@
 #include "checkpoint.h"
 
 #include <cmath>
+#include <mutex>
 #include <cstring>
 
 namespace zjai {
@@ -136,14 +137,43 @@ Context::~Context() {
     }
     for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
     if (range_slots) (void)hipFree(range_slots);
-    if (attention_scratch) (void)hipFree(attention_scratch);
-    release_weight_stage();
+    if (scratch) give_scratch(device, scratch);
 }
 
-void Context::release_weight_stage() {
-    if (weight_stage) (void)hipFree(weight_stage);
-    weight_stage = nullptr;
-    weight_stage_bytes = 0;
+namespace {
+struct KeptScratch {
+    std::mutex mu;
+    std::map<int, void*> of_device;
+};
+KeptScratch& kept_scratch() {
+    static KeptScratch* k = new KeptScratch;  // never destroyed: contexts may be, as late as they like
+    return *k;
+}
+}  // namespace
+
+void* take_scratch(int device) {
+    {
+        KeptScratch& k = kept_scratch();
+        std::lock_guard<std::mutex> g(k.mu);
+        auto it = k.of_device.find(device);
+        if (it != k.of_device.end()) {
+            void* p = it->second;
+            k.of_device.erase(it);
+            return p;
+        }
+    }
+    void* p = nullptr;
+    ZJAI_HIP(hipMalloc(&p, CONTEXT_SCRATCH_BYTES));
+    return p;
+}
+
+void give_scratch(int device, void* p) {
+    {
+        KeptScratch& k = kept_scratch();
+        std::lock_guard<std::mutex> g(k.mu);
+        if (k.of_device.emplace(device, p).second) return;
+    }
+    (void)hipFree(p);
 }
 
 void range_slots_init(Context& ctx) {
@@ -272,22 +302,20 @@ static void* upload_as(Context& ctx, const std::vector<float>& host, int dtype, 
 
 // A packed f32 weight ([..][16 outputs][16 channels] blocks) as three bf16 pieces per value in
 // the fragment order of split.h, split on the device: on the host a HOP luma net's weights took
-// 4 ms of its 9 ms. The f32 copy goes through a buffer that the context keeps (the largest layer's
-// size), on the null stream as the plain uploads.
+// 4 ms of its 9 ms. The f32 copy goes through the context's scratch, piece by piece in stream order.
 static void* upload_split(Context& ctx, const std::vector<float>& host, size_t* bytes_out, size_t* total) {
     Context& c = ctx.top();
     const size_t n = host.size() * 4, bytes = n / 2 * 3;
-    if (c.weight_stage_bytes < n) {
-        c.release_weight_stage();
-        ZJAI_HIP(hipMalloc(&c.weight_stage, std::max(n, size_t(4) << 20)));
-        c.weight_stage_bytes = std::max(n, size_t(4) << 20);
-    }
-    ZJAI_HIP(hipMemcpy(c.weight_stage, host.data(), n, hipMemcpyHostToDevice));
+    static_assert(CONTEXT_SCRATCH_BYTES % 1024 == 0, "whole blocks");
     void* dev = nullptr;
     ZJAI_HIP(hipMalloc(&dev, bytes));
     std::unique_ptr<void, hipError_t (*)(void*)> keep(dev, hipFree);
-    ZJAI_HIP(launch_split_weights((const float*)c.weight_stage, dev, (long long)(host.size() / 256), nullptr));
-    ZJAI_HIP(hipStreamSynchronize(nullptr));
+    for (size_t off = 0; off < n; off += CONTEXT_SCRATCH_BYTES) {
+        const size_t k = std::min(n - off, CONTEXT_SCRATCH_BYTES);
+        ZJAI_HIP(hipMemcpyAsync(c.scratch, (const char*)host.data() + off, k, hipMemcpyHostToDevice, c.stream));
+        ZJAI_HIP(launch_split_weights((const float*)c.scratch, (char*)dev + off / 2 * 3, (long long)(k / 1024), c.stream));
+    }
+    ZJAI_HIP(hipStreamSynchronize(c.stream));
     keep.release();
     *bytes_out = bytes;
     *total += bytes;
